@@ -618,7 +618,8 @@ static size_t tile_bytes(int m, int n, int k, int maxrank)
 {
     size_t r = (size_t)(maxrank < k ? maxrank : k);
     /* FP64 buffers, factors, int8 Omega, int8 digit planes of Q */
-    return sizeof(double)*((size_t)m*k+2*(size_t)n*k+4*(size_t)k*k+
+    return sizeof(double)*((size_t)m*k+2*(size_t)n*k+(size_t)k*k+
+            (size_t)(k+15)*(k+63)+16+(size_t)k*r+
             (size_t)k+(size_t)(m+n)*r)+(size_t)(n+63)*k+
         4*(size_t)(m+63)*(size_t)(k+15)+8*(size_t)(k+15);
 }
@@ -716,6 +717,9 @@ int hip_driver_run(const hip_batch *B, STARSH_int ntiles, const int *pidx,
         {
             in.S_out = S_out;
             in.soff = so+b0;
+            /* the rounds of the mixed form steer by the singular values of
+             * tiles that are not final, and the widest are */
+            in.sv_rounds = 1;
         }
         if(x)
         {

@@ -1,0 +1,604 @@
+// Core SVD of the tiles whose p x p core does not fit in LDS (p >
+// CORE_LDS_PMAX, core.hip): one-sided block Jacobi with the work of every tile spread over
+// the chip.
+//
+// The columns of W = R2^T are split into blocks of 32.  A sweep visits every
+// pair of blocks once, in rounds of disjoint pairs (circle method), one
+// launch per round and one workgroup per block pair and tile:
+//   1. Gram matrix G (64 x 64) of the pair's columns on FP64 MFMA;
+//   2. one sweep of two-sided Jacobi on G in LDS, all 32 disjoint column
+//      pairs of a step at once, the rotations accumulated in J (64 x 64);
+//   3. W_pair <- W_pair J on FP64 MFMA (skipped when nothing rotated).
+// The rotations and the test |g_ij| > p eps |w_i| |w_j| are those of the
+// scalar one-sided method; G is formed afresh from the columns at every
+// visit, so its rounding never accumulates, and J is a product of exact-
+// to-rounding rotations whose large entries only mix columns of like norm,
+// so the small columns of a graded W keep their relative accuracy.  A sweep
+// without rotations ends a tile.
+//
+// What bounds it: a workgroup per tile (the scalar method with column
+// blocks in LDS, one rotation per half-wave) left the chip idle below 256
+// tiles and paid LDS traffic of O(p) per rotation; here a rotation costs
+// O(64) LDS traffic and the O(p) work is MFMA.  The inner Jacobi is bound by
+// LDS bandwidth (128 KB per step of 32 rotations).  Blocks of 32 keep G and
+// J (65 KB) at two workgroups per CU; the whole 63-step sweep over the 64
+// columns converges in 6 outer sweeps where 32 cross steps per visit need
+// 7-8 (numpy model on sin(kr)/r, exp and Matern cores).
+// Measured on MI355X, all launches of one compression, against one
+// workgroup per tile: 2D exp N=9973, tile 1000, SVD engine (10 cores of
+// 1000, 45 of 200-500) 1570 -> 32 ms; sin(kr)/r N=25000, tile 1536 (17 of
+// 400, 85 of 130-210) 163 -> 12 ms; 3D Matern N=65536, tile 2048, mixed
+// (up to 528) 191 -> 81 ms; a round of 500 pairs takes 120-160 us, of 1700
+// pairs 280 us.
+#include <float.h>
+#include <math.h>
+#include "pipeline.h"
+#include "jacobi_rotation.h"
+
+typedef double double4_t __attribute__((ext_vector_type(4)));
+
+namespace {
+
+constexpr int BW = 32;          // columns per block
+constexpr int PW = 2*BW;        // columns per block pair
+constexpr int NT = 256;
+
+__device__ inline int ld_of(int p)
+{
+    return (p+15)/16*16;
+}
+
+// Number of column blocks, rounded up to even (the last may be empty).
+__device__ inline int blocks_of(int p)
+{
+    const int nb = (p+BW-1)/BW;
+    return nb+(nb & 1);
+}
+
+// jacobi_rotation() with two reciprocal square roots and no division: with
+// d = be - al, h = 2 ga and r = sqrt(d^2 + h^2), c^2 = (1 + |d|/r)/2 and
+// s = sign(d) h/(2 r c), the smaller of the two angles.  Outside the range
+// where the squares are safe it is jacobi_rotation() itself.
+__device__ inline void rotation(double al, double be, double ga, double &c,
+        double &s)
+{
+    const double d = be-al, h = 2.0*ga;
+    const double big = fmax(fabs(d), fabs(h));
+    if(big >= 1e-140 && big < 1e140)
+    {
+        const double ir = rsqrt(fma(d, d, h*h));
+        const double q = fma(0.5*fabs(d), ir, 0.5);
+        const double y = rsqrt(q);
+        c = q*y;
+        s = (d >= 0.0 ? 0.5 : -0.5)*h*ir*y;
+    }
+    else
+        jacobi_rotation(al, be, ga, c, s);
+}
+
+// Exponent of the scale of W and the start of a tile's Jacobi state.
+__global__ __launch_bounds__(256) void jb_max_kernel(TileDesc *tiles,
+        const double *ws, int lds_p)
+{
+    TileDesc &td = tiles[blockIdx.x];
+    const int p = td.p, k = td.k;
+    if(p <= lds_p)
+        return;
+    __shared__ double part[4];
+    const double *R2 = ws+td.r_off;
+    double v = 0.0;
+    // R2 is upper triangular up to rounding, but every entry is taken
+    for(int c = threadIdx.x >> 6; c < p; c += 4)
+        for(int i = threadIdx.x & 63; i < p; i += 64)
+            v = fmax(v, fabs(R2[(int64_t)c*k+i]));
+    for(int o = 32; o > 0; o >>= 1)
+        v = fmax(v, __shfl_xor(v, o, 64));
+    if((threadIdx.x & 63) == 0)
+        part[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if(threadIdx.x == 0)
+    {
+        const double wm = fmax(fmax(part[0], part[1]), fmax(part[2],
+                    part[3]));
+        int e = 0;
+        if(wm > 0.0 && wm < INFINITY)
+            frexp(wm, &e);
+        td.wexp = e;
+        td.jrot = 0;
+        td.jdone = 0;
+        td.sweeps = 0;
+        td.off2 = 0.0;
+    }
+}
+
+// W = R2^T 2^-wexp (the power of two that brings the largest entry into
+// [1/2, 1), exact), rows padded to 16 and columns to 64 with zeros: zero
+// columns never rotate.  One 32 x 32 patch per workgroup, transposed in
+// LDS.
+__global__ __launch_bounds__(256) void jb_init_kernel(const TileDesc *tiles,
+        double *ws, int lds_p)
+{
+    const TileDesc &td = tiles[blockIdx.y];
+    const int p = td.p, k = td.k;
+    if(p <= lds_p)
+        return;
+    const int ld = ld_of(p), nc = blocks_of(p)*BW;
+    const int pr = (ld+31)/32;
+    const int bi = blockIdx.x % pr, bj = blockIdx.x / pr;
+    if(bj*32 >= nc)
+        return;
+    const double *R2 = ws+td.r_off;
+    double *W = ws+td.j_off;
+    const double scale = ldexp(1.0, -td.wexp);
+    __shared__ double patch[32][33];
+    const int x = threadIdx.x & 31, y = threadIdx.x >> 5;
+    // W(i, j) = R2(j, i): column i of R2 is read along j
+    for(int r = y; r < 32; r += 8)
+    {
+        const int i = bi*32+r, j = bj*32+x;
+        patch[r][x] = i < p && j < p ? R2[(int64_t)i*k+j]*scale : 0.0;
+    }
+    __syncthreads();
+    for(int r = y; r < 32; r += 8)
+    {
+        const int i = bi*32+x, j = bj*32+r;
+        if(i < ld)
+            W[(int64_t)j*ld+i] = patch[x][r];
+    }
+}
+
+// One round of a sweep: workgroup (x, tile) handles pair x of the circle
+// method on the tile's column blocks.
+__global__ __launch_bounds__(NT, 2) void jb_round_kernel(TileDesc *tiles,
+        double *ws, int lds_p, int round)
+{
+    __shared__ double G[PW*PW];
+    __shared__ double J[PW*PW];
+    __shared__ int perm[PW];
+    TileDesc &td = tiles[blockIdx.y];
+    const int p = td.p;
+    if(p <= lds_p || td.jdone)
+        return;
+    const int nbe = blocks_of(p);
+    const int x = blockIdx.x, y = nbe-1-x;
+    if(round >= nbe-1 || x >= nbe/2)
+        return;
+    const int bi = x == 0 ? 0 : 1+(x-1+round) % (nbe-1);
+    const int bj = 1+(y-1+round) % (nbe-1);
+    const int ld = ld_of(p);
+    double *W = ws+td.j_off;
+    double *WI = W+(int64_t)bi*BW*ld, *WJ = W+(int64_t)bj*BW*ld;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lc = lane & 15, lr = lane >> 4;
+    const int nrb = ld/16;
+
+    // ---- 1. G = [WI WJ]^T [WI WJ], rows split over the waves in blocks of
+    // 16.  A and B operand have the same layout (lane: column lane%16, row
+    // lane/16 of a step); any order of the rows gives the same sum, so a
+    // lane takes rows 4 (lane/16) .. +3 of the block in its four steps and
+    // loads 32 contiguous bytes.
+    double4_t g[10];
+#pragma unroll
+    for(int t = 0; t < 10; t++)
+        g[t] = double4_t{0.0, 0.0, 0.0, 0.0};
+    for(int rb = wave; rb < nrb; rb += 4)
+    {
+        double f[4][4];
+#pragma unroll
+        for(int c = 0; c < 4; c++)
+        {
+            const double *src = (c < 2 ? WI : WJ)+
+                (int64_t)((c & 1)*16+lc)*ld+rb*16+4*lr;
+#pragma unroll
+            for(int v = 0; v < 4; v++)
+                f[c][v] = src[v];
+        }
+#pragma unroll
+        for(int v = 0; v < 4; v++)
+        {
+            int t = 0;
+#pragma unroll
+            for(int a = 0; a < 4; a++)
+#pragma unroll
+                for(int b = a; b < 4; b++, t++)
+                    g[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(f[a][v],
+                            f[b][v], g[t], 0, 0, 0);
+        }
+    }
+    // sum over the waves in a fixed order: (0 + 2) + (1 + 3), through G and
+    // J as scratch
+    auto put = [&](double *dst) {
+#pragma unroll
+        for(int t = 0; t < 10; t++)
+#pragma unroll
+            for(int v = 0; v < 4; v++)
+                dst[(t*4+v)*64+lane] = g[t][v];
+    };
+    auto add = [&](const double *src) {
+#pragma unroll
+        for(int t = 0; t < 10; t++)
+#pragma unroll
+            for(int v = 0; v < 4; v++)
+                g[t][v] += src[(t*4+v)*64+lane];
+    };
+    if(wave == 2)
+        put(G);
+    if(wave == 3)
+        put(J);
+    __syncthreads();
+    if(wave == 0)
+        add(G);
+    if(wave == 1)
+    {
+        add(J);
+        put(J);
+    }
+    __syncthreads();
+    if(wave == 0)
+    {
+        add(J);
+        int t = 0;
+#pragma unroll
+        for(int a = 0; a < 4; a++)
+#pragma unroll
+            for(int b = a; b < 4; b++, t++)
+#pragma unroll
+                for(int v = 0; v < 4; v++)
+                {
+                    // D layout: row lane/16 + 4 v, column lane%16
+                    const int i = a*16+lr+4*v, j = b*16+lc;
+                    G[i*PW+j] = g[t][v];
+                    if(b > a)
+                        G[j*PW+i] = g[t][v];
+                }
+    }
+    __syncthreads();
+    for(int e = threadIdx.x; e < PW*PW; e += NT)
+        J[e] = (e & (PW-1)) == (e >> 6) ? 1.0 : 0.0;
+
+    // ---- 2. one sweep of Jacobi on G.  Lane l of every wave computes the
+    // rotation of column pair l%32 of the step (so the step needs no
+    // exchange of rotations between waves); the 2 x 2 blocks (row pair i,
+    // column pair j = l%32) and the rows of J are split over the waves.  J
+    // is one step behind, so that its LDS traffic overlaps the latency of
+    // the next rotations.
+    const double ctol = (double)p*DBL_EPSILON;
+    const int pj = lane & 31, half = lane >> 5;
+    bool rotated = false;
+    const int a0 = pj, b0 = PW-1-pj;    // positions of the pair at step 0
+    double pc = 1.0, ps = 0.0;          // rotation J has not seen yet
+    int pa = 0, pb = 1;
+    __syncthreads();
+    for(int step = 0; step < PW-1; step++)
+    {
+        const int ca = a0 == 0 ? 0 : 1+(a0-1+step) % (PW-1);
+        const int cb = 1+(b0-1+step) % (PW-1);
+        const double al = G[ca*PW+ca], be = G[cb*PW+cb];
+        const double ga = G[ca*PW+cb];
+        // J <- J R of the previous rotating step
+#pragma unroll
+        for(int q = 0; q < 8; q++)
+        {
+            double *row = J+(wave*16+q*2+half)*PW;
+            const double u = row[pa], v = row[pb];
+            row[pa] = pc*u-ps*v;
+            row[pb] = ps*u+pc*v;
+        }
+        pc = 1.0;
+        ps = 0.0;
+        double c = 1.0, s = 0.0;
+        const bool rot = jr_rotates(al, be, ga, ctol);
+        if(rot)
+            rotation(al, be, ga, c, s);
+        if(__ballot(rot) == 0)
+            continue;               // the same in every wave
+        rotated = true;
+        // every wave has read its rotations before G changes
+        __syncthreads();
+        // G <- R^T G R
+#pragma unroll
+        for(int q = 0; q < 4; q++)
+        {
+            const int i = wave*8+q*2+half;      // row pair
+            const int ra = __shfl(ca, i, 64), rb = __shfl(cb, i, 64);
+            const double ci = __shfl(c, i, 64), si = __shfl(s, i, 64);
+            const double gaa = G[ra*PW+ca], gab = G[ra*PW+cb];
+            const double gba = G[rb*PW+ca], gbb = G[rb*PW+cb];
+            const double xaa = c*gaa-s*gab, xab = s*gaa+c*gab;
+            const double xba = c*gba-s*gbb, xbb = s*gba+c*gbb;
+            double yab = ci*xab-si*xbb, yba = si*xaa+ci*xba;
+            if(i == pj && rot)
+                yab = yba = 0.0;
+            G[ra*PW+ca] = ci*xaa-si*xba;
+            G[ra*PW+cb] = yab;
+            G[rb*PW+ca] = yba;
+            G[rb*PW+cb] = si*xab+ci*xbb;
+        }
+        pc = c;
+        ps = s;
+        pa = ca;
+        pb = cb;
+        __syncthreads();
+    }
+    if(!rotated)
+        return;
+#pragma unroll
+    for(int q = 0; q < 8; q++)
+    {
+        double *row = J+(wave*16+q*2+half)*PW;
+        const double u = row[pa], v = row[pb];
+        row[pa] = pc*u-ps*v;
+        row[pb] = ps*u+pc*v;
+    }
+    if(threadIdx.x == 0)
+        atomicAdd(&td.jrot, 1);
+    // the columns leave sorted by norm, the larger ones to the first block:
+    // clusters of nearly equal singular values (a diagonal tile of points
+    // on equal spheres) converge in 14-16 sweeps sorted and 26 unsorted
+    if(threadIdx.x < PW)
+    {
+        const double v = G[threadIdx.x*(PW+1)];
+        int pos = 0;
+        for(int l = 0; l < PW; l++)
+        {
+            const double o = G[l*(PW+1)];
+            pos += o > v || (o == v && l < (int)threadIdx.x);
+        }
+        perm[bi < bj ? pos : pos^BW] = threadIdx.x;
+    }
+    __syncthreads();
+
+    // ---- 3. W_pair <- W_pair J, rows split over the waves in blocks of
+    // 16; each wave reads all columns of its rows before it writes them.
+    // J is held as B operand in registers (16 steps of 4 rows x 4 column
+    // groups).  Logical row i of the block is physical row 4 (i%4) + i/4,
+    // so that the output lane stores 4 consecutive rows.
+    double jb[16][4];
+#pragma unroll
+    for(int q = 0; q < 16; q++)
+#pragma unroll
+        for(int n = 0; n < 4; n++)
+            jb[q][n] = J[(4*q+lr)*PW+perm[16*n+lc]];
+    const int prow = 4*(lc & 3)+(lc >> 2);
+    for(int rb = wave; rb < nrb; rb += 4)
+    {
+        double4_t acc[4];
+#pragma unroll
+        for(int n = 0; n < 4; n++)
+            acc[n] = double4_t{0.0, 0.0, 0.0, 0.0};
+        double a[16];
+#pragma unroll
+        for(int q = 0; q < 16; q++)
+            a[q] = (q < 8 ? WI : WJ)[(int64_t)(4*(q & 7)+lr)*ld+rb*16+prow];
+#pragma unroll
+        for(int q = 0; q < 16; q++)
+#pragma unroll
+            for(int n = 0; n < 4; n++)
+                acc[n] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q], jb[q][n],
+                        acc[n], 0, 0, 0);
+#pragma unroll
+        for(int n = 0; n < 4; n++)
+        {
+            double *dst = (n < 2 ? WI : WJ)+(int64_t)((n & 1)*16+lc)*ld+
+                rb*16+4*lr;
+#pragma unroll
+            for(int v = 0; v < 4; v++)
+                dst[v] = acc[n][v];
+        }
+    }
+}
+
+// Whether the tile may end with the verdict "rank above the limit" alone
+// (its singular values are not asked for), and that limit.
+__device__ inline bool rank_limit(const TileDesc &td, int lds_p, int &limit)
+{
+    const int mn = td.m < td.n ? td.m : td.n;
+    limit = td.maxrank;
+    if((td.rule & RSDD_RULE_HALF) && mn/2-1 < limit)
+        limit = mn/2-1;
+    return td.nosv && td.p > lds_p && !td.jdone && td.p > limit;
+}
+
+// Squared norms of W's columns (to the tile's S) and the sum of the squares
+// of the Gram matrix's strict upper triangle (td.off2): one workgroup per
+// block pair I <= J.
+__global__ __launch_bounds__(NT) void jb_off_kernel(TileDesc *tiles,
+        double *ws, int lds_p)
+{
+    __shared__ double part[3][16*64];
+    TileDesc &td = tiles[blockIdx.y];
+    int limit;
+    if(!rank_limit(td, lds_p, limit))
+        return;
+    const int p = td.p, nb = (p+BW-1)/BW;
+    int bi = 0, rest = blockIdx.x;
+    while(bi < nb && rest >= nb-bi)
+        rest -= nb-bi++;
+    if(bi >= nb)
+        return;
+    const int bj = bi+rest, ld = ld_of(p);
+    const double *WI = ws+td.j_off+(int64_t)bi*BW*ld;
+    const double *WJ = ws+td.j_off+(int64_t)bj*BW*ld;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lc = lane & 15, lr = lane >> 4;
+    double4_t g[2][2];
+#pragma unroll
+    for(int a = 0; a < 2; a++)
+#pragma unroll
+        for(int b = 0; b < 2; b++)
+            g[a][b] = double4_t{0.0, 0.0, 0.0, 0.0};
+    for(int rb = wave; rb < ld/16; rb += 4)
+#pragma unroll
+        for(int v = 0; v < 4; v++)
+        {
+            double fa[2], fb[2];
+#pragma unroll
+            for(int c = 0; c < 2; c++)
+            {
+                fa[c] = WI[(int64_t)(c*16+lc)*ld+rb*16+4*lr+v];
+                fb[c] = WJ[(int64_t)(c*16+lc)*ld+rb*16+4*lr+v];
+            }
+#pragma unroll
+            for(int a = 0; a < 2; a++)
+#pragma unroll
+                for(int b = 0; b < 2; b++)
+                    g[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[a],
+                            fb[b], g[a][b], 0, 0, 0);
+        }
+    if(wave > 0)
+#pragma unroll
+        for(int t = 0; t < 16; t++)
+            part[wave-1][t*64+lane] = g[t >> 3][(t >> 2) & 1][t & 3];
+    __syncthreads();
+    if(wave > 0)
+        return;
+    double off = 0.0;
+#pragma unroll
+    for(int t = 0; t < 16; t++)
+    {
+        const int a = t >> 3, b = (t >> 2) & 1, v = t & 3;
+        const double x = ((g[a][b][v]+part[0][t*64+lane])+
+                part[1][t*64+lane])+part[2][t*64+lane];
+        const int i = bi*BW+a*16+lr+4*v, j = bj*BW+b*16+lc;
+        if(i < j)
+            off += x*x;
+        else if(i == j && i < p)
+            ws[td.s_off+i] = x;
+    }
+    for(int o = 32; o > 0; o >>= 1)
+        off += __shfl_xor(off, o, 64);
+    if(lane == 0)
+        atomicAdd(&td.off2, off);
+}
+
+// Ends the tiles whose rank is certainly above the limit.  With d the
+// squared column norms of W in descending order and E the off-diagonal part
+// of W^T W, Hoffman and Wielandt's theorem gives sum |lambda_i - d_i|^2 <=
+// |E|_F^2, so the energy past the limit, sum_{i > limit} lambda_i, is at
+// least sum_{i > limit} d_i - sqrt(p - limit) |E|_F.  Twice the energy that
+// the rank rule allows (tol^2 of the total) is asked for, far more than any
+// rounding, so the verdict is the one the converged singular values give.
+__global__ __launch_bounds__(256) void jb_cert_kernel(TileDesc *tiles,
+        const double *ws, int lds_p)
+{
+    __shared__ double d[1024];
+    __shared__ double part[2][4];
+    TileDesc &td = tiles[blockIdx.x];
+    int limit;
+    if(!rank_limit(td, lds_p, limit))
+        return;
+    const int p = td.p;
+    for(int i = threadIdx.x; i < p; i += 256)
+        d[i] = ws[td.s_off+i];
+    __syncthreads();
+    double tail = 0.0, total = 0.0;
+    for(int i = threadIdx.x; i < p; i += 256)
+    {
+        const double v = d[i];
+        int pos = 0;
+        for(int l = 0; l < p; l++)
+            pos += d[l] > v || (d[l] == v && l < i);
+        total += v;
+        if(pos >= limit)
+            tail += v;
+    }
+    for(int o = 32; o > 0; o >>= 1)
+    {
+        tail += __shfl_xor(tail, o, 64);
+        total += __shfl_xor(total, o, 64);
+    }
+    if((threadIdx.x & 63) == 0)
+    {
+        part[0][threadIdx.x >> 6] = tail;
+        part[1][threadIdx.x >> 6] = total;
+    }
+    __syncthreads();
+    if(threadIdx.x == 0)
+    {
+        const double t2 = ldexp(td.tail2, -2*td.wexp);
+        tail = part[0][0]+part[0][1]+part[0][2]+part[0][3]+t2;
+        total = part[1][0]+part[1][1]+part[1][2]+part[1][3]+t2;
+        const double low = tail-sqrt(2.0*td.off2*(p-limit));
+        if(low > 2.0*td.tol*td.tol*total && low > 1e-12*total)
+            td.jdone = 2;
+        td.off2 = 0.0;
+    }
+}
+
+// End of a sweep: tiles without a rotation are done; *active counts the
+// tiles that are not.
+__global__ __launch_bounds__(256) void jb_sweep_kernel(TileDesc *tiles,
+        int ntiles, int lds_p, int *active)
+{
+    int c = 0;
+    for(int t = threadIdx.x; t < ntiles; t += blockDim.x)
+    {
+        TileDesc &td = tiles[t];
+        if(td.p <= lds_p || td.jdone)
+            continue;
+        if(td.jrot == 0)
+            td.jdone = 1;
+        else
+        {
+            td.sweeps++;
+            td.jrot = 0;
+            c++;
+        }
+    }
+    for(int o = 32; o > 0; o >>= 1)
+        c += __shfl_xor(c, o, 64);
+    __shared__ int part[4];
+    if((threadIdx.x & 63) == 0)
+        part[threadIdx.x >> 6] = c;
+    __syncthreads();
+    if(threadIdx.x == 0)
+        *active = part[0]+part[1]+part[2]+part[3];
+}
+
+} // namespace
+
+// Jacobi sweeps on every tile with p > lds_p: W (columns orthogonal on
+// return) in the tile's j_off region, ld = p rounded up to 16, scaled by
+// 2^-wexp, td.jdone 1; tiles that ended early with a rank certainly above
+// the limit have jdone 2, tiles that did not converge 0.  certify: some
+// tile may end that way.  h_active: pinned host int.
+int pipeline_jacobi_block(TileDesc *d_tiles, int ntiles, double *ws,
+        int lds_p, int pmax, int max_sweeps, bool certify, int *d_active,
+        int *h_active, hipStream_t s)
+{
+    const int nb = (pmax+BW-1)/BW, nbe = nb+(nb & 1);
+    const int patches = (pmax+31)/32*nbe;
+    hipLaunchKernelGGL(jb_max_kernel, dim3(ntiles), dim3(256), 0, s, d_tiles,
+            ws, lds_p);
+    hipLaunchKernelGGL(jb_init_kernel, dim3(patches, ntiles), dim3(256), 0,
+            s, d_tiles, ws, lds_p);
+    HIP_TRY(hipGetLastError());
+    for(int sweep = 0; sweep < max_sweeps; sweep++)
+    {
+        for(int round = 0; round < nbe-1; round++)
+            hipLaunchKernelGGL(jb_round_kernel, dim3(nbe/2, ntiles),
+                    dim3(NT), 0, s, d_tiles, ws, lds_p, round);
+        // tiles headed for a rank above the limit: two sweeps are enough for
+        // most, the others are tried again
+        if(certify && (sweep == 1 || sweep == 3 || sweep == 6))
+        {
+            hipLaunchKernelGGL(jb_off_kernel, dim3(nb*(nb+1)/2, ntiles),
+                    dim3(NT), 0, s, d_tiles, ws, lds_p);
+            hipLaunchKernelGGL(jb_cert_kernel, dim3(ntiles), dim3(256), 0,
+                    s, d_tiles, ws, lds_p);
+        }
+        hipLaunchKernelGGL(jb_sweep_kernel, dim3(1), dim3(256), 0, s,
+                d_tiles, ntiles, lds_p, d_active);
+        HIP_TRY(hipGetLastError());
+        // no core of this size converges in two sweeps unless it was
+        // diagonal from the start
+        if(sweep < 1)
+            continue;
+        HIP_TRY(hipMemcpyAsync(h_active, d_active, sizeof(int),
+                    hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+        if(*h_active == 0)
+            break;
+    }
+    return STARSH_SUCCESS;
+}

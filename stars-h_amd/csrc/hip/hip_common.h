@@ -73,6 +73,7 @@ struct TileDesc
     int64_t bt_off;    // Bt = A^T Q (n x k, ld n)
     int64_t q2_off;    // Q2 (n x k, ld n)
     int64_t r_off;     // R2 (k x k, ld k)
+    int64_t j_off;     // working matrix of a core beyond LDS
     int64_t w_off;     // X_r (p x r, ld p): left singular vectors of B
     int64_t s_off;     // singular values, k entries
     int64_t u_off;     // U (m x maxrank, ld m)
@@ -98,6 +99,12 @@ struct TileDesc
     int64_t sel_off;   // selected columns (RSDD_RULE_SELECT), k ints
     int64_t piv_off;   // column pivots of B (piv_k ints), -1: none
     int piv_k;
+    // block Jacobi of a core beyond LDS: exponent of W's scale, rotations
+    // in the current sweep, finished, sweeps with rotations
+    int wexp, jrot, jdone, sweeps;
+    int nosv;          // singular values not asked for: a rank above the
+                       // limit may be decided before they have converged
+    double off2;       // squares of the Gram matrix's upper triangle
 };
 
 __device__ inline double matern_closed(double nu, double x)

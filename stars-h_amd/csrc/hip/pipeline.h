@@ -89,10 +89,26 @@ int pipeline_qdigits(const TileDesc *d_tiles, int ntiles, int kmax,
 int pipeline_proj_i8(const TileDesc *d_tiles, int ntiles, int nmax, int kmax,
         const GemmArgs &g, const signed char *d_qd, hipStream_t s);
 
+// Largest core kept in LDS by one workgroup; larger ones (up to 1024) are
+// rotated in the tile's j_off region (core_block.hip).
+constexpr int CORE_LDS_PMAX = 128;
+
+// Doubles of a tile's j_off region for a core of up to p rows.
+inline int64_t core_work_doubles(int p)
+{
+    return p <= CORE_LDS_PMAX ? 0 :
+        (int64_t)((p+15)/16*16)*((p+63)/64*64);
+}
+
 // One-sided Jacobi SVD of R2, singular values, rank by the reference rule
-// (each tile's own maxrank and tol) and X_r.
+// (each tile's own maxrank and tol) and X_r.  certify: some tile with nosv
+// has p above its rank limit.  d_active: a device int, h_active: a pinned
+// host int.
 int pipeline_core(TileDesc *d_tiles, int ntiles, double *ws, int pmax,
-        hipStream_t s);
+        bool certify, int *d_active, int *h_active, hipStream_t s);
+int pipeline_jacobi_block(TileDesc *d_tiles, int ntiles, double *ws,
+        int lds_p, int pmax, int max_sweeps, bool certify, int *d_active,
+        int *h_active, hipStream_t s);
 
 // Exact engines (exact.hip): sketch Y = A[:, sel] (RSDD_RULE_SELECT tiles,
 // k columns from d_sel at each tile's sel_off), and the first piv_k column

@@ -393,6 +393,9 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
             d.k = mn;
         if(d.k < 1)
             d.k = 1;
+        const int kfull = pr.maxrank+pr.oversample;
+        d.nosv = in->S_out == nullptr || (in->sv_rounds &&
+                d.k >= (kfull < mn ? kfull : mn));
         d.gen = in->d_a == nullptr;
         d.rule = in->rule;
         d.sel_off = in->sel_off ? in->sel_off[t] : 0;
@@ -451,8 +454,11 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
         d.q_off = off; off += m*k;
         d.bt_off = off; off += n*k;
         d.q2_off = off; off += n*k;
-        d.r_off = off; off += 2*k*k;
-        d.w_off = off; off += 2*k*k;
+        d.r_off = off; off += k*k;
+        off = (off+15)/16*16;
+        d.j_off = off;
+        off += core_work_doubles((int)(k < CORE_PMAX ? k : CORE_PMAX));
+        d.w_off = off; off += k*rmax;
         d.s_off = off; off += k;
         d.u_off = uvoff; uvoff += m*rmax;
         d.v_off = uvoff; uvoff += n*rmax;
@@ -597,9 +603,12 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
     // to its tail, as for the truncation itself, so the rank rule stays
     // conservative (flag 8).
     int pmax = 0;
-    bool capped = false;
+    bool capped = false, certify = false;
     for(int t = 0; t < nt; t++)
     {
+        const int half = (h[t].m < h[t].n ? h[t].m : h[t].n)/2-1;
+        certify |= h[t].nosv && (h[t].p > h[t].maxrank ||
+                ((h[t].rule & RSDD_RULE_HALF) && h[t].p > half));
         if(h[t].p > CORE_PMAX)
         {
             std::vector<double> nb(h[t].p-CORE_PMAX);
@@ -632,7 +641,9 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
         dump("R2", d_ws+h[0].r_off, (int64_t)h[0].k*h[0].k, s);
     }
     // 6. core SVD and rank
-    TRY(pipeline_core(d_tiles, nt, d_ws, pmax, s));
+    TRY(probe.init());
+    TRY(pipeline_core(d_tiles, nt, d_ws, pmax, certify, (int *)active.p,
+                probe.h, s));
     HIP_TRY(hipMemcpyAsync(h.data(), d_tiles, sizeof(TileDesc)*nt,
                 hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));

@@ -50,6 +50,8 @@ typedef struct rsdd_input
                                     columns (0: 1e-13) */
     double *S_out;               /* optional: k singular values per tile */
     const int64_t *soff;
+    int sv_rounds;               /* S_out is only read for tiles narrower
+                                    than min(maxrank+oversample, m, n) */
     int *rows_out;               /* optional: sketch width k per tile */
     /* Exact engines (SDD, RRQR): RSDD_RULE_HALF also declares a tile
      * false far-field when 2 rank >= min(m, n) (dsdd.c:53, dqp3.c:84);
