@@ -193,10 +193,10 @@ int starsh_hip_fp64_probe(double *mfma_tflops, double *valu_tflops);
  *                         size, default), 64, 128 or 256;
  *   "gemm_rw"             16-row groups per wave of those GEMMs: 0 (by
  *                         size, default), 1 or 2;
- *   "qr_panel"            panel width of the block Gram-Schmidt: 0 (by
- *                         batch, default: 8 columns for batches of more
- *                         than 1536 tiles), 4 or 8 (8 only for tiles of
- *                         at most 2048 rows);
+ *   "qr_panel"            panel width inside the blocks of the block
+ *                         Gram-Schmidt: 0 (by size, default), 4 or 8 (8,
+ *                         the default there, only for tiles of at most
+ *                         2048 rows);
  *   "proj_int8"           projection B^T = A^T Q of the mixed form on
  *                         int8 digit planes of both operands (1, default)
  *                         or on FP64 MFMA (0);

@@ -620,7 +620,7 @@ static size_t tile_bytes(int m, int n, int k, int maxrank)
     /* FP64 buffers, factors, int8 Omega, int8 digit planes of Q */
     return sizeof(double)*((size_t)m*k+2*(size_t)n*k+(size_t)k*k+
             (size_t)(k+15)*(k+63)+16+(size_t)k*r+
-            (size_t)k+(size_t)(m+n)*r)+(size_t)(n+63)*k+
+            (size_t)33*k+(size_t)(m+n)*r)+(size_t)(n+63)*k+
         4*(size_t)(m+63)*(size_t)(k+15)+8*(size_t)(k+15);
 }
 

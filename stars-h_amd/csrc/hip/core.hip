@@ -366,11 +366,12 @@ int pipeline_core(TileDesc *d_tiles, int ntiles, double *ws, int pmax,
         return STARSH_WRONG_PARAMETER;
     const int pm = pmax > 0 ? pmax : 1;
     const int lds_p = pm <= CORE_LDS_PMAX ? pm : CORE_LDS_PMAX;
-    // Up to 64 rows four waves keep a group of 8 or more lanes per column
-    // pair and leave room for other tiles on the CU; above, W fills most of
-    // the LDS, one workgroup runs per CU, and sixteen waves take half the
-    // time (55 cores of 40-110 rows: 4.8 -> 2.4 ms).
-    if(lds_p <= 64)
+    // Four waves per tile keep a group of 8 or more lanes per column pair up
+    // to 64 rows and leave room for other tiles on the CU; above, and with
+    // few tiles, W fills the LDS or the chip is not full and sixteen waves
+    // win (55 cores of 40-110 rows: 4.8 -> 2.4 ms; 820 of 34-96: 2.2
+    // against 2.7 ms, so they keep four).
+    if(lds_p <= 64 || (lds_p <= 96 && ntiles > 512))
     {
         const int info = launch_core<256>(d_tiles, ntiles, ws, lds_p,
                 jacobi_max_sweeps, s);

@@ -104,6 +104,9 @@ struct TileDesc
     int wexp, jrot, jdone, sweeps;
     int nosv;          // singular values not asked for: a rank above the
                        // limit may be decided before they have converged
+    // Gram-Schmidt: the block last taken by the first pass, end of its kept
+    // range
+    int gs_blk, gs_end;
     double off2;       // squares of the Gram matrix's upper triangle
 };
 

@@ -41,18 +41,24 @@ int pipeline_gen_gemm(int proj, const TileDesc *d_tiles, int ntiles,
 int pipeline_colnorm(const TileDesc *d_tiles, int ntiles, int which,
         double *ws, double *d_norm, int kmax, hipStream_t s);
 
-// Block Gram-Schmidt applied twice for a panel of jb columns at j0 (each
-// pass: projection against the previous columns, then CGS2 inside the
-// panel with deflation).  which: 0 = Q (width k), 1 = Q2 (width p; the
-// panel is read from Bt and written to Q2).  Columns whose norm after
-// projection is at most tau_first times their original norm in the first
-// pass, or tau_second in the second, are set to zero and flagged in
-// d_keep.  A tile whose whole panel was dropped in the first pass is marked
-// done; *d_active counts the tiles that still have panels to process.
-int pipeline_panel(const TileDesc *d_tiles, int ntiles, int which,
-        double *ws, int j0, int jb, int kmax, double tau_first,
-        double tau_second, int *d_keep, int rows_max, int *d_active,
-        hipStream_t s);
+// Block Gram-Schmidt applied twice for the GS_BLOCK columns at j0 (a
+// multiple of GS_BLOCK), in panels of pb (qr.hip).  which: 0 = Q (width k),
+// 1 = Q2 (width p; the columns are read from Bt and written to Q2).  Columns
+// whose norm after projection is at most tau_first times their original norm
+// in the first pass, or tau_second in the second, are set to zero and
+// flagged in d_keep.  A tile whose whole panel was dropped in the first pass
+// is marked done; *d_active counts the tiles that still have blocks to
+// process.  d_norms: ntiles x kmax doubles, d_coef: ntiles x kmax x GS_BLOCK.
+// The first block (j0 = 0) takes GS_FIRST columns.
+constexpr int GS_BLOCK = 32, GS_FIRST = 64;
+inline int gs_next(int j0)
+{
+    return j0+(j0 == 0 ? GS_FIRST : GS_BLOCK);
+}
+int pipeline_gs_block(TileDesc *d_tiles, int ntiles, int which, double *ws,
+        int j0, int pb, int kmax, double tau_first, double tau_second,
+        int *d_keep, double *d_norms, double *d_coef, int rows_max,
+        int *d_active, hipStream_t s);
 
 // *d_active = number of tiles with a nonzero width (k or p).
 int pipeline_count_active(const TileDesc *d_tiles, int ntiles, int which,

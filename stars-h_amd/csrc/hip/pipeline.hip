@@ -76,7 +76,7 @@ struct Pool
 Pool ws_pool, uv_pool, pack_pool, stage_pool{nullptr, 0, true};
 // The small per-batch buffers (tile descriptors, kept-column flags, norms,
 // int8 Omega and digit planes, counters, R2 partials, selected columns,
-// pivots), kept too: a hipMalloc / hipFree pair per buffer and batch cost
+// pivots, Gram-Schmidt coefficients), kept too: a hipMalloc / hipFree pair per buffer and batch cost
 // host time on every call, and hipFree waits for the device.
 constexpr size_t SMALL_UNIT = (size_t)1 << 20;
 Pool tiles_pool{nullptr, 0, false, SMALL_UNIT},
@@ -87,14 +87,15 @@ Pool tiles_pool{nullptr, 0, false, SMALL_UNIT},
      qd_pool{nullptr, 0, false, SMALL_UNIT},
      part_pool{nullptr, 0, false, SMALL_UNIT},
      sel_pool{nullptr, 0, false, SMALL_UNIT},
-     piv_pool{nullptr, 0, false, SMALL_UNIT};
+     piv_pool{nullptr, 0, false, SMALL_UNIT},
+     coef_pool{nullptr, 0, false, SMALL_UNIT};
 
 // Host view of the device counter of tiles still in a BCGS2 run.  The
-// counter is copied to pinned memory after every panel; the host reads it
-// LAG panels later (so the stream always holds queued work) and stops
-// launching once no tile is left.
-constexpr int LAG = 3;
-constexpr int NSLOT = 4;
+// counter is copied to pinned memory after every block of columns; the host
+// reads it LAG blocks later (so the stream always holds queued work) and
+// stops launching once no tile is left.
+constexpr int LAG = 1;
+constexpr int NSLOT = 2;
 
 struct ActiveProbe
 {
@@ -114,26 +115,20 @@ struct ActiveProbe
 
 ActiveProbe probe;
 
-// Panel width of the block Gram-Schmidt: 0 (by batch, default), 4, or 8
-// (tiles of at most 2048 rows); set by starsh_hip_set_option("qr_panel").
-// A 4-column panel keeps two tiles resident per CU (512 on the chip), an
-// 8-column one a single tile, with half the launches and half the re-reads
-// of earlier columns.  Batches of up to PANEL8_TILES tiles are done in at
-// most three rounds of 4-column workgroups and take them (C2, 820 tiles:
-// 10.1 ms against 11.7 ms with 8 columns); larger ones take 8 columns (C3,
-// 2080 tiles: 1.61 s against 1.72 s in the plain form).
+// Panel width inside a block of the Gram-Schmidt: 0 (default: 8 for tiles of
+// at most 2048 rows), 4, or 8 (again up to 2048 rows); set by
+// starsh_hip_set_option("qr_panel").
 int qr_panel_width = 0;
 // The width chosen by the autotuner for the current call (0 = by batch);
 // the option above wins.
 int qr_panel_tuned = 0;
-constexpr int PANEL8_TILES = 1536;
 
 // Projection of the mixed form on int8 digit planes (1, default) or FP64
 // MFMA (0); set by starsh_hip_set_option("proj_int8").
 int proj_int8 = 1;
 
 // Gram-Schmidt panels as one captured hipGraph (option "qr_graph" 1)
-// instead of host launches pruned by the lagged probe: every panel up to
+// instead of host launches pruned by the lagged probe: every block up to
 // the batch's width is in the graph (finished tiles return at once), and
 // the executable graph is kept and replayed while its arguments (the
 // pooled buffers, sizes and thresholds) are unchanged, so a repeated
@@ -144,13 +139,14 @@ struct PanelGraph
 {
     struct Key
     {
-        const void *tiles, *ws, *keep, *active;
+        const void *tiles, *ws, *keep, *active, *norms, *coef;
         int ntiles, which, kmax, width_max, rows_max, pb;
         double tau_first;
         bool operator==(const Key &o) const
         {
             return tiles == o.tiles && ws == o.ws && keep == o.keep &&
-                active == o.active && ntiles == o.ntiles &&
+                active == o.active && norms == o.norms &&
+                coef == o.coef && ntiles == o.ntiles &&
                 which == o.which && kmax == o.kmax &&
                 width_max == o.width_max && rows_max == o.rows_max &&
                 pb == o.pb && tau_first == o.tau_first;
@@ -167,17 +163,17 @@ struct PanelGraph
 PanelGraph panel_graphs[2];      // which = 0, 1
 
 int bcgs2(TileDesc *d_tiles, int ntiles, int which, double *ws, int kmax,
-        int width_max, int rows_max, int *d_keep, double tau_first,
-        int *d_active, hipStream_t s)
+        int width_max, int rows_max, int *d_keep, double *d_norms,
+        double *d_coef, double tau_first, int *d_active, hipStream_t s)
 {
     const int pw = qr_panel_width ? qr_panel_width : qr_panel_tuned;
-    const bool wide = pw == 8 || (pw == 0 && ntiles > PANEL8_TILES);
+    const bool wide = pw != 4;
     const int pb = rows_max <= 2048 && wide ? 8 : 4;
     if(qr_graph)
     {
         PanelGraph &pg = panel_graphs[which ? 1 : 0];
-        const PanelGraph::Key key{d_tiles, ws, d_keep, d_active, ntiles,
-            which, kmax, width_max, rows_max, pb, tau_first};
+        const PanelGraph::Key key{d_tiles, ws, d_keep, d_active, d_norms,
+            d_coef, ntiles, which, kmax, width_max, rows_max, pb, tau_first};
         TRY(pipeline_count_active(d_tiles, ntiles, which, d_active, s));
         // captured and launched on a stream of its own, ordered after and
         // before the library stream's work by events: the copy-back threads
@@ -199,10 +195,10 @@ int bcgs2(TileDesc *d_tiles, int ntiles, int which, double *ws, int kmax,
                         hipStreamCaptureModeThreadLocal));
             int info = STARSH_SUCCESS;
             for(int j0 = 0; info == STARSH_SUCCESS && j0 < width_max;
-                    j0 += pb)
-                info = pipeline_panel(d_tiles, ntiles, which, ws, j0, pb,
-                        kmax, tau_first, TAU_SECOND, d_keep, rows_max,
-                        d_active, cs);
+                    j0 = gs_next(j0))
+                info = pipeline_gs_block(d_tiles, ntiles, which, ws, j0, pb,
+                        kmax, tau_first, TAU_SECOND, d_keep, d_norms,
+                        d_coef, rows_max, d_active, cs);
             hipError_t e = hipStreamEndCapture(cs, &graph);
             if(info != STARSH_SUCCESS || e != hipSuccess)
             {
@@ -228,19 +224,22 @@ int bcgs2(TileDesc *d_tiles, int ntiles, int which, double *ws, int kmax,
     }
     TRY(probe.init());
     TRY(pipeline_count_active(d_tiles, ntiles, which, d_active, s));
-    int panel = 0;
-    for(int j0 = 0; j0 < width_max; j0 += pb, panel++)
+    int block = 0;
+    for(int j0 = 0; j0 < width_max; j0 = gs_next(j0), block++)
     {
-        if(panel >= LAG)
+        if(block > LAG)
         {
-            const int slot = (panel-LAG) % NSLOT;
+            const int slot = (block-LAG-1) % NSLOT;
             HIP_TRY(hipEventSynchronize(probe.ev[slot]));
             if(probe.h[slot] == 0)
                 break;
         }
-        TRY(pipeline_panel(d_tiles, ntiles, which, ws, j0, pb, kmax,
-                    tau_first, TAU_SECOND, d_keep, rows_max, d_active, s));
-        const int slot = panel % NSLOT;
+        TRY(pipeline_gs_block(d_tiles, ntiles, which, ws, j0, pb, kmax,
+                    tau_first, TAU_SECOND, d_keep, d_norms, d_coef, rows_max,
+                    d_active, s));
+        if(gs_next(j0) >= width_max)
+            break;
+        const int slot = block % NSLOT;
         HIP_TRY(hipMemcpyAsync(probe.h+slot, d_active, sizeof(int),
                     hipMemcpyDeviceToHost, s));
         HIP_TRY(hipEventRecord(probe.ev[slot], s));
@@ -480,7 +479,7 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
     // part: split-K partials of R2, kept until the batch has synchronised
     Pool &tiles = tiles_pool, &keep = keep_pool, &norms = norms_pool,
          &om8 = om8_pool, &active = active_pool, &qd = qd_pool,
-         &part = part_pool, &selbuf = sel_pool, &pivbuf = piv_pool;
+         &part = part_pool, &coef = coef_pool, &selbuf = sel_pool, &pivbuf = piv_pool;
     if(nsel > 0)
     {
         TRY(selbuf.reserve(sizeof(int)*(size_t)nsel));
@@ -501,6 +500,7 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
     TRY(tiles.reserve(sizeof(TileDesc)*nt));
     TRY(keep.reserve(sizeof(int)*(size_t)nt*kmax));
     TRY(norms.reserve(sizeof(double)*(size_t)nt*kmax));
+    TRY(coef.reserve(sizeof(double)*(size_t)nt*kmax*GS_BLOCK));
     TRY(uv_pool.reserve(sizeof(double)*(uvoff > 0 ? uvoff : 1)));
     TRY(active.reserve(sizeof(int)));
     TileDesc *d_tiles = (TileDesc *)tiles.p;
@@ -569,6 +569,7 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
     // columns of panels that are never launched count as dropped
     HIP_TRY(hipMemsetAsync(keep.p, 0, sizeof(int)*(size_t)nt*kmax, s));
     TRY(bcgs2(d_tiles, nt, 0, d_ws, kmax, kmax, mmax, (int *)keep.p,
+                (double *)norms.p, (double *)coef.p,
                 in->tau > 0 ? in->tau : TAU_FIRST, (int *)active.p, s));
     dump("Qfull", d_ws+h[0].q_off, (int64_t)h[0].m*h[0].k, s);
     TRY(pipeline_compact(d_tiles, nt, d_ws, (int *)keep.p, kmax, s));
@@ -632,7 +633,8 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
     if(pmax > 0)
     {
         TRY(bcgs2(d_tiles, nt, 1, d_ws, kmax, pmax, nmax, (int *)keep.p,
-                    TAU_FIRST, (int *)active.p, s));
+                    (double *)norms.p, (double *)coef.p, TAU_FIRST,
+                    (int *)active.p, s));
         dump("Q2", d_ws+h[0].q2_off, (int64_t)h[0].n*h[0].p, s);
         const int nz = pipeline_r2_split(nt, pmax, nmax);
         if(nz > 1)
@@ -699,7 +701,7 @@ void rsdd_release_pools(void)
     pack_pool.release();
     stage_pool.release();
     for(Pool *q : {&tiles_pool, &keep_pool, &norms_pool, &om8_pool,
-                &active_pool, &qd_pool, &part_pool, &sel_pool, &piv_pool})
+                &active_pool, &qd_pool, &part_pool, &sel_pool, &piv_pool, &coef_pool})
         q->release();
     for(PanelGraph &pg : panel_graphs)
         pg.reset();
