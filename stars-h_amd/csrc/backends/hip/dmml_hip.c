@@ -21,13 +21,11 @@
 struct starsh_hip_tlr
 {
     STARSH_int nrows, ncols;
-    int ntiles, nchunks;
-    tlr_tile *d_tiles;
-    tlr_chunk *d_chunks;
-    tlr_entry *d_entries;
-    double *d_fac;
+    tlr_plan plan;
     size_t fac_doubles;
-    int64_t tmp_units;       /* sum over far tiles of 2 r, plus n per twin */
+    int64_t tmp_units;       /* sum over far tiles of 2 r */
+    int64_t noalloc_units;   /* the same plus n per twin tile: the size the
+                                allocation-free product is limited by */
     double *d_tmp;
     int tmp_nrhs;            /* right-hand sides d_tmp has room for */
 };
@@ -36,10 +34,10 @@ void starsh_hip_tlr_free(starsh_hip_tlr *T)
 {
     if(T == NULL)
         return;
-    starsh_hip_free(T->d_tiles);
-    starsh_hip_free(T->d_chunks);
-    starsh_hip_free(T->d_entries);
-    starsh_hip_free(T->d_fac);
+    starsh_hip_free(T->plan.d_units);
+    starsh_hip_free(T->plan.d_chunks);
+    starsh_hip_free(T->plan.d_entries);
+    starsh_hip_free(T->plan.d_fac);
     starsh_hip_free(T->d_tmp);
     free(T);
 }
@@ -53,6 +51,49 @@ static int upload(void **d, const void *h, size_t bytes)
     if(info != STARSH_SUCCESS)
         return info;
     return starsh_hip_memcpy_h2d(*d, h, bytes);
+}
+
+/* Offsets of a far-field tile's factors and coefficients. */
+typedef struct
+{
+    int64_t u_off, v_off, tmp_off;
+} tlr_far;
+
+/* Entries a contribution of `cols` columns takes. */
+static int64_t pieces(int64_t cols)
+{
+    return (cols+TLR_ENTRY_COLS-1)/TLR_ENTRY_COLS;
+}
+
+static int64_t add_units(tlr_unit *u, int64_t f_off, int len, int r,
+        int64_t x_off, int64_t out_off)
+{
+    int64_t n = 0;
+    for(int c = 0; c < r; c += 32, n++)
+    {
+        u[n].f_off = f_off+(int64_t)c*len;
+        u[n].x_off = x_off;
+        u[n].out_off = out_off+c;
+        u[n].len = len;
+        u[n].nc = r-c < 32 ? r-c : 32;
+    }
+    return n;
+}
+
+static int64_t add_entries(tlr_entry *e, int kind, int64_t f_off, int ld,
+        int64_t cols, int64_t src_off)
+{
+    int64_t n = 0;
+    for(int64_t c = 0; c < cols; c += TLR_ENTRY_COLS, n++)
+    {
+        memset(e+n, 0, sizeof(*e));
+        e[n].kind = kind;
+        e[n].f_off = f_off+(kind == 2 ? c : c*ld);
+        e[n].src_off = src_off+c;
+        e[n].ld = ld;
+        e[n].cols = (int)(cols-c < TLR_ENTRY_COLS ? cols-c : TLR_ENTRY_COLS);
+    }
+    return n;
 }
 
 int starsh_hip_tlr_new(starsh_hip_tlr **out, STARSH_blrm *M)
@@ -84,32 +125,34 @@ int starsh_hip_tlr_new(starsh_hip_tlr **out, STARSH_blrm *M)
         nfac += (size_t)R->size[i]*C->size[j];
     }
     /* entries per block row: far i == b, far twin j == b, near i == b,
-     * near twin j == b */
+     * near twin j == b, each of at most TLR_ENTRY_COLS columns; units: 32
+     * columns of a factor whose coefficients are needed (V, and U of a
+     * tile with a twin) */
+    int64_t nunits = 0;
+    for(STARSH_int bi = 0; bi < nfar; bi++)
+        nunits += (int64_t)((M->far_rank[bi]+31)/32)*
+            (symm && F->block_far[2*bi] != F->block_far[2*bi+1] ? 2 : 1);
     int64_t *count = calloc(nbr+1, sizeof(int64_t));
     double *hfac = malloc(sizeof(double)*(nfac > 0 ? nfac : 1));
-    tlr_tile *htiles = malloc(sizeof(tlr_tile)*(nfar > 0 ? nfar : 1));
+    tlr_unit *hunits = malloc(sizeof(tlr_unit)*(nunits > 0 ? nunits : 1));
+    tlr_far *hfar = malloc(sizeof(tlr_far)*(nfar > 0 ? nfar : 1));
     int64_t *nearoff = malloc(sizeof(int64_t)*(nnear > 0 ? nnear : 1));
     starsh_hip_tlr *T = calloc(1, sizeof(*T));
     tlr_entry *hent = NULL;
     tlr_chunk *hch = NULL;
     int info = STARSH_MALLOC_ERROR;
-    if(!count || !hfac || !htiles || !nearoff || !T)
+    if(!count || !hfac || !hunits || !hfar || !nearoff || !T)
         goto fail;
     T->nrows = P->shape[0];
     T->ncols = P->shape[P->ndim-1];
     size_t off = 0;
-    int64_t tmp = 0;
+    int64_t tmp = 0, twins = 0, nu = 0;
     for(STARSH_int bi = 0; bi < nfar; bi++)
     {
         STARSH_int i = F->block_far[2*bi], j = F->block_far[2*bi+1];
         int m = (int)R->size[i], n = (int)C->size[j], r = M->far_rank[bi];
-        tlr_tile *t = &htiles[bi];
-        t->m = m;
-        t->n = n;
-        t->rank = r;
-        t->r0 = R->start[i];
-        t->c0 = C->start[j];
-        t->twin = symm && i != j;
+        const int twin = symm && i != j;
+        tlr_far *t = &hfar[bi];
         t->u_off = (int64_t)off;
         if(r > 0)
             memcpy(hfac+off, M->far_U[bi]->data, sizeof(double)*m*r);
@@ -120,15 +163,15 @@ int starsh_hip_tlr_new(starsh_hip_tlr **out, STARSH_blrm *M)
         off += (size_t)n*r;
         t->tmp_off = tmp;
         tmp += 2*(int64_t)r;
-        t->p_off = tmp;
-        if(t->twin && r > 0)
-            tmp += n;
-        if(r > 0)
-        {
-            count[i]++;
-            if(t->twin)
-                count[j]++;
-        }
+        if(twin && r > 0)
+            twins += n;
+        nu += add_units(hunits+nu, t->v_off, n, r, C->start[j], t->tmp_off);
+        if(twin)
+            nu += add_units(hunits+nu, t->u_off, m, r, R->start[i],
+                    t->tmp_off+r);
+        count[i] += pieces(r);
+        if(twin)
+            count[j] += pieces(r);
     }
     for(STARSH_int bi = 0; bi < nnear; bi++)
     {
@@ -141,9 +184,9 @@ int starsh_hip_tlr_new(starsh_hip_tlr **out, STARSH_blrm *M)
             P->kernel(m, n, R->pivot+R->start[i], C->pivot+C->start[j],
                     R->data, C->data, hfac+off, m);
         off += (size_t)m*n;
-        count[i]++;
+        count[i] += pieces(n);
         if(symm && i != j)
-            count[j]++;
+            count[j] += pieces(m);
     }
     /* CSR of entries by block row */
     int64_t nent = 0;
@@ -164,84 +207,67 @@ int starsh_hip_tlr_new(starsh_hip_tlr **out, STARSH_blrm *M)
     memcpy(fill, count, sizeof(int64_t)*nbr);
     for(STARSH_int bi = 0; bi < nfar; bi++)
     {
-        const tlr_tile *t = &htiles[bi];
-        if(t->rank <= 0)
-            continue;
+        const tlr_far *t = &hfar[bi];
         STARSH_int i = F->block_far[2*bi], j = F->block_far[2*bi+1];
-        tlr_entry *e = &hent[fill[i]++];
-        memset(e, 0, sizeof(*e));
-        e->kind = 0;
-        e->f_off = t->u_off;
-        e->ld = t->m;
-        e->cols = t->rank;
-        e->src_off = t->tmp_off;
-        if(t->twin)
-        {
-            /* V (U^T X_i), formed by the coefficient pass */
-            e = &hent[fill[j]++];
-            memset(e, 0, sizeof(*e));
-            e->kind = 3;
-            e->ld = t->n;
-            e->src_off = t->p_off;
-        }
+        int m = (int)R->size[i], n = (int)C->size[j], r = M->far_rank[bi];
+        fill[i] += add_entries(hent+fill[i], 0, t->u_off, m, r, t->tmp_off);
+        if(symm && i != j)
+            fill[j] += add_entries(hent+fill[j], 0, t->v_off, n, r,
+                    t->tmp_off+r);
     }
     for(STARSH_int bi = 0; bi < nnear; bi++)
     {
         STARSH_int i = F->block_near[2*bi], j = F->block_near[2*bi+1];
         int m = (int)R->size[i], n = (int)C->size[j];
-        tlr_entry *e = &hent[fill[i]++];
-        memset(e, 0, sizeof(*e));
-        e->kind = 1;
-        e->f_off = nearoff[bi];
-        e->ld = m;
-        e->cols = n;
-        e->src_off = C->start[j];
+        fill[i] += add_entries(hent+fill[i], 1, nearoff[bi], m, n,
+                C->start[j]);
         if(symm && i != j)
-        {
-            e = &hent[fill[j]++];
-            memset(e, 0, sizeof(*e));
-            e->kind = 2;
-            e->f_off = nearoff[bi];
-            e->ld = m;
-            e->cols = m;
-            e->src_off = R->start[i];
-        }
+            fill[j] += add_entries(hent+fill[j], 2, nearoff[bi], m, m,
+                    R->start[i]);
     }
     free(fill);
-    /* chunks of 64 rows of every block row */
+    /* strips of every block row: 64 rows, fewer where that would leave the
+     * chip without two workgroups per CU */
+    int strip = 64;
+    while(strip > 16 && T->nrows/strip < 512)
+        strip /= 2;
     int64_t nch = 0;
     for(STARSH_int b = 0; b < nbr; b++)
-        nch += (R->size[b]+63)/64;
+        nch += (R->size[b]+strip-1)/strip;
     hch = malloc(sizeof(tlr_chunk)*(nch > 0 ? nch : 1));
     if(!hch)
         goto fail;
     nch = 0;
     for(STARSH_int b = 0; b < nbr; b++)
-        for(STARSH_int r0 = 0; r0 < R->size[b]; r0 += 64)
+        for(STARSH_int r0 = 0; r0 < R->size[b]; r0 += strip)
         {
             tlr_chunk *c = &hch[nch++];
             c->row0 = R->start[b]+r0;
             c->rofs = (int)r0;
-            c->nrows = (int)(R->size[b]-r0 < 64 ? R->size[b]-r0 : 64);
+            c->nrows = (int)(R->size[b]-r0 < strip ? R->size[b]-r0 : strip);
             c->first = (int)count[b];
             c->last = (int)count[b+1];
         }
-    T->ntiles = (int)nfar;
-    T->nchunks = (int)nch;
+    T->plan.nunits = (int)nu;
+    T->plan.nchunks = (int)nch;
+    T->plan.strip = strip;
     T->fac_doubles = off;
     T->tmp_units = tmp;
-    info = upload((void **)&T->d_fac, hfac, sizeof(double)*off);
+    T->noalloc_units = tmp+twins;
+    info = upload((void **)&T->plan.d_fac, hfac, sizeof(double)*off);
     if(info == STARSH_SUCCESS)
-        info = upload((void **)&T->d_tiles, htiles, sizeof(tlr_tile)*nfar);
+        info = upload((void **)&T->plan.d_units, hunits, sizeof(tlr_unit)*nu);
     if(info == STARSH_SUCCESS)
-        info = upload((void **)&T->d_entries, hent, sizeof(tlr_entry)*nent);
+        info = upload((void **)&T->plan.d_entries, hent,
+                sizeof(tlr_entry)*nent);
     if(info == STARSH_SUCCESS)
-        info = upload((void **)&T->d_chunks, hch, sizeof(tlr_chunk)*nch);
+        info = upload((void **)&T->plan.d_chunks, hch, sizeof(tlr_chunk)*nch);
     if(info != STARSH_SUCCESS)
         goto fail;
     free(count);
     free(hfac);
-    free(htiles);
+    free(hunits);
+    free(hfar);
     free(nearoff);
     free(hent);
     free(hch);
@@ -250,7 +276,8 @@ int starsh_hip_tlr_new(starsh_hip_tlr **out, STARSH_blrm *M)
 fail:
     free(count);
     free(hfac);
-    free(htiles);
+    free(hunits);
+    free(hfar);
     free(nearoff);
     free(hent);
     free(hch);
@@ -284,9 +311,8 @@ int starsh_hip_tlr_dmml(starsh_hip_tlr *T, int nrhs, double alpha,
     int info = tmp_reserve(T, nrhs);
     if(info != STARSH_SUCCESS)
         return info;
-    return starsh_hip_tlr_apply(T->d_tiles, T->ntiles, T->d_chunks,
-            T->nchunks, T->d_entries, T->d_fac, T->d_tmp, nrhs, alpha, d_A,
-            lda, beta, d_B, ldb);
+    return starsh_hip_tlr_apply(&T->plan, T->d_tmp, nrhs, alpha, d_A, lda,
+            beta, d_B, ldb);
 }
 
 int starsh_hip_current_device(void);
@@ -299,7 +325,7 @@ int starsh_hip_tlr_dmml_noalloc(starsh_hip_tlr *T, int nrhs, double alpha,
         return STARSH_WRONG_PARAMETER;
     if(nrhs == 0)
         return STARSH_SUCCESS;
-    const int64_t need = (T->tmp_units > 0 ? T->tmp_units : 1)*
+    const int64_t need = (T->noalloc_units > 0 ? T->noalloc_units : 1)*
         (int64_t)nrhs;
     if(need > TLR_SCRATCH_DOUBLES)
     {
@@ -318,9 +344,8 @@ int starsh_hip_tlr_dmml_noalloc(starsh_hip_tlr *T, int nrhs, double alpha,
         STARSH_ERROR("the product scratch is not set up on this device");
         return STARSH_UNKNOWN_ERROR;
     }
-    return starsh_hip_tlr_apply(T->d_tiles, T->ntiles, T->d_chunks,
-            T->nchunks, T->d_entries, T->d_fac, ptr, nrhs, alpha, d_A, lda,
-            beta, d_B, ldb);
+    return starsh_hip_tlr_apply(&T->plan, ptr, nrhs, alpha, d_A, lda, beta,
+            d_B, ldb);
 }
 
 int starsh_hip_tlr_bench(starsh_hip_tlr *T, int nrhs, int reps,
@@ -345,8 +370,7 @@ int starsh_hip_tlr_bench(starsh_hip_tlr *T, int nrhs, int reps,
         info = starsh_hip_memcpy_h2d(dx, hx, sizeof(double)*nx);
     }
     if(info == STARSH_SUCCESS)
-        info = starsh_hip_tlr_time(T->d_tiles, T->ntiles, T->d_chunks,
-                T->nchunks, T->d_entries, T->d_fac, T->d_tmp, nrhs, dx,
+        info = starsh_hip_tlr_time(&T->plan, T->d_tmp, nrhs, dx,
                 (int)T->ncols, dy, (int)T->nrows, reps, seconds);
     /* algorithmic bytes: every factor and near tile read once, X read,
      * Y written */
@@ -403,12 +427,6 @@ int starsh_blrm__dmml_hip(STARSH_blrm *matrix, int nrhs, double alpha,
     return info;
 }
 
-/* Reads a device scalar (the copy waits for the library stream). */
-static int fetch(const double *d, double *h)
-{
-    return starsh_hip_memcpy_d2h(h, d, sizeof(double));
-}
-
 int starsh_itersolvers__dcg_hip(STARSH_blrm *matrix, int nrhs, double *B,
         int ldb, double *X, int ldx, double tol, double *work)
 {
@@ -427,20 +445,20 @@ int starsh_itersolvers__dcg_hip(STARSH_blrm *matrix, int nrhs, double *B,
     }
     const size_t nn = (size_t)n*nrhs;
     double *dB = NULL, *dX = NULL, *dR = NULL, *dP = NULL, *dQ = NULL;
-    double *dpart = NULL, *dscal = NULL;
-    double *rscheck = malloc(sizeof(double)*3*nrhs);
-    double *rsold = rscheck ? rscheck+nrhs : NULL;
-    double *rsnew = rscheck ? rscheck+2*nrhs : NULL;
+    double *dpart = NULL;
+    tlr_cg_state *dst = NULL, *hst = malloc(sizeof(tlr_cg_state)*nrhs);
     int result = -1;
-    if(rscheck == NULL)
+    if(hst == NULL)
         info = STARSH_MALLOC_ERROR;
     double **bufs[] = {&dB, &dX, &dR, &dP, &dQ};
     for(int b = 0; b < 5 && info == STARSH_SUCCESS; b++)
         info = starsh_hip_malloc((void **)bufs[b], sizeof(double)*nn);
     if(info == STARSH_SUCCESS)
-        info = starsh_hip_malloc((void **)&dpart, sizeof(double)*256);
+        info = starsh_hip_malloc((void **)&dpart, sizeof(double)*
+                TLR_CG_PART(nrhs));
     if(info == STARSH_SUCCESS)
-        info = starsh_hip_malloc((void **)&dscal, sizeof(double));
+        info = starsh_hip_malloc((void **)&dst, sizeof(tlr_cg_state)*
+                TLR_CG_STATES(nrhs));
     for(int q = 0; q < nrhs && info == STARSH_SUCCESS; q++)
     {
         info = starsh_hip_memcpy_h2d(dB+(size_t)q*n, B+(size_t)q*ldb,
@@ -456,58 +474,34 @@ int starsh_itersolvers__dcg_hip(STARSH_blrm *matrix, int nrhs, double *B,
         info = starsh_hip_vaxpy((int64_t)nn, 1.0, dB, dR);
     if(info == STARSH_SUCCESS)
         info = starsh_hip_vcopy((int64_t)nn, dR, dP);
-    for(int q = 0; q < nrhs && info == STARSH_SUCCESS; q++)
-    {
-        double rr = 0.0;
-        info = starsh_hip_vdot(n, dR+(size_t)q*n, dR+(size_t)q*n, dpart,
-                dscal);
-        if(info == STARSH_SUCCESS)
-            info = fetch(dscal, &rr);
-        rsold[q] = sqrt(rr);
-        rscheck[q] = rsold[q]*tol;
-        rsnew[q] = rscheck[q];
-        rsold[q] *= rsold[q];
-    }
-    int finished = 0;
+    if(info == STARSH_SUCCESS)
+        info = starsh_hip_cg_start(n, nrhs, tol, dR, dpart, dst);
+    /* The iterations are queued without waiting: a column that has met its
+     * stopping rule is left alone by the kernels, and the states are read
+     * back after 4, 8 and then every 16 iterations (two dot products read
+     * back per iteration took as long as its kernels). */
+    int look = 4, batch = 4;
     for(int it = 0; it < n && info == STARSH_SUCCESS; it++)
     {
         info = starsh_hip_tlr_dmml(T, nrhs, 1.0, dP, n, 0.0, dQ, n);
-        for(int q = 0; q < nrhs && info == STARSH_SUCCESS; q++)
+        if(info == STARSH_SUCCESS)
+            info = starsh_hip_cg_iteration(n, nrhs, it, dP, dQ, dX, dR,
+                    dpart, dst);
+        if(info != STARSH_SUCCESS || (it+1 < look && it+1 < n))
+            continue;
+        batch = batch < 16 ? 2*batch : 16;
+        look += batch;
+        info = starsh_hip_memcpy_d2h(hst, dst+(size_t)((it+1) & 1)*nrhs,
+                sizeof(tlr_cg_state)*nrhs);
+        int last = -1, finished = 0;
+        for(int q = 0; info == STARSH_SUCCESS && q < nrhs; q++)
         {
-            if(rscheck[q] < 0)
-                continue;
-            double *p = dP+(size_t)q*n, *np = dQ+(size_t)q*n;
-            double *r = dR+(size_t)q*n, *x = dX+(size_t)q*n;
-            double pq = 0.0, rr = 0.0;
-            info = starsh_hip_vdot(n, p, np, dpart, dscal);
-            if(info == STARSH_SUCCESS)
-                info = fetch(dscal, &pq);
-            if(info != STARSH_SUCCESS)
-                break;
-            const double a = rsold[q]/pq;
-            info = starsh_hip_vaxpy(n, a, p, x);
-            if(info == STARSH_SUCCESS)
-                info = starsh_hip_vaxpy(n, -a, np, r);
-            if(info == STARSH_SUCCESS)
-                info = starsh_hip_vdot(n, r, r, dpart, dscal);
-            if(info == STARSH_SUCCESS)
-                info = fetch(dscal, &rr);
-            if(info != STARSH_SUCCESS)
-                break;
-            rsnew[q] = sqrt(rr);
-            if(rsnew[q] < rscheck[q])
-            {
-                finished++;
-                rscheck[q] = -1.0;
-                continue;
-            }
-            rsnew[q] *= rsnew[q];
-            info = starsh_hip_vxpby(n, r, rsnew[q]/rsold[q], p);
-            rsold[q] = rsnew[q];
+            finished += hst[q].done >= 0;
+            last = hst[q].done > last ? hst[q].done : last;
         }
         if(info == STARSH_SUCCESS && finished == nrhs)
         {
-            result = it;
+            result = last;
             break;
         }
     }
@@ -517,8 +511,8 @@ int starsh_itersolvers__dcg_hip(STARSH_blrm *matrix, int nrhs, double *B,
     for(int b = 0; b < 5; b++)
         starsh_hip_free(*bufs[b]);
     starsh_hip_free(dpart);
-    starsh_hip_free(dscal);
-    free(rscheck);
+    starsh_hip_free(dst);
+    free(hst);
     starsh_hip_tlr_free(T);
     if(info != STARSH_SUCCESS)
         return -1;

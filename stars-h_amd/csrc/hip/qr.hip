@@ -44,75 +44,6 @@ __global__ __launch_bounds__(256) void colnorm_kernel(const TileDesc *tiles,
     }
 }
 
-// Sum over the 64 lanes of a wave of each of V values (V a power of two,
-// at most 64) by recursive halving: at every level O (32, 16, ..., 1) a
-// lane keeps half of its values, the upper half if lane & O, and adds its
-// partner's copy of them (partners as in lane_partner / swap_sum), so
-// V-1+log2(64/V) exchanges reduce all V.  On return the lane holds the
-// total of value index halving_index<V>(lane).  The steps are unrolled by
-// template recursion.
-template <int H, int O>
-struct Halve
-{
-    template <int V>
-    static __device__ inline void run(double (&v)[V], int lane)
-    {
-        if constexpr(O >= 16)
-        {
-            // the swap hands the lower (even-row) lane's v[i] and the
-            // upper lane's v[i+H] to the partner that keeps them
-#pragma unroll
-            for(int i = 0; i < H; i++)
-                v[i] = swap_sum<O>(v[i], v[i+H]);
-        }
-        else
-        {
-            const bool up = (lane & O) != 0;
-#pragma unroll
-            for(int i = 0; i < H; i++)
-            {
-                const double send = up ? v[i] : v[i+H];
-                const double keep = up ? v[i+H] : v[i];
-                v[i] = keep+lane_partner<O>(send);
-            }
-        }
-        Halve<H/2, O/2>::run(v, lane);
-    }
-};
-
-template <int O>
-struct Halve<0, O>
-{
-    template <int V>
-    static __device__ inline void run(double (&v)[V], int lane)
-    {
-        (void)lane;
-        if constexpr(O >= 1)
-        {
-            v[0] = pair_sum<O>(v[0]);
-            Halve<0, O/2>::run(v, lane);
-        }
-    }
-};
-
-template <int V>
-__device__ inline double halving_sum(double (&v)[V], int lane)
-{
-    Halve<V/2, 32>::run(v, lane);
-    return v[0];
-}
-
-template <int V>
-__device__ inline int halving_index(int lane)
-{
-    int idx = 0;
-#pragma unroll
-    for(int st = 0; (V >> (st+1)) >= 1; st++)
-        if(lane & (32 >> st))
-            idx += V >> (st+1);
-    return idx;
-}
-
 // ---- Block Gram-Schmidt applied twice (BCGS2)
 //
 // The columns of Q (which = 0: m rows, width k) or Q2 (which = 1: n rows,

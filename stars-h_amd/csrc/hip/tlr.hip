@@ -6,289 +6,352 @@
 // tiles add D X_j (and D^T X_i).
 //
 // Two launches, both deterministic (no atomics):
-//  1. tlr_coef_kernel, one workgroup per far-field tile: the r x nrhs
-//     coefficients T = V^T X_j; for a tile with a twin (symmetric format,
-//     i != j) it first forms T' = U^T X_i (one read of U), then takes T and
-//     the twin's whole contribution P = V T' (n x nrhs) from one read of V;
-//  2. tlr_rows_kernel: per chunk of 64 rows of one block row, the sum of all
-//     contributions to those rows (U T, P, D X_j, D^T X_i) in a fixed
-//     order: lane = row, wave w takes entries w, w+4, ... of the block row,
-//     and the four partial sums are added in LDS in wave order.
-// A twin tile's U is read twice (for T' and for U T) and its V once, 1.5
-// reads per factor instead of 2 for coefficient and row passes that each
-// read both factors: a factor of a 1600-row tile does not stay on a CU
-// between two uses.
+//  1. one workgroup per 32 columns of a factor: the coefficients T = V^T X_j
+//     and, for a tile with a twin (symmetric format, i != j), T' = U^T X_i;
+//  2. one workgroup per strip of 64, 32 or 16 rows of one block row: the sum
+//     of all contributions to those rows (U T, V T', D X_j, D^T X_i) in a
+//     fixed order: wave w takes entries w, w+4, ... (wide ones come in
+//     pieces) and the four partial sums are added in LDS in wave order.
+// With one right-hand side a lane multiplies its own values; with more, up
+// to 16 at a time go through FP64 MFMA (the columns past nrhs are zeros).
+//
+// What bounds it: HBM; every factor is read twice, every dense tile once.
+// Measured on MI355X, before and after (one workgroup per tile forming U^T X
+// and then V (U^T X) row by row, and strips of 64 rows, dense tiles one
+// column at a time, right-hand sides in groups of four that each re-read
+// everything):
+//   N=2500, tile 250, 1 rhs (launch-bound)                  27.7 -> 10.7 us
+//   N=64000, tile 1600, ranks 8-31, 1 rhs, 358 MB, read
+//     twice at 5.3 TB/s                                      144 -> 138 us
+//   N=30000, tile 1700, nonsymmetric, ranks to 90, 12 dense
+//     tiles, 10 rhs, 812 MB                                 4470 -> 260 us
+//   CG iteration, N=10000, tile 1000, 10 dense tiles         610 -> 72 us
+// Reading U once for U^T X and keeping V (U^T X) (1.5 reads instead of 2)
+// needs a workgroup per tile: 96 + 40 us for the second line against 64 + 70.
 #include <stdio.h>
 #include "hip_common.h"
 #include "tlr.h"
 
+typedef double double4_t __attribute__((ext_vector_type(4)));
+
 namespace {
 
-constexpr int RHS_GROUP = 4;
-constexpr int COL_BLOCK = 16;
+constexpr int RHS = 16;         // right-hand sides per group
 
-// One pass over a factor F (len x r, ld len) for right-hand sides q0 ..
-// q0+nq-1 (nq <= NQ, NQ = 1 or RHS_GROUP): column sums
-// S[c][q] = sum_l F[l][c] X[l][q] into S + c + q r, and with Tp (r x nrhs,
-// ld r) also the rows P[l][q] = sum_c F[l][c] Tp[c][q] into P + l + q len.
-// Columns go in blocks of 16 (8) with 64-row chunks of the factor striped over
-// the four waves (lane = row); a block's column sums are reduced over the
-// lanes by shuffles and over the waves in LDS in wave order, and each row
-// of P is owned by one lane, which adds the blocks in column order.
-template <int NQ>
-__device__ __forceinline__ void factor_pass(const double *F, int len, int r,
-        const double *X, int ldx, int q0, int nq, double *S, const double *Tp,
-        double *P, double (*red)[COL_BLOCK][RHS_GROUP], double *tp)
+// Sums of one 16 x 16 fragment over its k: four MFMA steps' worth of a lane's
+// values f (row lane%16 of op(F)) times b.  With one right-hand side a lane
+// adds up its own products (v[0]; summed over the four lane groups at the
+// end), with more the MFMA does (row lane/16 + 4 v, column lane%16).
+template <bool ONE>
+struct Acc
 {
-    // columns per block: 16, or 8 with four right-hand sides (registers)
-    constexpr int CB = NQ == 1 ? COL_BLOCK : COL_BLOCK/2;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for(int cb = 0; cb < r; cb += CB)
+    double4_t v = {0.0, 0.0, 0.0, 0.0};
+    __device__ inline void add(double f, double b)
     {
-        const int nc = r-cb < CB ? r-cb : CB;
-        if(Tp && threadIdx.x < COL_BLOCK*RHS_GROUP)
-        {
-            const int u = threadIdx.x % COL_BLOCK, q = threadIdx.x/COL_BLOCK;
-            tp[threadIdx.x] = u < nc && q < nq ?
-                Tp[cb+u+(int64_t)(q0+q)*r] : 0.0;
-        }
-        __syncthreads();
-        double s[CB][NQ] = {};
-        // one chunk at a time (two in flight measured no faster)
-#pragma unroll 1
-        for(int l = wave*64+lane; l-lane < len; l += 256)
-        {
-            const bool ok = l < len;
-            // loads of the columns that exist only (unconditional loads
-            // from clamped addresses measured 35% slower on 1600-row tiles
-            // of rank 7-31: the extra loads cost more than the branches)
-            double x[NQ], v[CB];
-#pragma unroll
-            for(int q = 0; q < NQ; q++)
-                x[q] = ok && q < nq ? X[l+(int64_t)(q0+q)*ldx] : 0.0;
-#pragma unroll
-            for(int u = 0; u < CB; u++)
-                v[u] = ok && u < nc ? F[(int64_t)(cb+u)*len+l] : 0.0;
-#pragma unroll
-            for(int u = 0; u < CB; u++)
-#pragma unroll
-                for(int q = 0; q < NQ; q++)
-                    s[u][q] = fma(v[u], x[q], s[u][q]);
-            if(Tp && ok)
-#pragma unroll
-                for(int q = 0; q < NQ; q++)
-                    if(q < nq)
-                    {
-                        double p = 0.0;
-#pragma unroll
-                        for(int u = 0; u < CB; u++)
-                            p = fma(v[u], tp[u+q*COL_BLOCK], p);
-                        double *pp = P+l+(int64_t)q*len;
-                        *pp = cb == 0 ? p : *pp+p;
-                    }
-        }
-#pragma unroll
-        for(int u = 0; u < CB; u++)
-#pragma unroll
-            for(int q = 0; q < NQ; q++)
-                if(u < nc && q < nq)
-                {
-                    double t = s[u][q];
-#pragma unroll
-                    for(int o = 32; o > 0; o >>= 1)
-                        t += __shfl_xor(t, o, 64);
-                    s[u][q] = t;
-                }
-        if(lane == 0)
-#pragma unroll
-            for(int u = 0; u < CB; u++)
-#pragma unroll
-                for(int q = 0; q < NQ; q++)
-                    red[wave][u][q] = s[u][q];
-        __syncthreads();
-        if(threadIdx.x < COL_BLOCK*RHS_GROUP)
-        {
-            const int u = threadIdx.x % COL_BLOCK, q = threadIdx.x/COL_BLOCK;
-            if(u < nc && q < nq)
-                S[cb+u+(int64_t)(q0+q)*r] = ((red[0][u][q]+red[1][u][q])+
-                        red[2][u][q])+red[3][u][q];
-        }
-        __syncthreads();
+        if constexpr(ONE)
+            v[0] = fma(f, b, v[0]);
+        else
+            v = __builtin_amdgcn_mfma_f64_16x16x4f64(f, b, v, 0, 0, 0);
     }
+    __device__ inline void close()
+    {
+        if constexpr(ONE)
+        {
+            v[0] += __shfl_xor(v[0], 16, 64);
+            v[0] += __shfl_xor(v[0], 32, 64);
+        }
+    }
+    // values per lane and the row of value q
+    static constexpr int N = ONE ? 1 : 4;
+    static __device__ inline int row(int q, int lane)
+    {
+        return ONE ? lane & 15 : (lane >> 4)+4*q;
+    }
+};
+
+// S = F^T x for 32 columns of a factor F (len rows), one right-hand side: a
+// lane takes a row of a 64-row chunk (512 contiguous bytes of a column per
+// load), the chunks are striped over the four waves, and a wave's sums over
+// its lanes come from one recursive halving of all its columns.  (The MFMA
+// operand layout below, 32 bytes of 16 columns per row group, read the short
+// factors of a 64000-row operator, 16 columns of 1600 rows, at 2.7 TB/s.)
+__global__ __launch_bounds__(256) void tlr_coef1_kernel(const tlr_unit *units,
+        const double *fac, const double *x, double *tmp)
+{
+    constexpr int C = 32;
+    __shared__ double part[4][C];
+    const tlr_unit u = units[blockIdx.x];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const double *F = fac+u.f_off, *X = x+u.x_off;
+    double s[C];
+#pragma unroll
+    for(int c = 0; c < C; c++)
+        s[c] = 0.0;
+#pragma unroll 1
+    for(int l = wave*64+lane; l-lane < u.len; l += 256)
+    {
+        const bool in = l < u.len;
+        const double xl = in ? X[l] : 0.0;
+#pragma unroll
+        for(int h = 0; h < C; h += 16)
+            if(u.nc > h)        // uniform, as is every test of nc
+            {
+                double f[16];
+#pragma unroll
+                for(int c = 0; c < 16; c++)
+                    f[c] = in && h+c < u.nc ? F[(int64_t)(h+c)*u.len+l] : 0.0;
+#pragma unroll
+                for(int c = 0; c < 16; c++)
+                    s[h+c] = fma(f[c], xl, s[h+c]);
+            }
+    }
+    if(u.nc > 16)
+    {
+        const double t = halving_sum<32>(s, lane);
+        if((lane & 1) == 0)
+            part[wave][halving_index<32>(lane)] = t;
+    }
+    else
+    {
+        double s16[16];
+#pragma unroll
+        for(int c = 0; c < 16; c++)
+            s16[c] = s[c];
+        const double t = halving_sum<16>(s16, lane);
+        if((lane & 3) == 0)
+            part[wave][halving_index<16>(lane)] = t;
+    }
+    __syncthreads();
+    const int c = threadIdx.x;
+    if(c < u.nc)
+        tmp[u.out_off+c] = ((part[0][c]+part[1][c])+part[2][c])+part[3][c];
 }
 
-// one right-hand side: at most 128 VGPRs, four workgroups per CU, so that
-// the 820 tiles of a 40 x 40 symmetric format run in one round
-template <int NQ>
-__global__ __launch_bounds__(256, NQ == 1 ? 4 : 1) void tlr_coef_kernel(
-        const tlr_tile *tiles, const double *fac, const double *x, int ldx,
-        int nrhs, double *tmp)
+// The same for up to 16 right-hand sides on MFMA: rows split over the four
+// waves in groups of 64, a lane taking rows 4 (lane/16) .. +3 of each block
+// of 16 (any order of the rows gives the same sum), so that it loads 32
+// contiguous bytes of a column.
+__global__ __launch_bounds__(256) void tlr_coef_kernel(const tlr_unit *units,
+        const double *fac, const double *x, int ldx, int nrhs, double *tmp)
 {
-    __shared__ double red[4][COL_BLOCK][RHS_GROUP];
-    __shared__ double tp[COL_BLOCK*RHS_GROUP];
-    const tlr_tile t = tiles[blockIdx.x];
-    if(t.rank <= 0)
-        return;
-    double *T = tmp+t.tmp_off*nrhs;            // V^T X_j, r x nrhs
-    double *Tt = tmp+(t.tmp_off+t.rank)*nrhs;  // U^T X_i
-    double *P = tmp+t.p_off*nrhs;              // V T', n x nrhs
-    for(int q0 = 0; q0 < nrhs; q0 += NQ)
+    __shared__ double part[3][2][256];
+    const tlr_unit u = units[blockIdx.x];
+    const int q0 = blockIdx.y*RHS, nq = min(nrhs-q0, RHS);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lc = lane & 15, lr = lane >> 4;
+    const double *F[2];
+    bool ok[2];
+#pragma unroll
+    for(int a = 0; a < 2; a++)
     {
-        const int nq = nrhs-q0 < NQ ? nrhs-q0 : NQ;
-        if(t.twin)
+        ok[a] = a*16+lc < u.nc;
+        F[a] = fac+u.f_off+(int64_t)(ok[a] ? a*16+lc : 0)*u.len;
+    }
+    const bool okq = lc < nq;
+    const double *X = x+u.x_off+(int64_t)(okq ? q0+lc : q0)*ldx;
+    Acc<false> acc[2];
+    const int nrb = (u.len+15)/16;
+    const bool two = u.nc > 16;     // uniform
+    for(int g0 = wave*4; g0 < nrb; g0 += 16)
+    {
+        double f[4][2][4], b[4][4];
+        if((g0+4)*16 <= u.len)
         {
-            factor_pass<NQ>(fac+t.u_off, t.m, t.rank, x+t.r0, ldx, q0, nq,
-                    Tt, nullptr, nullptr, red, tp);
-            // Tt, written by other threads of this workgroup, is visible
-            // after the barrier that ended the pass
-            factor_pass<NQ>(fac+t.v_off, t.n, t.rank, x+t.c0, ldx, q0, nq,
-                    T, Tt, P+(int64_t)q0*t.n, red, tp);
+            // uniform: a whole group
+#pragma unroll
+            for(int h = 0; h < 4; h++)
+            {
+                const int r = (g0+h)*16+4*lr;
+#pragma unroll
+                for(int v = 0; v < 4; v++)
+                {
+                    f[h][0][v] = ok[0] ? F[0][r+v] : 0.0;
+                    b[h][v] = okq ? X[r+v] : 0.0;
+                }
+                if(two)
+#pragma unroll
+                    for(int v = 0; v < 4; v++)
+                        f[h][1][v] = ok[1] ? F[1][r+v] : 0.0;
+            }
         }
         else
-            factor_pass<NQ>(fac+t.v_off, t.n, t.rank, x+t.c0, ldx, q0, nq,
-                    T, nullptr, nullptr, red, tp);
+#pragma unroll
+            for(int h = 0; h < 4; h++)
+#pragma unroll
+                for(int v = 0; v < 4; v++)
+                {
+                    const int r = (g0+h)*16+4*lr+v;
+                    const bool in = r < u.len;
+                    f[h][0][v] = in && ok[0] ? F[0][r] : 0.0;
+                    f[h][1][v] = in && ok[1] ? F[1][r] : 0.0;
+                    b[h][v] = in && okq ? X[r] : 0.0;
+                }
+#pragma unroll
+        for(int h = 0; h < 4; h++)
+#pragma unroll
+            for(int v = 0; v < 4; v++)
+            {
+                acc[0].add(f[h][0][v], b[h][v]);
+                if(two)
+                    acc[1].add(f[h][1][v], b[h][v]);
+            }
     }
+    if(wave > 0)
+#pragma unroll
+        for(int a = 0; a < 2; a++)
+#pragma unroll
+            for(int q = 0; q < 4; q++)
+                part[wave-1][a][q*64+lane] = acc[a].v[q];
+    __syncthreads();
+    if(wave == 0 && okq)
+#pragma unroll
+        for(int a = 0; a < 2; a++)
+#pragma unroll
+            for(int q = 0; q < 4; q++)
+            {
+                const int c = a*16+Acc<false>::row(q, lane);
+                if(c < u.nc)
+                    tmp[(u.out_off+c)*nrhs+q0+lc] =
+                        ((acc[a].v[q]+part[0][a][q*64+lane])+
+                         part[1][a][q*64+lane])+part[2][a][q*64+lane];
+            }
 }
 
-template <int NQ>
+// Rows of a strip of 16 RF rows of one block row.
+template <int RF, bool ONE>
 __global__ __launch_bounds__(256) void tlr_rows_kernel(const tlr_chunk *chunks,
         const tlr_entry *entries, const double *fac, const double *tmp,
         const double *x, int ldx, int nrhs, double alpha, double beta,
         double *y, int ldy)
 {
-    __shared__ double part[4][RHS_GROUP][64];
+    __shared__ double part[3][RF][Acc<ONE>::N*64];
     const tlr_chunk ch = chunks[blockIdx.x];
-    // the wave index as a wave-uniform value: entries and coefficients
-    // are then read through the scalar unit
+    const int q0 = blockIdx.y*RHS, nq = min(nrhs-q0, RHS);
     const int lane = threadIdx.x & 63;
+    // the wave index as a wave-uniform value: entries are then read through
+    // the scalar unit
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const bool row_ok = lane < ch.nrows;
-    for(int q0 = 0; q0 < nrhs; q0 += NQ)
+    const int lc = lane & 15, lr = lane >> 4;
+    const bool okq = ONE || lc < nq;
+    const int qx = ONE ? q0 : okq ? q0+lc : q0;
+    // rows past the strip repeat its last one (their sums are not stored)
+    int row[RF];
+#pragma unroll
+    for(int a = 0; a < RF; a++)
+        row[a] = ch.rofs+min(a*16+lc, ch.nrows-1);
+    Acc<ONE> acc[RF];
+    for(int e = ch.first+wave; e < ch.last; e += 4)
     {
-        const int nq = nrhs-q0 < NQ ? nrhs-q0 : NQ;
-        double acc[NQ] = {};
-        for(int e = ch.first+wave; e < ch.last; e += 4)
+        const tlr_entry en = entries[e];
+        // element (row, k) of F: kinds 0 and 1 column-major, kind 2 (D^T)
+        // row-major
+        const bool tr = en.kind == 2;
+        const double *F[RF];
+#pragma unroll
+        for(int a = 0; a < RF; a++)
+            F[a] = fac+en.f_off+(tr ? (int64_t)row[a]*en.ld : row[a]);
+        const int64_t fs = tr ? 1 : en.ld;
+        const double *T = en.kind == 0 ? tmp+en.src_off*nrhs+qx :
+            x+en.src_off+(int64_t)qx*ldx;
+        const int ts = en.kind == 0 ? nrhs : 1;
+        int k0 = 0;
+        // a lane's four steps take k = 4 (lane/16) .. +3 of a block of 16
+        for(; k0+16 <= en.cols; k0 += 16)
         {
-            const tlr_entry en = entries[e];
-            if(!row_ok)
-                continue;
-            if(en.kind == 0)
-            {
-                // four independent partial sums over the factor columns
-                const double *F = fac+en.f_off+ch.rofs+lane;
-                const double *T = tmp+en.src_off*nrhs;
-                double a4[4][NQ] = {};
-                int c = 0;
-                // sixteen, then eight factor columns in flight at a time
-                // (column c always goes to partial sum c mod 4)
-                for(; c+16 <= en.cols; c += 16)
-                {
-                    double f16[16];
+            double f[RF][4], b[4];
 #pragma unroll
-                    for(int u = 0; u < 16; u++)
-                        f16[u] = F[(int64_t)(c+u)*en.ld];
+            for(int a = 0; a < RF; a++)
 #pragma unroll
-                    for(int u = 0; u < 16; u++)
+                for(int v = 0; v < 4; v++)
+                    f[a][v] = F[a][(k0+4*lr+v)*fs];
 #pragma unroll
-                        for(int q = 0; q < NQ; q++)
-                            if(NQ == 1 || q < nq)
-                                a4[u & 3][q] = fma(f16[u], T[c+u+
-                                        (int64_t)(q0+q)*en.cols], a4[u & 3][q]);
-                }
-                for(; c+8 <= en.cols; c += 8)
-                {
-                    double f8[8];
+            for(int v = 0; v < 4; v++)
+                b[v] = okq ? T[(int64_t)(k0+4*lr+v)*ts] : 0.0;
 #pragma unroll
-                    for(int u = 0; u < 8; u++)
-                        f8[u] = F[(int64_t)(c+u)*en.ld];
+            for(int v = 0; v < 4; v++)
 #pragma unroll
-                    for(int u = 0; u < 8; u++)
-#pragma unroll
-                        for(int q = 0; q < NQ; q++)
-                            if(NQ == 1 || q < nq)
-                                a4[u & 3][q] = fma(f8[u], T[c+u+
-                                        (int64_t)(q0+q)*en.cols], a4[u & 3][q]);
-                }
-                for(; c+4 <= en.cols; c += 4)
-#pragma unroll
-                    for(int u = 0; u < 4; u++)
-                    {
-                        const double f = F[(int64_t)(c+u)*en.ld];
-#pragma unroll
-                        for(int q = 0; q < NQ; q++)
-                            if(NQ == 1 || q < nq)
-                                a4[u][q] = fma(f, T[c+u+(int64_t)(q0+q)*
-                                        en.cols], a4[u][q]);
-                    }
-                for(; c < en.cols; c++)
-                {
-                    const double f = F[(int64_t)c*en.ld];
-#pragma unroll
-                    for(int q = 0; q < NQ; q++)
-                        if(NQ == 1 || q < nq)
-                            a4[0][q] = fma(f, T[c+(int64_t)(q0+q)*en.cols],
-                                    a4[0][q]);
-                }
-#pragma unroll
-                for(int q = 0; q < NQ; q++)
-                    acc[q] += (a4[0][q]+a4[1][q])+(a4[2][q]+a4[3][q]);
-            }
-            else if(en.kind == 3)
-            {
-                // a twin's contribution V T', formed by the coefficient pass
-                const double *P = tmp+en.src_off*nrhs+ch.rofs+lane;
-#pragma unroll
-                for(int q = 0; q < NQ; q++)
-                    if(NQ == 1 || q < nq)
-                        acc[q] += P[(int64_t)(q0+q)*en.ld];
-            }
-            else
-            {
-                const double *D = fac+en.f_off;
-                for(int c = 0; c < en.cols; c++)
-                {
-                    const int r = ch.rofs+lane;
-                    const double f = en.kind == 1 ?
-                        D[r+(int64_t)c*en.ld] : D[c+(int64_t)r*en.ld];
-#pragma unroll
-                    for(int q = 0; q < NQ; q++)
-                        if(NQ == 1 || q < nq)
-                            acc[q] = fma(f, x[en.src_off+c+
-                                    (int64_t)(q0+q)*ldx], acc[q]);
-                }
-            }
+                for(int a = 0; a < RF; a++)
+                    acc[a].add(f[a][v], b[v]);
         }
-#pragma unroll
-        for(int q = 0; q < NQ; q++)
-            part[wave][q][lane] = acc[q];
-        __syncthreads();
-        if(wave == 0 && row_ok)
+        if(k0 < en.cols)
         {
-            for(int q = 0; q < nq; q++)
+            // the last 1-15 columns, loaded together: step v takes
+            // k = k0 + 4 v + lane/16
+            const int steps = (en.cols-k0+3)/4;     // uniform
+            double f[RF][4], b[4];
+#pragma unroll
+            for(int v = 0; v < 4; v++)
+                if(v < steps)
+                {
+                    const int k = k0+4*v+lr;
+                    const bool okk = k < en.cols;
+#pragma unroll
+                    for(int a = 0; a < RF; a++)
+                        f[a][v] = okk ? F[a][k*fs] : 0.0;
+                    b[v] = okq && okk ? T[(int64_t)k*ts] : 0.0;
+                }
+#pragma unroll
+            for(int v = 0; v < 4; v++)
+                if(v < steps)
+#pragma unroll
+                    for(int a = 0; a < RF; a++)
+                        acc[a].add(f[a][v], b[v]);
+        }
+    }
+#pragma unroll
+    for(int a = 0; a < RF; a++)
+    {
+        acc[a].close();
+        if(wave > 0)
+#pragma unroll
+            for(int q = 0; q < Acc<ONE>::N; q++)
+                part[wave-1][a][q*64+lane] = acc[a].v[q];
+    }
+    __syncthreads();
+    if(wave == 0 && (ONE ? lane < 16 : okq))
+#pragma unroll
+        for(int a = 0; a < RF; a++)
+#pragma unroll
+            for(int q = 0; q < Acc<ONE>::N; q++)
             {
-                const double s = ((part[0][q][lane]+part[1][q][lane])+
-                        part[2][q][lane])+part[3][q][lane];
-                double *yy = y+(int64_t)(q0+q)*ldy+ch.row0+lane;
+                const int r = a*16+Acc<ONE>::row(q, lane);
+                if(r >= ch.nrows)
+                    continue;
+                const double s = ((acc[a].v[q]+part[0][a][q*64+lane])+
+                        part[1][a][q*64+lane])+part[2][a][q*64+lane];
+                double *yy = y+(int64_t)(ONE ? q0 : q0+lc)*ldy+ch.row0+r;
                 *yy = beta == 0.0 ? alpha*s : fma(alpha, s, beta*(*yy));
             }
-        }
-        __syncthreads();
-    }
 }
 
-// ---- vector kernels of conjugate gradients (one column of length n)
+// ---- vector kernels of conjugate gradients, one column of length n per
+// blockIdx.y (columns n apart).  Nothing of an iteration goes to the host:
+// the dot products stay as partial sums of at most CG_BLOCKS blocks, which
+// every block of the next kernel adds up in the same order, and a column that
+// has converged is left alone from then on.
 
-constexpr int DOT_BLOCKS = 256;
+constexpr int CG_BLOCKS = 256;
 
-// part[b] = sum over the block's grid-stride share of a[i]*b[i]
-__global__ __launch_bounds__(256) void dot_kernel(const double *a,
-        const double *b, int64_t n, double *part)
+// Sum of part[0 .. nb) by the whole block (nb <= 256 = blockDim.x), the same
+// value in every thread.
+__device__ inline double sum_parts(const double *part, int nb)
 {
     __shared__ double red[4];
-    double s = 0.0;
-    for(int64_t i = (int64_t)blockIdx.x*256+threadIdx.x; i < n;
-            i += (int64_t)gridDim.x*256)
-        s = fma(a[i], b[i], s);
+    double s = (int)threadIdx.x < nb ? part[threadIdx.x] : 0.0;
+#pragma unroll
+    for(int o = 32; o > 0; o >>= 1)
+        s += __shfl_xor(s, o, 64);
+    if((threadIdx.x & 63) == 0)
+        red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    s = ((red[0]+red[1])+red[2])+red[3];
+    __syncthreads();
+    return s;
+}
+
+__device__ inline void store_part(double s, double *out)
+{
+    __shared__ double red[4];
 #pragma unroll
     for(int o = 32; o > 0; o >>= 1)
         s += __shfl_xor(s, o, 64);
@@ -296,19 +359,87 @@ __global__ __launch_bounds__(256) void dot_kernel(const double *a,
         red[threadIdx.x >> 6] = s;
     __syncthreads();
     if(threadIdx.x == 0)
-        part[blockIdx.x] = ((red[0]+red[1])+red[2])+red[3];
+        *out = ((red[0]+red[1])+red[2])+red[3];
 }
 
-// out[0] = sum of part[0..np) in index order
-__global__ void sum_kernel(const double *part, int np, double *out)
+// part[b] = the block's share of a . b
+__global__ __launch_bounds__(256) void cg_dot_kernel(const double *a,
+        const double *b, int64_t n, double *part)
 {
-    if(threadIdx.x == 0 && blockIdx.x == 0)
+    a += blockIdx.y*n;
+    b += blockIdx.y*n;
+    double s = 0.0;
+    for(int64_t i = (int64_t)blockIdx.x*256+threadIdx.x; i < n;
+            i += (int64_t)gridDim.x*256)
+        s = fma(a[i], b[i], s);
+    store_part(s, part+(int64_t)blockIdx.y*CG_BLOCKS+blockIdx.x);
+}
+
+// State of a column before iteration 0 from |r|^2 (cg.c:44-52): the check
+// value tol |r_0| and |r_0|^2.
+__global__ __launch_bounds__(256) void cg_start_kernel(const double *part,
+        int nb, double tol, tlr_cg_state *st)
+{
+    const double rr = sum_parts(part+(int64_t)blockIdx.x*CG_BLOCKS, nb);
+    if(threadIdx.x == 0)
     {
-        double s = 0.0;
-        for(int i = 0; i < np; i++)
-            s += part[i];
-        out[0] = s;
+        const double rs = sqrt(rr);
+        tlr_cg_state &s = st[blockIdx.x];
+        s.rsold = rs*rs;
+        s.rscheck = rs*tol;
+        s.done = -1;
     }
+}
+
+// x += a p, r -= a q with a = rsold/(p . q); part2 = shares of |r|^2
+__global__ __launch_bounds__(256) void cg_step_kernel(int64_t n,
+        const tlr_cg_state *st, const double *part1, const double *p,
+        const double *q, double *x, double *r, double *part2)
+{
+    const tlr_cg_state s = st[blockIdx.y];
+    if(s.done >= 0)
+        return;
+    const int64_t o = blockIdx.y*n;
+    const double pq = sum_parts(part1+(int64_t)blockIdx.y*CG_BLOCKS,
+            gridDim.x);
+    const double a = s.rsold/pq;
+    double rr = 0.0;
+    for(int64_t i = (int64_t)blockIdx.x*256+threadIdx.x; i < n;
+            i += (int64_t)gridDim.x*256)
+    {
+        x[o+i] = fma(a, p[o+i], x[o+i]);
+        const double v = fma(-a, q[o+i], r[o+i]);
+        r[o+i] = v;
+        rr = fma(v, v, rr);
+    }
+    store_part(rr, part2+(int64_t)blockIdx.y*CG_BLOCKS+blockIdx.x);
+}
+
+// The stopping rule |r| < tol |r_0|, else p = r + |r|^2/rsold p; the new
+// state goes to st2 (other blocks still read st).
+__global__ __launch_bounds__(256) void cg_next_kernel(int64_t n, int it,
+        const tlr_cg_state *st, tlr_cg_state *st2, const double *part2,
+        const double *r, double *p)
+{
+    tlr_cg_state s = st[blockIdx.y];
+    if(s.done < 0)
+    {
+        const double rs = sqrt(sum_parts(part2+(int64_t)blockIdx.y*CG_BLOCKS,
+                    gridDim.x));
+        if(rs < s.rscheck)
+            s.done = it;
+        else
+        {
+            const double b = rs*rs/s.rsold;
+            s.rsold = rs*rs;
+            const int64_t o = blockIdx.y*n;
+            for(int64_t i = (int64_t)blockIdx.x*256+threadIdx.x; i < n;
+                    i += (int64_t)gridDim.x*256)
+                p[o+i] = fma(b, p[o+i], r[o+i]);
+        }
+    }
+    if(blockIdx.x == 0 && threadIdx.x == 0)
+        st2[blockIdx.y] = s;
 }
 
 // y = a*x + y
@@ -327,15 +458,6 @@ __global__ __launch_bounds__(256) void copy_kernel(int64_t n, const double *x,
     for(int64_t i = (int64_t)blockIdx.x*256+threadIdx.x; i < n;
             i += (int64_t)gridDim.x*256)
         y[i] = x[i];
-}
-
-// p = r + b*p
-__global__ __launch_bounds__(256) void xpby_kernel(int64_t n,
-        const double *r, double b, double *p)
-{
-    for(int64_t i = (int64_t)blockIdx.x*256+threadIdx.x; i < n;
-            i += (int64_t)gridDim.x*256)
-        p[i] = fma(b, p[i], r[i]);
 }
 
 inline unsigned vec_grid(int64_t n)
@@ -384,49 +506,86 @@ extern "C" int tlr_scratch(int device, double **ptr)
     return STARSH_SUCCESS;
 }
 
-int starsh_hip_tlr_apply(const tlr_tile *d_tiles, int ntiles,
-        const tlr_chunk *d_chunks, int nchunks, const tlr_entry *d_entries,
-        const double *d_fac, double *d_tmp, int nrhs, double alpha,
-        const double *d_x, int ldx, double beta, double *d_y, int ldy)
+int starsh_hip_tlr_apply(const tlr_plan *pl, double *d_tmp, int nrhs,
+        double alpha, const double *d_x, int ldx, double beta, double *d_y,
+        int ldy)
 {
     if(nrhs <= 0)
         return STARSH_SUCCESS;
     hipStream_t s = starsh_hip_stream();
-    if(ntiles > 0)
+    const unsigned groups = (nrhs+RHS-1)/RHS;
+    if(pl->nunits > 0)
     {
         if(nrhs == 1)
-            hipLaunchKernelGGL(tlr_coef_kernel<1>, dim3(ntiles), dim3(256),
-                    0, s, d_tiles, d_fac, d_x, ldx, nrhs, d_tmp);
+            hipLaunchKernelGGL(tlr_coef1_kernel, dim3(pl->nunits), dim3(256),
+                    0, s, pl->d_units, pl->d_fac, d_x, d_tmp);
         else
-            hipLaunchKernelGGL(tlr_coef_kernel<RHS_GROUP>, dim3(ntiles),
-                    dim3(256), 0, s, d_tiles, d_fac, d_x, ldx, nrhs, d_tmp);
+            hipLaunchKernelGGL(tlr_coef_kernel, dim3(pl->nunits, groups),
+                    dim3(256), 0, s, pl->d_units, pl->d_fac, d_x, ldx, nrhs,
+                    d_tmp);
         HIP_TRY(hipGetLastError());
     }
-    if(nchunks > 0)
+    if(pl->nchunks > 0)
     {
-        if(nrhs == 1)
-            hipLaunchKernelGGL(tlr_rows_kernel<1>, dim3(nchunks), dim3(256),
-                    0, s, d_chunks, d_entries, d_fac, d_tmp, d_x, ldx, nrhs,
-                    alpha, beta, d_y, ldy);
-        else
-            hipLaunchKernelGGL(tlr_rows_kernel<RHS_GROUP>, dim3(nchunks),
-                    dim3(256), 0, s, d_chunks, d_entries, d_fac, d_tmp, d_x,
-                    ldx, nrhs, alpha, beta, d_y, ldy);
+#define ROWS(RF, ONE) hipLaunchKernelGGL((tlr_rows_kernel<RF, ONE>), \
+        dim3(pl->nchunks, groups), dim3(256), 0, s, pl->d_chunks, \
+        pl->d_entries, pl->d_fac, d_tmp, d_x, ldx, nrhs, alpha, beta, d_y, \
+        ldy)
+        const bool one = nrhs == 1;
+        switch(pl->strip)
+        {
+            case 16: if(one) ROWS(1, true); else ROWS(1, false); break;
+            case 32: if(one) ROWS(2, true); else ROWS(2, false); break;
+            case 64: if(one) ROWS(4, true); else ROWS(4, false); break;
+            default: return STARSH_WRONG_PARAMETER;
+        }
+#undef ROWS
         HIP_TRY(hipGetLastError());
     }
     return STARSH_SUCCESS;
 }
 
-// *d_out = sum a[i]*b[i] (device scalar; d_part holds DOT_BLOCKS doubles)
-int starsh_hip_vdot(int64_t n, const double *d_a, const double *d_b,
-        double *d_part, double *d_out)
+static unsigned cg_grid(int64_t n)
 {
-    hipStream_t s = starsh_hip_stream();
-    hipLaunchKernelGGL(dot_kernel, dim3(DOT_BLOCKS), dim3(256), 0, s, d_a,
-            d_b, n, d_part);
+    const int64_t g = (n+255)/256;
+    return (unsigned)(g < CG_BLOCKS ? (g > 0 ? g : 1) : CG_BLOCKS);
+}
+
+int starsh_hip_cg_start(int64_t n, int nrhs, double tol, const double *d_r,
+        double *d_part, tlr_cg_state *d_st)
+{
+    const unsigned nb = cg_grid(n);
+    for(int q = 0; q < nrhs; q += 65535)
+        hipLaunchKernelGGL(cg_dot_kernel, dim3(nb, nrhs-q < 65535 ? nrhs-q :
+                    65535), dim3(256), 0, starsh_hip_stream(), d_r+q*n,
+                d_r+q*n, n, d_part+(int64_t)q*CG_BLOCKS);
+    hipLaunchKernelGGL(cg_start_kernel, dim3(nrhs), dim3(256), 0,
+            starsh_hip_stream(), d_part, (int)nb, tol, d_st);
     HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(sum_kernel, dim3(1), dim3(64), 0, s, d_part,
-            DOT_BLOCKS, d_out);
+    return STARSH_SUCCESS;
+}
+
+int starsh_hip_cg_iteration(int64_t n, int nrhs, int it, double *d_p,
+        const double *d_q, double *d_x, double *d_r, double *d_part,
+        tlr_cg_state *d_st)
+{
+    const unsigned nb = cg_grid(n);
+    hipStream_t s = starsh_hip_stream();
+    for(int q = 0; q < nrhs; q += 65535)
+    {
+        const unsigned cnt = nrhs-q < 65535 ? nrhs-q : 65535;
+        const tlr_cg_state *st = d_st+(int64_t)(it & 1)*nrhs+q;
+        tlr_cg_state *st2 = d_st+(int64_t)((it+1) & 1)*nrhs+q;
+        double *part1 = d_part+(int64_t)q*CG_BLOCKS;
+        double *part2 = part1+(int64_t)nrhs*CG_BLOCKS;
+        const int64_t o = q*n;
+        hipLaunchKernelGGL(cg_dot_kernel, dim3(nb, cnt), dim3(256), 0, s,
+                d_p+o, d_q+o, n, part1);
+        hipLaunchKernelGGL(cg_step_kernel, dim3(nb, cnt), dim3(256), 0, s, n,
+                st, part1, d_p+o, d_q+o, d_x+o, d_r+o, part2);
+        hipLaunchKernelGGL(cg_next_kernel, dim3(nb, cnt), dim3(256), 0, s, n,
+                it, st, st2, part2, d_r+o, d_p+o);
+    }
     HIP_TRY(hipGetLastError());
     return STARSH_SUCCESS;
 }
@@ -447,24 +606,15 @@ int starsh_hip_vcopy(int64_t n, const double *d_x, double *d_y)
     return STARSH_SUCCESS;
 }
 
-int starsh_hip_vxpby(int64_t n, const double *d_r, double b, double *d_p)
-{
-    hipLaunchKernelGGL(xpby_kernel, dim3(vec_grid(n)), dim3(256), 0,
-            starsh_hip_stream(), n, d_r, b, d_p);
-    HIP_TRY(hipGetLastError());
-    return STARSH_SUCCESS;
-}
-
 // Seconds per starsh_hip_tlr_apply (mean over reps launches after one
 // warm-up), measured with events on the library stream.
-int starsh_hip_tlr_time(const tlr_tile *d_tiles, int ntiles,
-        const tlr_chunk *d_chunks, int nchunks, const tlr_entry *d_entries,
-        const double *d_fac, double *d_tmp, int nrhs, const double *d_x,
-        int ldx, double *d_y, int ldy, int reps, double *seconds)
+int starsh_hip_tlr_time(const tlr_plan *pl, double *d_tmp, int nrhs,
+        const double *d_x, int ldx, double *d_y, int ldy, int reps,
+        double *seconds)
 {
     hipStream_t s = starsh_hip_stream();
-    int info = starsh_hip_tlr_apply(d_tiles, ntiles, d_chunks, nchunks,
-            d_entries, d_fac, d_tmp, nrhs, 1.0, d_x, ldx, 0.0, d_y, ldy);
+    int info = starsh_hip_tlr_apply(pl, d_tmp, nrhs, 1.0, d_x, ldx, 0.0,
+            d_y, ldy);
     if(info != STARSH_SUCCESS)
         return info;
     hipEvent_t e0, e1;
@@ -472,8 +622,8 @@ int starsh_hip_tlr_time(const tlr_tile *d_tiles, int ntiles,
     HIP_TRY(hipEventCreate(&e1));
     HIP_TRY(hipEventRecord(e0, s));
     for(int r = 0; r < reps && info == STARSH_SUCCESS; r++)
-        info = starsh_hip_tlr_apply(d_tiles, ntiles, d_chunks, nchunks,
-                d_entries, d_fac, d_tmp, nrhs, 1.0, d_x, ldx, 0.0, d_y, ldy);
+        info = starsh_hip_tlr_apply(pl, d_tmp, nrhs, 1.0, d_x, ldx, 0.0, d_y,
+                ldy);
     HIP_TRY(hipEventRecord(e1, s));
     HIP_TRY(hipEventSynchronize(e1));
     float ms = 0.f;

@@ -1,0 +1,169 @@
+"""Products with compressed matrices at the sizes where the kernels of
+csrc/hip/tlr.hip change course: row strips of 16, 32 and 64, tiles that are
+no multiple of 16 or 64 rows, ranks around the 16- and 32-column groups and
+the 64-column pieces of an entry, one right-hand side (lane sums) and more
+(MFMA, groups of 16), dense tiles and their transposes."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import starsh_hip as S
+
+pytestmark = pytest.mark.gpu
+
+
+def _array(a):
+    A = C.POINTER(S.Array)()
+    assert S.lib().array_from_buffer(
+        C.byref(A), C.c_int(2), (C.c_int*2)(*a.shape), C.c_char(b"d"),
+        C.c_char(b"F"), a.ctypes.data_as(C.c_void_p)) == 0
+    return A
+
+
+def _ints(v):
+    libc = C.CDLL(None)
+    libc.malloc.restype = C.c_void_p
+    a = (S.STARSH_int*max(1, len(v)))(*v)
+    p = libc.malloc(C.c_size_t(C.sizeof(a)))
+    C.memmove(p, a, C.sizeof(a))
+    return C.cast(p, C.POINTER(S.STARSH_int))
+
+
+def _operator(N, nb, symm, ranks, rng):
+    """A BLRM of random factors; ranks cycle over the tiles, -1: dense.
+    Returns it, the dense matrix and what has to stay alive."""
+    p = S.TLRProblem("spatial", N, 2, nb, symm=symm, kernel="exp",
+                     points=rng.random((2, N)))
+    st, sz = p.cluster_ranges()
+    A = np.zeros((N, N))
+    far, near, U, V, D, rk, keep = [], [], [], [], [], [], [p]
+    for t, (i, j) in enumerate(p.tiles()):
+        r = ranks[t % len(ranks)]
+        ri, rj = slice(st[i], st[i]+sz[i]), slice(st[j], st[j]+sz[j])
+        if r < 0:
+            d = np.asfortranarray(rng.standard_normal((sz[i], sz[j])))
+            keep.append(d)
+            near += [i, j]
+            D.append(_array(d))
+            block = d
+        else:
+            r = min(r, sz[i], sz[j])
+            u = np.asfortranarray(rng.standard_normal((sz[i], r)))
+            v = np.asfortranarray(rng.standard_normal((sz[j], r)))
+            keep += [u, v]
+            far += [i, j]
+            rk.append(r)
+            U.append(_array(u))
+            V.append(_array(v))
+            block = u @ v.T
+        A[ri, rj] = block
+        if symm == "S" and i != j:
+            A[rj, ri] = block.T
+    F = C.POINTER(S.BLRF)()
+    assert S.lib().starsh_blrf_new_from_coo(
+        C.byref(F), p.P, C.c_char(symm.encode()), p.C, p.C,
+        S.STARSH_int(len(rk)), _ints(far), S.STARSH_int(len(D)),
+        _ints(near), C.c_int(p.F.contents.type)) == 0
+    M = S.BLRM()
+    PA = C.POINTER(S.Array)
+    M.format = F
+    M.far_rank = (C.c_int*max(1, len(rk)))(*rk)
+    M.far_U = (PA*max(1, len(U)))(*U)
+    M.far_V = (PA*max(1, len(V)))(*V)
+    M.near_D = (PA*max(1, len(D)))(*D)
+    M.onfly = 0
+    return M, A, keep
+
+
+@pytest.mark.parametrize("N,nb,symm,ranks", [
+    (40, 40, "S", [3]),
+    (37, 15, "N", [1, 0, 15, -1]),
+    (331, 47, "S", [16, 17, -1, 0, 1]),
+    (1030, 250, "S", [31, 32, 33, -1]),
+    (1030, 250, "N", [64, 65, 15, -1, 100]),
+    (500, 100, "S", [0]),
+    (17000, 2048, "S", [5, 40, 1]),
+    (33000, 1601, "N", [2, 18])])
+def test_products(N, nb, symm, ranks):
+    L = S.lib()
+    rng = np.random.default_rng(N)
+    if N > 5000:
+        # too large to hold densely: products of the factors instead
+        M, apply, keep = _large(N, nb, symm, ranks, rng)
+    else:
+        M, A, keep = _operator(N, nb, symm, ranks, rng)
+
+        def apply(X):
+            return A @ X
+    for nrhs in ([1, 3] if N > 5000 else [1, 2, 15, 16, 17, 33]):
+        print(f"N={N} nb={nb} {symm} ranks {ranks} nrhs {nrhs}", flush=True)
+        X = np.asfortranarray(rng.standard_normal((N, nrhs)))
+        Y = np.asfortranarray(rng.standard_normal((N, nrhs)))
+        ref = 1.5*apply(X)-0.25*Y
+        dp = C.POINTER(C.c_double)
+        assert L.starsh_blrm__dmml_hip(
+            C.cast(C.byref(M), C.c_void_p), nrhs, 1.5, X.ctypes.data_as(dp),
+            N, -0.25, Y.ctypes.data_as(dp), N) == 0
+        # sums of at most N products of up to 100 terms each
+        scale = max(np.max(np.abs(ref)), 1.0)
+        assert np.max(np.abs(Y-ref)) <= 1e-13*scale*np.sqrt(N)
+
+
+def _large(N, nb, symm, ranks, rng):
+    p = S.TLRProblem("spatial", N, 2, nb, symm=symm, kernel="exp",
+                     points=rng.random((2, N)))
+    st, sz = p.cluster_ranges()
+    parts, U, V, rk, keep = [], [], [], [], [p]
+    for t, (i, j) in enumerate(p.tiles()):
+        r = ranks[t % len(ranks)]
+        u = np.asfortranarray(rng.standard_normal((sz[i], r)))
+        v = np.asfortranarray(rng.standard_normal((sz[j], r)))
+        parts.append((slice(st[i], st[i]+sz[i]), slice(st[j], st[j]+sz[j]),
+                      u, v, symm == "S" and i != j))
+        keep += [u, v]
+        rk.append(r)
+        U.append(_array(u))
+        V.append(_array(v))
+    M = S.BLRM()
+    PA = C.POINTER(S.Array)
+    M.format = p.F
+    M.far_rank = (C.c_int*len(rk))(*rk)
+    M.far_U = (PA*len(U))(*U)
+    M.far_V = (PA*len(V))(*V)
+    M.onfly = 0
+
+    def apply(X):
+        Y = np.zeros_like(X)
+        for ri, rj, u, v, both in parts:
+            Y[ri] += u @ (v.T @ X[rj])
+            if both:
+                Y[rj] += v @ (u.T @ X[ri])
+        return Y
+    return M, apply, keep
+
+
+@pytest.mark.parametrize("nrhs", [1, 3])
+def test_cg_columns_stop_on_their_own(nrhs):
+    """Columns that converge at different iterations, among them one that
+    is solved from the start, against the dense solution."""
+    N = 700
+    fn = S.init("HIP", oversample=16)
+    rng = np.random.default_rng(3)
+    p = S.TLRProblem("spatial", N, 2, 100, kernel="exp", beta=0.1,
+                     noise=0.5, points=rng.random((2, N)))
+    assert p.approximate(60, 1e-9, 0, fn) == 0
+    A = p.dmml(np.eye(N))
+    X = rng.standard_normal((N, nrhs))
+    if nrhs > 1:
+        X[:, 1] = np.linalg.eigh(0.5*(A+A.T))[1][:, -1]
+    B = A @ X
+    it, Y = p.cg(B, np.zeros_like(B), 1e-10)
+    print("iterations", it, flush=True)
+    assert 0 < it < N
+    # |x - x'| <= cond |r|/|b| |x|, cond below |A|/noise
+    cond = np.linalg.norm(A, 2)/0.5
+    for q in range(nrhs):
+        assert np.linalg.norm(Y[:, q]-X[:, q]) <= 2e-10*cond*np.linalg.norm(
+            X[:, q])
+    p.free_matrix()
