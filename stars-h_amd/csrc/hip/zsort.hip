@@ -10,15 +10,23 @@
 //   key = sum_{b, d} bit b of u_d at position b*ndim + d,
 // with points of equal key in their original order when the key has an
 // even number of 1 bits and in reverse order when odd (each 1 bit reverses
-// them once).  Here that order is produced by a stable LSD radix sort on
-// the composite key (Morton key, then the original index or its reverse by
-// that parity), 8 bits per pass:
+// them once).  Here a stable LSD radix sort on the Morton key, 8 bits per
+// pass, leaves equal keys in their original order, and the gather reverses
+// the groups of odd parity:
 //   zs_minmax_*   per-dimension min and max (exact, any reduction order);
 //   zs_key        the key words of every point;
-//   zs_hist       per-tile digit counts;  zs_scan  offsets (digit-major);
-//   zs_scatter    stable scatter: each tile ranks its points by digit in
-//                 their order, with wave ballots for ranks inside a wave;
-//   zs_gather     the permuted coordinates.
+//   zs_load       the word being sorted by, in the current order;
+//   zs_hist       per-tile digit counts;  zs_scan  offsets within a digit;
+//   zs_scatter    stable scatter of (word, index): each tile ranks its points
+//                 by digit in their order, with wave ballots for ranks
+//                 inside a wave;
+//   zs_gather     groups of equal keys, permutation and coordinates.
+//
+// What bounds it: launches and the scattered writes of a pass.  A million
+// points in 3D (12 passes) take 0.50 ms on MI355X; with one workgroup
+// scanning all digit counts of a pass (432 of the 510 us of a pass), all key
+// words moved in every pass and three passes for the tie-break it was 7.6
+// ms.
 #include <stdio.h>
 #include <algorithm>
 #include <utility>
@@ -69,67 +77,95 @@ __global__ __launch_bounds__(ZT) void zs_minmax_partial(const double *x,
     }
 }
 
-__global__ void zs_minmax_final(const double *part, int nb, int ndim,
-        double *mm)
+// One block per dimension: mm[d] = min, mm[ndim + d] = max.
+__global__ __launch_bounds__(ZT) void zs_minmax_final(const double *part,
+        int nb, int ndim, double *mm)
 {
-    // one thread per dimension: mm[d] = min, mm[ndim + d] = max
-    const int d = threadIdx.x;
-    if(d >= ndim)
-        return;
+    __shared__ double smin[ZT/64], smax[ZT/64];
+    const int d = blockIdx.x;
     double lo = INFINITY, hi = -INFINITY;
-    for(int b = 0; b < nb; b++)
+    for(int b = threadIdx.x; b < nb; b += ZT)
     {
         lo = fmin(lo, part[((int64_t)b*ndim+d)*2]);
         hi = fmax(hi, part[((int64_t)b*ndim+d)*2+1]);
     }
-    mm[d] = lo;
-    mm[ndim+d] = hi;
+    for(int o = 32; o > 0; o >>= 1)
+    {
+        lo = fmin(lo, __shfl_xor(lo, o, 64));
+        hi = fmax(hi, __shfl_xor(hi, o, 64));
+    }
+    if((threadIdx.x & 63) == 0)
+    {
+        smin[threadIdx.x >> 6] = lo;
+        smax[threadIdx.x >> 6] = hi;
+    }
+    __syncthreads();
+    if(threadIdx.x == 0)
+    {
+        for(int w = 1; w < ZT/64; w++)
+        {
+            lo = fmin(lo, smin[w]);
+            hi = fmax(hi, smax[w]);
+        }
+        mm[d] = lo;
+        mm[ndim+d] = hi;
+    }
 }
 
-// Key words of point i (SoA, nw words of n): word 0 = tie-break (original
-// index, or its reverse when the key has an odd number of 1 bits), words
-// 1..ndim = the Morton key, least significant word first.
+// Key words of point i (SoA, NDIM words of n, least significant first).
+template <int NDIM>
 __global__ __launch_bounds__(ZT) void zs_key(const double *x, int64_t n,
-        int ndim, const double *mm, uint32_t *key, uint32_t *idx)
+        const double *mm, uint32_t *key, uint32_t *idx)
 {
     const int64_t i = (int64_t)blockIdx.x*ZT+threadIdx.x;
     if(i >= n)
         return;
-    uint32_t u[4];
-    for(int d = 0; d < ndim; d++)
+    uint32_t u[NDIM];
+#pragma unroll
+    for(int d = 0; d < NDIM; d++)
     {
-        const double lo = mm[d], range = mm[ndim+d]-lo;
+        const double lo = mm[d], range = mm[NDIM+d]-lo;
         // the reference's expression: (x - min)/range*UINT32_MAX, then
         // conversion to uint32 (truncation)
         const double v = (x[(int64_t)d*n+i]-lo)/range*4294967295.0;
         u[d] = (uint32_t)v;
     }
-    // bit b of u_d goes to key bit b*ndim + d; key word w holds bits
+    // bit b of u_d goes to key bit b*NDIM + d; key word w holds bits
     // 32w .. 32w+31
-    uint32_t w[4] = {0, 0, 0, 0};
+    uint32_t w[NDIM];
+#pragma unroll
+    for(int q = 0; q < NDIM; q++)
+        w[q] = 0;
+#pragma unroll
     for(int b = 0; b < 32; b++)
-        for(int d = 0; d < ndim; d++)
+#pragma unroll
+        for(int d = 0; d < NDIM; d++)
         {
-            const int pos = b*ndim+d;
+            const int pos = b*NDIM+d;
             w[pos >> 5] |= ((u[d] >> b) & 1u) << (pos & 31);
         }
-    int ones = 0;
-    for(int q = 0; q < ndim; q++)
-        ones += __popc(w[q]);
-    key[i] = (ones & 1) ? (uint32_t)(n-1-i) : (uint32_t)i;
-    for(int q = 0; q < ndim; q++)
-        key[(int64_t)(q+1)*n+i] = w[q];
+#pragma unroll
+    for(int q = 0; q < NDIM; q++)
+        key[(int64_t)q*n+i] = w[q];
     idx[i] = (uint32_t)i;
 }
 
-__device__ inline uint32_t digit_of(const uint32_t *key, int64_t n, int word,
-        int shift, int64_t i)
+// wk[i] = the word of the point at place i.
+__global__ __launch_bounds__(ZT) void zs_load(const uint32_t *key, int64_t n,
+        const uint32_t *idx, uint32_t *wk)
 {
-    return (key[(int64_t)word*n+i] >> shift) & (NDIG-1);
+    const int64_t i = (int64_t)blockIdx.x*ZT+threadIdx.x;
+    if(i < n)
+        wk[i] = key[min((int64_t)idx[i], n-1)];
 }
 
-__global__ __launch_bounds__(ZT) void zs_hist(const uint32_t *key,
-        int64_t n, int word, int shift, uint32_t *hist, int ntile)
+__device__ inline uint32_t digit_of(const uint32_t *wk, int shift, int64_t i)
+{
+    return (wk[i] >> shift) & (NDIG-1);
+}
+
+__global__ __launch_bounds__(ZT) void zs_hist(const uint32_t *wk, int64_t n,
+        int shift, uint32_t *hist, int ntile)
 {
     __shared__ uint32_t cnt[NDIG];
     cnt[threadIdx.x] = 0;
@@ -139,52 +175,71 @@ __global__ __launch_bounds__(ZT) void zs_hist(const uint32_t *key,
     {
         const int64_t i = t0+r*ZT+threadIdx.x;
         if(i < n)
-            atomicAdd(&cnt[digit_of(key, n, word, shift, i)], 1u);
+            atomicAdd(&cnt[digit_of(wk, shift, i)], 1u);
     }
     __syncthreads();
     hist[(int64_t)threadIdx.x*ntile+blockIdx.x] = cnt[threadIdx.x];
 }
 
-// Exclusive scan of m values in one block of 1024 threads (sequential
-// chunks, running total carried between them).
-__global__ __launch_bounds__(1024) void zs_scan(uint32_t *v, int64_t m)
+// Exclusive scan over a block of ZT threads; *total is the sum.
+__device__ inline uint32_t block_scan(uint32_t v, uint32_t *wsum,
+        uint32_t *total)
 {
-    __shared__ uint32_t s[1024];
-    __shared__ uint32_t carry;
-    if(threadIdx.x == 0)
-        carry = 0;
-    __syncthreads();
-    for(int64_t c0 = 0; c0 < m; c0 += 1024)
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t x = v;
+    for(int o = 1; o < 64; o <<= 1)
     {
-        const int64_t i = c0+threadIdx.x;
-        const uint32_t x = i < m ? v[i] : 0;
-        s[threadIdx.x] = x;
-        __syncthreads();
-        for(int o = 1; o < 1024; o <<= 1)
-        {
-            const uint32_t y = threadIdx.x >= (unsigned)o ?
-                s[threadIdx.x-o] : 0;
-            __syncthreads();
-            s[threadIdx.x] += y;
-            __syncthreads();
-        }
-        if(i < m)
-            v[i] = carry+s[threadIdx.x]-x;
-        __syncthreads();
-        if(threadIdx.x == 1023)
-            carry += s[1023];
-        __syncthreads();
+        const uint32_t y = __shfl_up(x, o, 64);
+        if(lane >= o)
+            x += y;
     }
+    if(lane == 63)
+        wsum[wave] = x;
+    __syncthreads();
+    uint32_t before = 0, all = 0;
+    for(int w = 0; w < ZT/64; w++)
+    {
+        before += w < wave ? wsum[w] : 0;
+        all += wsum[w];
+    }
+    __syncthreads();
+    *total = all;
+    return before+x-v;
 }
 
-__global__ __launch_bounds__(ZT) void zs_scatter(const uint32_t *key,
-        const uint32_t *idx, uint32_t *key2, uint32_t *idx2, int64_t n,
-        int nw, int word, int shift, const uint32_t *off, int ntile)
+// One block per digit: exclusive scan of its ntile counts in place, their
+// sum to total[digit].
+__global__ __launch_bounds__(ZT) void zs_scan(uint32_t *hist, int ntile,
+        uint32_t *total)
+{
+    __shared__ uint32_t wsum[ZT/64];
+    uint32_t *v = hist+(int64_t)blockIdx.x*ntile;
+    uint32_t carry = 0;
+    for(int c0 = 0; c0 < ntile; c0 += ZT)
+    {
+        const int i = c0+threadIdx.x;
+        uint32_t sum;
+        const uint32_t x = block_scan(i < ntile ? v[i] : 0, wsum, &sum);
+        if(i < ntile)
+            v[i] = carry+x;
+        carry += sum;
+    }
+    if(threadIdx.x == 0)
+        total[blockIdx.x] = carry;
+}
+
+__global__ __launch_bounds__(ZT) void zs_scatter(const uint32_t *wk,
+        const uint32_t *idx, uint32_t *wk2, uint32_t *idx2, int64_t n,
+        int shift, const uint32_t *off, const uint32_t *total, int ntile)
 {
     __shared__ uint32_t base[NDIG];      // tile offset + points placed so far
     __shared__ uint32_t wcnt[ZT/64][NDIG];
+    __shared__ uint32_t wsum[ZT/64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    base[threadIdx.x] = off[(int64_t)threadIdx.x*ntile+blockIdx.x];
+    // digit offsets: every block scans the 256 totals for itself
+    uint32_t all;
+    base[threadIdx.x] = block_scan(total[threadIdx.x], wsum, &all)+
+        off[(int64_t)threadIdx.x*ntile+blockIdx.x];
     const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64-lane));
     const int64_t t0 = (int64_t)blockIdx.x*TILE;
     for(int r = 0; r < ZI; r++)
@@ -195,7 +250,8 @@ __global__ __launch_bounds__(ZT) void zs_scatter(const uint32_t *key,
         // points of this round, in order: thread t takes t0 + r*ZT + t
         const int64_t i = t0+r*ZT+threadIdx.x;
         const bool valid = i < n;
-        const uint32_t dg = valid ? digit_of(key, n, word, shift, i) : 0;
+        const uint32_t word = valid ? wk[i] : 0;
+        const uint32_t dg = (word >> shift) & (NDIG-1);
         // lanes of this wave with the same digit
         uint64_t peers = __ballot(valid);
         for(int b = 0; b < 8; b++)
@@ -216,8 +272,7 @@ __global__ __launch_bounds__(ZT) void zs_scatter(const uint32_t *key,
             // test keeps a wrong offset from writing out of bounds
             if(pos >= (uint64_t)n)
                 pos = (uint32_t)(n-1);
-            for(int q = 0; q < nw; q++)
-                key2[(int64_t)q*n+pos] = key[(int64_t)q*n+i];
+            wk2[pos] = word;
             idx2[pos] = idx[i];
         }
         __syncthreads();
@@ -229,13 +284,62 @@ __global__ __launch_bounds__(ZT) void zs_scatter(const uint32_t *key,
     }
 }
 
+// -1, 0, 1 as the key of point a is below, equal to or above that of b.
+__device__ inline int key_cmp(const uint32_t *key, int64_t n, int ndim,
+        uint32_t a, uint32_t b)
+{
+    for(int q = ndim-1; q >= 0; q--)
+    {
+        const uint32_t ka = key[(int64_t)q*n+a], kb = key[(int64_t)q*n+b];
+        if(ka != kb)
+            return ka < kb ? -1 : 1;
+    }
+    return 0;
+}
+
+// The point of place i: idx[i], or, in a group of equal keys (places lo ..
+// hi-1, found by bisection) with an odd number of 1 bits, idx[lo+hi-1-i].
+// wk: the most significant key words in order.
 __global__ __launch_bounds__(ZT) void zs_gather(const double *x, int64_t n,
-        int ndim, const uint32_t *idx, double *y, int64_t *order)
+        int ndim, const uint32_t *key, const uint32_t *wk,
+        const uint32_t *idx, double *y, int64_t *order)
 {
     const int64_t i = (int64_t)blockIdx.x*ZT+threadIdx.x;
     if(i >= n)
         return;
     uint32_t j = idx[i];
+    const bool tied = (i > 0 && wk[i-1] == wk[i] &&
+            key_cmp(key, n, ndim, idx[i-1], j) == 0) ||
+        (i+1 < n && wk[i+1] == wk[i] &&
+         key_cmp(key, n, ndim, idx[i+1], j) == 0);
+    if(tied)
+    {
+        int ones = 0;
+        for(int q = 0; q < ndim; q++)
+            ones += __popc(key[(int64_t)q*n+j]);
+        if(ones & 1)
+        {
+            int64_t lo = 0, hi = i;         // first place not below j's key
+            while(lo < hi)
+            {
+                const int64_t mid = (lo+hi)/2;
+                if(key_cmp(key, n, ndim, idx[mid], j) < 0)
+                    lo = mid+1;
+                else
+                    hi = mid;
+            }
+            int64_t first = i+1, last = n;  // first place above it
+            while(first < last)
+            {
+                const int64_t mid = (first+last)/2;
+                if(key_cmp(key, n, ndim, idx[mid], j) <= 0)
+                    first = mid+1;
+                else
+                    last = mid;
+            }
+            j = idx[lo+first-1-i];
+        }
+    }
     j = j < (uint64_t)n ? j : 0;
     for(int d = 0; d < ndim; d++)
         y[(int64_t)d*n+i] = x[(int64_t)d*n+j];
@@ -260,48 +364,58 @@ extern "C" int starsh_hip_zsort(const double *d_x, int64_t n, int ndim,
     if(info != STARSH_SUCCESS)
         return info;
     hipStream_t s = starsh_hip_stream();
-    const int nw = ndim+1;
     const int ntile = (int)((n+TILE-1)/TILE);
     const int nbmm = (int)std::min<int64_t>((n+ZT-1)/ZT, 1024);
-    // scratch: min/max partials, key words and indices twice, histogram
+    // scratch: min/max partials, key words, the sorted word and the indices
+    // twice, histogram and digit totals
     size_t bytes = sizeof(double)*((size_t)nbmm*ndim*2+2*ndim)+
-        sizeof(uint32_t)*(2*(size_t)n*nw+2*(size_t)n+(size_t)NDIG*ntile);
+        sizeof(uint32_t)*((size_t)n*ndim+4*(size_t)n+(size_t)NDIG*ntile+
+                NDIG);
     char *buf = nullptr;
     HIP_TRY(hipMallocAsync((void **)&buf, bytes, s));
     double *part = (double *)buf;
     double *mm = part+(size_t)nbmm*ndim*2;
     uint32_t *key = (uint32_t *)(mm+2*ndim);
-    uint32_t *key2 = key+(size_t)n*nw;
-    uint32_t *idx = key2+(size_t)n*nw;
+    uint32_t *wk = key+(size_t)n*ndim;
+    uint32_t *wk2 = wk+n;
+    uint32_t *idx = wk2+n;
     uint32_t *idx2 = idx+n;
     uint32_t *hist = idx2+n;
+    uint32_t *total = hist+(size_t)NDIG*ntile;
     const unsigned nb = (unsigned)((n+ZT-1)/ZT);
     hipLaunchKernelGGL(zs_minmax_partial, dim3(nbmm), dim3(ZT), 0, s, d_x, n,
             ndim, part);
-    hipLaunchKernelGGL(zs_minmax_final, dim3(1), dim3(64), 0, s, part, nbmm,
-            ndim, mm);
-    hipLaunchKernelGGL(zs_key, dim3(nb), dim3(ZT), 0, s, d_x, n, ndim, mm,
-            key, idx);
-    // word 0 (tie-break) needs only the bits of indices below n
-    int tbits = 0;
-    while(tbits < 32 && ((int64_t)1 << tbits) < n)
-        tbits++;
-    for(int word = 0; word < nw; word++)
+    hipLaunchKernelGGL(zs_minmax_final, dim3(ndim), dim3(ZT), 0, s, part,
+            nbmm, ndim, mm);
+    switch(ndim)
+    {
+        case 1: hipLaunchKernelGGL(zs_key<1>, dim3(nb), dim3(ZT), 0, s, d_x,
+                    n, mm, key, idx); break;
+        case 2: hipLaunchKernelGGL(zs_key<2>, dim3(nb), dim3(ZT), 0, s, d_x,
+                    n, mm, key, idx); break;
+        case 3: hipLaunchKernelGGL(zs_key<3>, dim3(nb), dim3(ZT), 0, s, d_x,
+                    n, mm, key, idx); break;
+        default: hipLaunchKernelGGL(zs_key<4>, dim3(nb), dim3(ZT), 0, s, d_x,
+                    n, mm, key, idx); break;
+    }
+    for(int word = 0; word < ndim; word++)
+    {
+        hipLaunchKernelGGL(zs_load, dim3(nb), dim3(ZT), 0, s,
+                key+(size_t)word*n, n, idx, wk);
         for(int shift = 0; shift < 32; shift += 8)
         {
-            if(word == 0 && shift >= tbits)
-                break;
-            hipLaunchKernelGGL(zs_hist, dim3(ntile), dim3(ZT), 0, s, key, n,
-                    word, shift, hist, ntile);
-            hipLaunchKernelGGL(zs_scan, dim3(1), dim3(1024), 0, s, hist,
-                    (int64_t)NDIG*ntile);
-            hipLaunchKernelGGL(zs_scatter, dim3(ntile), dim3(ZT), 0, s, key,
-                    idx, key2, idx2, n, nw, word, shift, hist, ntile);
-            std::swap(key, key2);
+            hipLaunchKernelGGL(zs_hist, dim3(ntile), dim3(ZT), 0, s, wk, n,
+                    shift, hist, ntile);
+            hipLaunchKernelGGL(zs_scan, dim3(NDIG), dim3(ZT), 0, s, hist,
+                    ntile, total);
+            hipLaunchKernelGGL(zs_scatter, dim3(ntile), dim3(ZT), 0, s, wk,
+                    idx, wk2, idx2, n, shift, hist, total, ntile);
+            std::swap(wk, wk2);
             std::swap(idx, idx2);
         }
+    }
     hipLaunchKernelGGL(zs_gather, dim3(nb), dim3(ZT), 0, s, d_x, n, ndim,
-            idx, d_y, d_order);
+            key, wk, idx, d_y, d_order);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipFreeAsync(buf, s));
     HIP_TRY(hipStreamSynchronize(s));
