@@ -33,8 +33,11 @@ double starsh_blrm__dfe_hip_tiles(STARSH_blrm *matrix, double *far_err,
     int64_t *vo = malloc(sizeof(int64_t)*(nt+1));
     double *a2 = malloc(sizeof(double)*(nt+1));
     double *d2 = malloc(sizeof(double)*(nt+1));
-    double *hU = NULL, *hV = NULL, *dU = NULL, *dV = NULL;
-    if(!m || !n || !rk || !r0 || !c0 || !uo || !vo || !a2 || !d2)
+    const double **seg = malloc(sizeof(*seg)*(2*nfar+1));
+    int64_t *seglen = malloc(sizeof(int64_t)*(2*nfar+1));
+    double *dU = NULL, *dV = NULL;
+    if(!m || !n || !rk || !r0 || !c0 || !uo || !vo || !a2 || !d2 || !seg ||
+            !seglen)
         goto done;
     int64_t su = 0, sv = 0;
     for(STARSH_int bi = 0; bi < nt; bi++)
@@ -55,19 +58,18 @@ double starsh_blrm__dfe_hip_tiles(STARSH_blrm *matrix, double *far_err,
         su += (int64_t)m[bi]*rk[bi];
         sv += (int64_t)n[bi]*rk[bi];
     }
-    hU = malloc(sizeof(double)*su+1);
-    hV = malloc(sizeof(double)*sv+1);
-    if(!hU || !hV)
-        goto done;
+    /* U of every far-field tile, then V */
     for(STARSH_int bi = 0; bi < nfar; bi++)
     {
-        memcpy(hU+uo[bi], M->far_U[bi]->data, sizeof(double)*m[bi]*rk[bi]);
-        memcpy(hV+vo[bi], M->far_V[bi]->data, sizeof(double)*n[bi]*rk[bi]);
+        seg[bi] = rk[bi] > 0 ? M->far_U[bi]->data : NULL;
+        seglen[bi] = (int64_t)m[bi]*rk[bi];
+        seg[nfar+bi] = rk[bi] > 0 ? M->far_V[bi]->data : NULL;
+        seglen[nfar+bi] = (int64_t)n[bi]*rk[bi];
     }
     if(starsh_hip_malloc((void **)&dU, sizeof(double)*su) != 0 ||
             starsh_hip_malloc((void **)&dV, sizeof(double)*sv) != 0 ||
-            starsh_hip_memcpy_h2d(dU, hU, sizeof(double)*su) != 0 ||
-            starsh_hip_memcpy_h2d(dV, hV, sizeof(double)*sv) != 0)
+            hip_upload_segments(dU, nfar, seg, seglen) != 0 ||
+            hip_upload_segments(dV, nfar, seg+nfar, seglen+nfar) != 0)
         goto done;
     if(starsh_hip_tile_errors(&hp.kd, hp.d_xr, hp.nr, hp.d_xc, hp.nc,
                 (int)nt, r0, c0, m, n, rk, dU, uo, dV, vo, a2, d2) != 0)
@@ -103,7 +105,7 @@ double starsh_blrm__dfe_hip_tiles(STARSH_blrm *matrix, double *far_err,
 done:
     starsh_hip_free(dU);
     starsh_hip_free(dV);
-    free(hU); free(hV); free(m); free(n); free(rk); free(r0); free(c0);
+    free(seg); free(seglen); free(m); free(n); free(rk); free(r0); free(c0);
     free(uo); free(vo); free(a2); free(d2);
     hip_driver_release(&hp);
     return result;

@@ -16,6 +16,7 @@
 #include <string.h>
 #include "common.h"
 #include "starsh-hip.h"
+#include "rsdd.h"
 #include "tlr.h"
 
 struct starsh_hip_tlr
@@ -133,7 +134,13 @@ int starsh_hip_tlr_new(starsh_hip_tlr **out, STARSH_blrm *M)
         nunits += (int64_t)((M->far_rank[bi]+31)/32)*
             (symm && F->block_far[2*bi] != F->block_far[2*bi+1] ? 2 : 1);
     int64_t *count = calloc(nbr+1, sizeof(int64_t));
-    double *hfac = malloc(sizeof(double)*(nfac > 0 ? nfac : 1));
+    /* the host arrays that make up the factor buffer, in order; dense tiles
+     * on the fly are generated into hnear first */
+    const STARSH_int nseg = 2*nfar+nnear;
+    const double **seg = malloc(sizeof(*seg)*(nseg > 0 ? nseg : 1));
+    int64_t *seglen = malloc(sizeof(int64_t)*(nseg > 0 ? nseg : 1));
+    double *hnear = M->onfly == 0 ? NULL : malloc(sizeof(double)*(nfac > 0 ?
+                nfac : 1));
     tlr_unit *hunits = malloc(sizeof(tlr_unit)*(nunits > 0 ? nunits : 1));
     tlr_far *hfar = malloc(sizeof(tlr_far)*(nfar > 0 ? nfar : 1));
     int64_t *nearoff = malloc(sizeof(int64_t)*(nnear > 0 ? nnear : 1));
@@ -141,7 +148,7 @@ int starsh_hip_tlr_new(starsh_hip_tlr **out, STARSH_blrm *M)
     tlr_entry *hent = NULL;
     tlr_chunk *hch = NULL;
     int info = STARSH_MALLOC_ERROR;
-    if(!count || !hfac || !hunits || !hfar || !nearoff || !T)
+    if(!count || !seg || !seglen || (M->onfly != 0 && !hnear) || !hunits || !hfar || !nearoff || !T)
         goto fail;
     T->nrows = P->shape[0];
     T->ncols = P->shape[P->ndim-1];
@@ -154,12 +161,12 @@ int starsh_hip_tlr_new(starsh_hip_tlr **out, STARSH_blrm *M)
         const int twin = symm && i != j;
         tlr_far *t = &hfar[bi];
         t->u_off = (int64_t)off;
-        if(r > 0)
-            memcpy(hfac+off, M->far_U[bi]->data, sizeof(double)*m*r);
+        seg[2*bi] = r > 0 ? M->far_U[bi]->data : NULL;
+        seglen[2*bi] = (int64_t)m*r;
         off += (size_t)m*r;
         t->v_off = (int64_t)off;
-        if(r > 0)
-            memcpy(hfac+off, M->far_V[bi]->data, sizeof(double)*n*r);
+        seg[2*bi+1] = r > 0 ? M->far_V[bi]->data : NULL;
+        seglen[2*bi+1] = (int64_t)n*r;
         off += (size_t)n*r;
         t->tmp_off = tmp;
         tmp += 2*(int64_t)r;
@@ -178,11 +185,11 @@ int starsh_hip_tlr_new(starsh_hip_tlr **out, STARSH_blrm *M)
         STARSH_int i = F->block_near[2*bi], j = F->block_near[2*bi+1];
         int m = (int)R->size[i], n = (int)C->size[j];
         nearoff[bi] = (int64_t)off;
-        if(M->onfly == 0)
-            memcpy(hfac+off, M->near_D[bi]->data, sizeof(double)*m*n);
-        else
+        seg[2*nfar+bi] = M->onfly == 0 ? M->near_D[bi]->data : hnear+off;
+        seglen[2*nfar+bi] = (int64_t)m*n;
+        if(M->onfly != 0)
             P->kernel(m, n, R->pivot+R->start[i], C->pivot+C->start[j],
-                    R->data, C->data, hfac+off, m);
+                    R->data, C->data, hnear+off, m);
         off += (size_t)m*n;
         count[i] += pieces(n);
         if(symm && i != j)
@@ -254,7 +261,10 @@ int starsh_hip_tlr_new(starsh_hip_tlr **out, STARSH_blrm *M)
     T->fac_doubles = off;
     T->tmp_units = tmp;
     T->noalloc_units = tmp+twins;
-    info = upload((void **)&T->plan.d_fac, hfac, sizeof(double)*off);
+    info = off == 0 ? STARSH_SUCCESS :
+        starsh_hip_malloc((void **)&T->plan.d_fac, sizeof(double)*off);
+    if(info == STARSH_SUCCESS)
+        info = hip_upload_segments(T->plan.d_fac, nseg, seg, seglen);
     if(info == STARSH_SUCCESS)
         info = upload((void **)&T->plan.d_units, hunits, sizeof(tlr_unit)*nu);
     if(info == STARSH_SUCCESS)
@@ -265,7 +275,9 @@ int starsh_hip_tlr_new(starsh_hip_tlr **out, STARSH_blrm *M)
     if(info != STARSH_SUCCESS)
         goto fail;
     free(count);
-    free(hfac);
+    free(seg);
+    free(seglen);
+    free(hnear);
     free(hunits);
     free(hfar);
     free(nearoff);
@@ -275,7 +287,9 @@ int starsh_hip_tlr_new(starsh_hip_tlr **out, STARSH_blrm *M)
     return STARSH_SUCCESS;
 fail:
     free(count);
-    free(hfac);
+    free(seg);
+    free(seglen);
+    free(hnear);
     free(hunits);
     free(hfar);
     free(nearoff);

@@ -706,6 +706,7 @@ void rsdd_release_pools(void)
     for(PanelGraph &pg : panel_graphs)
         pg.reset();
     rsdd_out_release();
+    hip_upload_release();
 }
 
 extern "C" int starsh_hip_proj_int8(int on)

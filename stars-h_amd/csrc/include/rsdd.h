@@ -120,6 +120,13 @@ int rsdd_out_submit(const double *d_src, int64_t len, int nseg,
 int rsdd_out_end(double *window_seconds, double *tail_seconds);
 void rsdd_out_release(void);
 
+/* Upload of nseg host arrays (len[q] doubles at src[q]), one after the other,
+ * to d_dst (csrc/hip/copyin.hip); waits for it.  hip_upload_release frees
+ * its pinned ring. */
+int hip_upload_segments(double *d_dst, int64_t nseg,
+        const double *const *src, const int64_t *len);
+void hip_upload_release(void);
+
 /* Frees the workspace and staging buffers kept between calls. */
 void rsdd_release_pools(void);
 

@@ -84,7 +84,8 @@ def _operator(N, nb, symm, ranks, rng):
     (1030, 250, "N", [64, 65, 15, -1, 100]),
     (500, 100, "S", [0]),
     (17000, 2048, "S", [5, 40, 1]),
-    (33000, 1601, "N", [2, 18])])
+    (33000, 1601, "N", [2, 18]),
+    (33000, 1601, "N", [30])])
 def test_products(N, nb, symm, ranks):
     L = S.lib()
     rng = np.random.default_rng(N)
@@ -141,6 +142,50 @@ def _large(N, nb, symm, ranks, rng):
                 Y[rj] += v @ (u.T @ X[ri])
         return Y
     return M, apply, keep
+
+
+def test_uploads_from_two_threads():
+    """Two operators uploaded at the same time (the second finds the pinned
+    ring taken): both hold the same factors, so their products are the
+    same, bit for bit."""
+    import threading
+    L = S.lib()
+    N = 20000
+    M, apply, keep = _large(N, 1000, "N", [10, 20], np.random.default_rng(1))
+    T = [C.c_void_p(), C.c_void_p()]
+    info = [None, None]
+
+    def make(q):
+        info[q] = L.starsh_hip_tlr_new(C.byref(T[q]), C.byref(M))
+
+    threads = [threading.Thread(target=make, args=(q,)) for q in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert info == [0, 0]
+    X = np.random.default_rng(2).standard_normal(N)
+    out = []
+    d = [C.c_void_p(), C.c_void_p()]
+    for x in d:
+        assert L.starsh_hip_malloc(C.byref(x), C.c_size_t(8*N)) == 0
+    vp = C.c_void_p
+    assert L.starsh_hip_memcpy_h2d(d[0], X.ctypes.data_as(vp),
+                                   C.c_size_t(8*N)) == 0
+    for t in T:
+        Y = np.zeros(N)
+        assert L.starsh_hip_tlr_dmml(t, C.c_int(1), C.c_double(1.0), d[0],
+                                     C.c_int(N), C.c_double(0.0), d[1],
+                                     C.c_int(N)) == 0
+        assert L.starsh_hip_memcpy_d2h(Y.ctypes.data_as(vp), d[1],
+                                       C.c_size_t(8*N)) == 0
+        out.append(Y)
+        L.starsh_hip_tlr_free(t)
+    for x in d:
+        L.starsh_hip_free(x)
+    assert np.array_equal(out[0], out[1])
+    ref = apply(X[:, None])[:, 0]
+    assert np.max(np.abs(out[0]-ref)) <= 1e-13*np.max(np.abs(ref))*np.sqrt(N)
 
 
 @pytest.mark.parametrize("nrhs", [1, 3])
