@@ -696,7 +696,6 @@ int hip_driver_run(const hip_batch *B, STARSH_int ntiles, const int *pidx,
             bytes += tb;
             st->flops_algorithmic += 4.0*m[b1]*(double)n[b1]*
                 (mr+os < mn ? mr+os : mn);
-            st->sketch_bytes_or_flops += 2.0*m[b1]*(double)n[b1]*kk;
             b1++;
         }
         RsddInput in;
@@ -757,6 +756,7 @@ int hip_driver_run(const hip_batch *B, STARSH_int ntiles, const int *pidx,
             break;
         st->device_seconds += out.device_seconds;
         st->dominant_kernel_seconds += out.sketch_seconds;
+        st->sketch_bytes_or_flops += out.sketch_flops;
         st->proj_kernel_seconds += out.proj_seconds;
         st->dominant_kernel_launches += 1;
         double tc = hip_driver_now();

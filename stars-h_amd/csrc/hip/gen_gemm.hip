@@ -26,10 +26,12 @@ int gen_gemm_tuned_rw[2] = {0, 0};
 
 // PROJ=false: rows are row points, K runs over column points.
 // PROJ=true : rows are column points, K runs over row points (A^T).
-// gnbm x gnbn is the block grid of the largest tile of the launch.
+// gnbm x gnbn is the block grid of the largest tile of the launch.  SKETCH:
+// columns cbeg..cend-1 only, and no tile whose range the columns before them
+// have exhausted already.
 template <int NDIM, int FAM, int BN, int RW, bool PROJ>
 __global__ __launch_bounds__(256) void gen_gemm_kernel(const TileDesc *tiles,
-        GemmArgs g, int ntiles, int gnbm, int gnbn)
+        GemmArgs g, int ntiles, int gnbm, int gnbn, int cbeg, int cend)
 {
     constexpr int NF = BN/16;
     constexpr int BMR = BM*RW;      // rows per block: RW 16-row groups/wave
@@ -45,7 +47,9 @@ __global__ __launch_bounds__(256) void gen_gemm_kernel(const TileDesc *tiles,
     int64_t nrow, nk;
     if(!PROJ)
     {
-        M = t.m; N = t.k; K = t.n;
+        if(t.flags & 1)
+            return;
+        M = t.m; N = t.k < cend ? t.k : cend; K = t.n;
         B = g.ws+t.om_off; ldb = t.n;
         C = g.ws+t.q_off; ldc = t.m;
         rbase = t.r0; kbase = t.c0;
@@ -63,9 +67,9 @@ __global__ __launch_bounds__(256) void gen_gemm_kernel(const TileDesc *tiles,
     }
     if(M <= 0 || N <= 0)
         return;
-    if(bm*BMR >= M || bn*BN >= N)
+    const int row0 = bm*BMR, col0 = cbeg+bn*BN;
+    if(row0 >= M || col0 >= N)
         return;
-    const int row0 = bm*BMR, col0 = bn*BN;
     // 16-column fragments that hold columns of this tile (wave-uniform)
     const int nf_live = (N-col0+15)/16 < NF ? (N-col0+15)/16 : NF;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -237,73 +241,62 @@ __global__ __launch_bounds__(256) void gen_gemm_kernel(const TileDesc *tiles,
 }
 
 template <int NDIM, int FAM, int BN, int RW, bool PROJ>
-int launch_one(const TileDesc *d_tiles, int ntiles, int mmax, int nmax,
-        const GemmArgs &g, hipStream_t s)
+int launch_one(const TileDesc *d_tiles, int ntiles, int mmax, int cbeg,
+        int cend, const GemmArgs &g, hipStream_t s)
 {
     const int nbm = (mmax+BM*RW-1)/(BM*RW);
-    const int nbn = (nmax+BN-1)/BN;
+    const int nbn = (cend-cbeg+BN-1)/BN;
     const int64_t grid = mapped_grid(ntiles, nbm, nbn, !PROJ);
     if(grid > 0x7fffffff)
         return STARSH_WRONG_PARAMETER;
     hipLaunchKernelGGL((gen_gemm_kernel<NDIM, FAM, BN, RW, PROJ>),
             dim3((unsigned)grid), dim3(256), 0, s, d_tiles, g, ntiles, nbm,
-            nbn);
+            nbn, cbeg, cend);
     HIP_TRY(hipGetLastError());
     return STARSH_SUCCESS;
-}
-
-template <int NDIM, int FAM, bool PROJ>
-int launch_nd(const TileDesc *d_tiles, int ntiles, int mmax, int nmax,
-        const GemmArgs &g, hipStream_t s)
-{
-    // By size (measured on MI355X at tile 1600): the sketch's wide
-    // column blocks reuse each generated entry most; the projection (N =
-    // kept columns, often just under a multiple of 256) wastes less on
-    // 128-column blocks with two 16-row groups per wave.
-    int bn, rw;
-    if(PROJ)
-    {
-        bn = nmax > 64 ? 128 : 64;
-        rw = nmax > 64 ? 2 : 1;
-    }
-    else
-    {
-        bn = nmax > 128 ? 256 : (nmax > 64 ? 128 : 64);
-        rw = 1;
-    }
-    if(gen_gemm_tuned_bn[PROJ] > 0)
-        bn = gen_gemm_tuned_bn[PROJ];
-    if(gen_gemm_tuned_rw[PROJ] > 0)
-        rw = gen_gemm_tuned_rw[PROJ];
-    if(gen_gemm_bn > 0)
-        bn = gen_gemm_bn;
-    if(gen_gemm_rw > 0)
-        rw = gen_gemm_rw;
-    if(bn == 256)
-        return rw == 2 ? launch_one<NDIM, FAM, 256, 2, PROJ>(d_tiles, ntiles,
-                mmax, nmax, g, s) : launch_one<NDIM, FAM, 256, 1, PROJ>(
-                d_tiles, ntiles, mmax, nmax, g, s);
-    if(bn == 128)
-        return rw == 2 ? launch_one<NDIM, FAM, 128, 2, PROJ>(d_tiles, ntiles,
-                mmax, nmax, g, s) : launch_one<NDIM, FAM, 128, 1, PROJ>(
-                d_tiles, ntiles, mmax, nmax, g, s);
-    return rw == 2 ? launch_one<NDIM, FAM, 64, 2, PROJ>(d_tiles, ntiles,
-            mmax, nmax, g, s) : launch_one<NDIM, FAM, 64, 1, PROJ>(d_tiles,
-            ntiles, mmax, nmax, g, s);
 }
 
 template <bool PROJ>
 struct GenLaunch
 {
     const TileDesc *tiles;
-    int ntiles, mmax, nmax;
+    int ntiles, mmax, cbeg, cend, bn, rw;
     const GemmArgs &g;
     hipStream_t s;
     template <int NDIM, int FAM> int operator()() const
     {
-        return launch_nd<NDIM, FAM, PROJ>(tiles, ntiles, mmax, nmax, g, s);
+#define ONE(BN, RW) return launch_one<NDIM, FAM, BN, RW, PROJ>(tiles, \
+        ntiles, mmax, cbeg, cend, g, s)
+        if(bn == 256)
+        {
+            if(rw == 2)
+                ONE(256, 2);
+            ONE(256, 1);
+        }
+        if(bn == 128)
+        {
+            if(rw == 2)
+                ONE(128, 2);
+            ONE(128, 1);
+        }
+        if(rw == 2)
+            ONE(64, 2);
+        ONE(64, 1);
+#undef ONE
     }
 };
+
+// Column block and row groups forced by the options or the autotuner (0:
+// not).
+int forced_bn(int proj)
+{
+    return gen_gemm_bn > 0 ? gen_gemm_bn : gen_gemm_tuned_bn[proj];
+}
+
+int forced_rw(int proj)
+{
+    return gen_gemm_rw > 0 ? gen_gemm_rw : gen_gemm_tuned_rw[proj];
+}
 
 } // namespace
 
@@ -333,14 +326,71 @@ extern "C" int starsh_hip_gen_gemm_bn(int bn)
     return STARSH_SUCCESS;
 }
 
-int pipeline_gen_gemm(int proj, const TileDesc *d_tiles, int ntiles,
-        int mmax, int nmax, const GemmArgs &g, hipStream_t s)
+// The sketch's columns go in chunks, computed as the Gram-Schmidt reaches
+// them: a tile whose range is exhausted by then has no use for the rest (the
+// random columns after that point are dropped unread).  A chunk is one column
+// block.  Wide blocks reuse each generated entry most (820 tiles of 1600,
+// 2D sqexp: 22.6 ms for a block of 256, 14.4 for 128), so the first chunk is
+// narrow only where tiles that need every column lose nothing by it: with
+// more than 256 columns, when the padding that the narrow blocks save pays
+// for them (417-448 and 513-640 columns, say, but not 449-512).  2D sqexp
+// N=64000, 416 columns, all tiles exhausted within 96: sketch 45.3 -> 15.3
+// ms; sin(kr)/r N=25000, 400 columns, 17 of 153 tiles needing all: 11.7 ->
+// 9.4 ms.
+int pipeline_sketch_chunks(int k, SketchChunk *c)
+{
+    const int fb = forced_bn(0), rw = forced_rw(0) > 0 ? forced_rw(0) : 1;
+    int n = 0;
+    auto add = [&](int beg, int bn) {
+        const int end = beg+bn < k ? beg+bn : k;
+        c[n++] = SketchChunk{beg, end, bn, rw};
+        return end;
+    };
+    // block for the last r columns, and its cost
+    auto block = [](int r) { return r <= 64 ? 64 : r <= 128 ? 128 : 256; };
+    auto cost = [](int bn) {
+        return bn == 64 ? 9.5 : bn == 128 ? 14.4 : 22.6; };
+    int beg = 0;
+    if(fb > 0)
+        while(beg < k)
+            beg = add(beg, fb);
+    else if(k <= 256)
+        add(0, block(k));
+    else
+    {
+        const int rest = k-128;
+        const double wide = (k+255)/256*cost(256);
+        const double narrow = cost(128)+rest/256*cost(256)+
+            (rest % 256 ? cost(block(rest % 256)) : 0.0);
+        beg = add(0, narrow <= 1.03*wide ? 128 : 256);
+        while(beg < k)
+            beg = add(beg, k-beg > 256 ? 256 : block(k-beg));
+    }
+    return n;
+}
+
+int pipeline_sketch_gen(const TileDesc *d_tiles, int ntiles, int mmax,
+        const SketchChunk &c, const GemmArgs &g, hipStream_t s)
+{
+    if(ntiles <= 0 || mmax <= 0 || c.end <= c.beg)
+        return STARSH_SUCCESS;
+    return dispatch_kernel(g.ndim, g.family, GenLaunch<false>{d_tiles,
+            ntiles, mmax, c.beg, c.end, c.bn, c.rw, g, s});
+}
+
+int pipeline_proj_gen(const TileDesc *d_tiles, int ntiles, int mmax,
+        int nmax, const GemmArgs &g, hipStream_t s)
 {
     if(ntiles <= 0 || mmax <= 0 || nmax <= 0)
         return STARSH_SUCCESS;
-    if(proj)
-        return dispatch_kernel(g.ndim, g.family, GenLaunch<true>{d_tiles,
-                ntiles, mmax, nmax, g, s});
-    return dispatch_kernel(g.ndim, g.family, GenLaunch<false>{d_tiles,
-            ntiles, mmax, nmax, g, s});
+    // By size (measured at tile 1600): N = kept columns, often just under a
+    // multiple of 256, wastes less on 128-column blocks with two 16-row
+    // groups per wave.
+    int bn = nmax > 64 ? 128 : 64, rw = nmax > 64 ? 2 : 1;
+    if(forced_bn(1) > 0)
+        bn = forced_bn(1);
+    if(forced_rw(1) > 0)
+        rw = forced_rw(1);
+    return dispatch_kernel(g.ndim, g.family, GenLaunch<true>{d_tiles, ntiles,
+            mmax, 0, nmax, bn, rw, g, s});
 }

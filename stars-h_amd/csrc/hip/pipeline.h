@@ -31,10 +31,20 @@ int pipeline_r2_split(int ntiles, int pmax, int kmax_rows);
 int pipeline_r2(const TileDesc *d_tiles, int ntiles, int pmax, int nz,
         double *d_part, const GemmArgs &g, hipStream_t s);
 
-// Sketch (proj = 0) or projection (proj = 1) with the kernel tile generated
-// in registers (gen_gemm.hip).
-int pipeline_gen_gemm(int proj, const TileDesc *d_tiles, int ntiles,
-        int mmax, int nmax, const GemmArgs &g, hipStream_t s);
+// Sketch and projection with the kernel tile generated in registers
+// (gen_gemm.hip).  The sketch of k columns goes in chunks (at most
+// SKETCH_CHUNKS): pipeline_sketch_chunks fills c and returns their number,
+// pipeline_sketch_gen computes one, skipping tiles with flag 1.
+struct SketchChunk
+{
+    int beg, end, bn, rw;
+};
+constexpr int SKETCH_CHUNKS = 64;
+int pipeline_sketch_chunks(int k, SketchChunk *c);
+int pipeline_sketch_gen(const TileDesc *d_tiles, int ntiles, int mmax,
+        const SketchChunk &c, const GemmArgs &g, hipStream_t s);
+int pipeline_proj_gen(const TileDesc *d_tiles, int ntiles, int mmax,
+        int nmax, const GemmArgs &g, hipStream_t s);
 
 // Column norms of the m x k buffers (which = 0) or of Bt (which = 2) into
 // d_norm (ntiles x kmax).

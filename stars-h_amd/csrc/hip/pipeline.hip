@@ -7,6 +7,7 @@
 #include <stdlib.h>
 #include <string.h>
 #include <algorithm>
+#include <functional>
 #include <map>
 #include <thread>
 #include <chrono>
@@ -162,15 +163,20 @@ struct PanelGraph
 };
 PanelGraph panel_graphs[2];      // which = 0, 1
 
+// need(c): makes the first c columns of the sketch available (the launches
+// it queues precede the block that reads them); empty if they all are.
 int bcgs2(TileDesc *d_tiles, int ntiles, int which, double *ws, int kmax,
         int width_max, int rows_max, int *d_keep, double *d_norms,
-        double *d_coef, double tau_first, int *d_active, hipStream_t s)
+        double *d_coef, double tau_first, int *d_active, hipStream_t s,
+        const std::function<int(int)> &need = nullptr)
 {
     const int pw = qr_panel_width ? qr_panel_width : qr_panel_tuned;
     const bool wide = pw != 4;
     const int pb = rows_max <= 2048 && wide ? 8 : 4;
     if(qr_graph)
     {
+        if(need)
+            TRY(need(width_max));
         PanelGraph &pg = panel_graphs[which ? 1 : 0];
         const PanelGraph::Key key{d_tiles, ws, d_keep, d_active, d_norms,
             d_coef, ntiles, which, kmax, width_max, rows_max, pb, tau_first};
@@ -234,6 +240,8 @@ int bcgs2(TileDesc *d_tiles, int ntiles, int which, double *ws, int kmax,
             if(probe.h[slot] == 0)
                 break;
         }
+        if(need)
+            TRY(need(std::min(gs_next(j0), width_max)));
         TRY(pipeline_gs_block(d_tiles, ntiles, which, ws, j0, pb, kmax,
                     tau_first, TAU_SECOND, d_keep, d_norms, d_coef, rows_max,
                     d_active, s));
@@ -532,18 +540,25 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
     {
         hipEvent_t e[6] = {nullptr, nullptr, nullptr, nullptr, nullptr,
             nullptr};
+        // begin and end of every sketch launch after the first
+        std::vector<hipEvent_t> more;
         ~Events()
         {
             for(auto x : e)
                 if(x)
                     (void)hipEventDestroy(x);
+            for(auto x : more)
+                (void)hipEventDestroy(x);
         }
     } evs;
     hipEvent_t *ev = evs.e;
     for(int e = 0; e < 6; e++)
         HIP_TRY(hipEventCreate(&ev[e]));
     HIP_TRY(hipEventRecord(ev[0], s));
-    // 1. sketch
+    // 1. sketch (of generated FP64 tiles its first chunk of columns: the
+    // others follow when the Gram-Schmidt reaches them)
+    SketchChunk chunk[SKETCH_CHUNKS];
+    int nchunk = 0, chunks_done = 0;
     HIP_TRY(hipEventRecord(ev[2], s));
     if(select)
         TRY(pipeline_select(d_tiles, nt, mmax, kmax, g.ndim, d_ws,
@@ -560,7 +575,11 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
         if(in->d_a)
             TRY(pipeline_gemm(GM_SKETCH_MEM, d_tiles, nt, mmax, kmax, g, s));
         else
-            TRY(pipeline_gen_gemm(0, d_tiles, nt, mmax, kmax, g, s));
+        {
+            nchunk = pipeline_sketch_chunks(kmax, chunk);
+            TRY(pipeline_sketch_gen(d_tiles, nt, mmax, chunk[0], g, s));
+            chunks_done = 1;
+        }
     }
     HIP_TRY(hipEventRecord(ev[3], s));
     dump("omega", d_ws+h[0].om_off, (int64_t)h[0].n*h[0].k, s);
@@ -570,7 +589,22 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
     HIP_TRY(hipMemsetAsync(keep.p, 0, sizeof(int)*(size_t)nt*kmax, s));
     TRY(bcgs2(d_tiles, nt, 0, d_ws, kmax, kmax, mmax, (int *)keep.p,
                 (double *)norms.p, (double *)coef.p,
-                in->tau > 0 ? in->tau : TAU_FIRST, (int *)active.p, s));
+                in->tau > 0 ? in->tau : TAU_FIRST, (int *)active.p, s,
+                nchunk <= 1 ? std::function<int(int)>() : [&](int c) -> int {
+                    while(chunks_done < nchunk && chunk[chunks_done].beg < c)
+                    {
+                        hipEvent_t e0, e1;
+                        HIP_TRY(hipEventCreate(&e0));
+                        evs.more.push_back(e0);
+                        HIP_TRY(hipEventCreate(&e1));
+                        evs.more.push_back(e1);
+                        HIP_TRY(hipEventRecord(e0, s));
+                        TRY(pipeline_sketch_gen(d_tiles, nt, mmax,
+                                    chunk[chunks_done++], g, s));
+                        HIP_TRY(hipEventRecord(e1, s));
+                    }
+                    return STARSH_SUCCESS;
+                }));
     dump("Qfull", d_ws+h[0].q_off, (int64_t)h[0].m*h[0].k, s);
     TRY(pipeline_compact(d_tiles, nt, d_ws, (int *)keep.p, kmax, s));
     dump("Q", d_ws+h[0].q_off, (int64_t)h[0].m*h[0].k, s);
@@ -588,7 +622,7 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
                     (const signed char *)qd.p, s));
     }
     else
-        TRY(pipeline_gen_gemm(1, d_tiles, nt, nmax, kmax, g, s));
+        TRY(pipeline_proj_gen(d_tiles, nt, nmax, kmax, g, s));
     HIP_TRY(hipEventRecord(ev[5], s));
     dump("Bt", d_ws+h[0].bt_off, (int64_t)h[0].n*h[0].k, s);
     // 4. truncation of B's rows
@@ -603,6 +637,19 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
     // first CORE_PMAX rows; the squared norms of the rows dropped are added
     // to its tail, as for the truncation itself, so the rank rule stays
     // conservative (flag 8).
+    // columns sketched: all, or, of a tile exhausted in the block at gs_blk,
+    // the chunks up to the one that holds that block
+    double sketch_flops = 0.0;
+    for(int t = 0; t < nt; t++)
+    {
+        int cols = h[t].k;
+        if(nchunk > 1 && (h[t].flags & 1))
+            for(int c = 0; c < nchunk; c++)
+                if(chunk[c].beg <= h[t].gs_blk && chunk[c].end < cols &&
+                        chunk[c].end > h[t].gs_blk)
+                    cols = chunk[c].end;
+        sketch_flops += 2.0*h[t].m*(double)h[t].n*cols;
+    }
     int pmax = 0;
     bool capped = false, certify = false;
     for(int t = 0; t < nt; t++)
@@ -678,7 +725,14 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
     HIP_TRY(hipEventElapsedTime(&ms_pr, ev[4], ev[5]));
     out->proj_seconds = ms_pr*1e-3;
     out->device_seconds = ms*1e-3;
+    for(size_t e = 0; e+1 < evs.more.size(); e += 2)
+    {
+        float more = 0;
+        HIP_TRY(hipEventElapsedTime(&more, evs.more[e], evs.more[e+1]));
+        ms_sk += more;
+    }
     out->sketch_seconds = ms_sk*1e-3;
+    out->sketch_flops = sketch_flops;
     for(int t = 0; t < nt; t++)
     {
         out->rank[t] = h[t].rank;

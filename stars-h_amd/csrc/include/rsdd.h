@@ -84,7 +84,8 @@ typedef struct rsdd_output
                                     the pipeline and valid until its next
                                     call */
     double device_seconds;
-    double sketch_seconds;       /* sketch kernel (HIP events) */
+    double sketch_seconds;       /* sketch kernels (HIP events) */
+    double sketch_flops;         /* 2 m n flop per sketch column computed */
     double proj_seconds;         /* projection kernels (HIP events) */
 } RsddOutput;
 
