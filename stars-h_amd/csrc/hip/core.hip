@@ -13,7 +13,7 @@
 // singular values; Jacobi on R2^T converges in fewer sweeps than on R2.
 #include <float.h>
 #include "pipeline.h"
-#include "jacobi_rotation.h"
+#include "jacobi_fast.h"
 
 namespace {
 
@@ -40,10 +40,10 @@ __device__ inline bool rotate_pair(double *wa, double *wb, int p, int g,
     al = group_sum(al, g);
     be = group_sum(be, g);
     ga = group_sum(ga, g);
-    if(!jr_rotates(al, be, ga, ctol))
+    if(!jr_rotates_fast(al, be, ga, ctol))
         return false;
     double c, s;
-    jacobi_rotation(al, be, ga, c, s);
+    jacobi_rotation_fast(al, be, ga, c, s);
     for(int i = gl; i < p; i += g)
     {
         double u = wa[i], v = wb[i];
@@ -80,10 +80,10 @@ __device__ inline bool rotate_pair_reg(double *wa, double *wb, int p, int g,
     al = group_sum(al, g);
     be = group_sum(be, g);
     ga = group_sum(ga, g);
-    if(!jr_rotates(al, be, ga, ctol))
+    if(!jr_rotates_fast(al, be, ga, ctol))
         return false;
     double c, s;
-    jacobi_rotation(al, be, ga, c, s);
+    jacobi_rotation_fast(al, be, ga, c, s);
 #pragma unroll
     for(int q = 0; q < E; q++)
     {
@@ -123,9 +123,10 @@ __device__ void jacobi(double *W, int p, int max_sweeps, int *sweeps_out)
             for(int pi = grp; pi < npairs; pi += ngroups)
             {
                 // Circle method: position 0 fixed, others rotate.
-                int x = pi, y = pe-1-pi;
-                int a = x == 0 ? 0 : 1+(x-1+round) % (pe-1);
-                int b = 1+(y-1+round) % (pe-1);
+                int a = pi+round, b = pe-1-pi+round;
+                a = a > pe-1 ? a-(pe-1) : a;
+                b = b > pe-1 ? b-(pe-1) : b;
+                a = pi == 0 ? 0 : a;
                 if(a > b)
                 {
                     int tmp = a;
@@ -358,7 +359,8 @@ extern "C" int starsh_hip_jacobi_sweeps(int sweeps)
 }
 
 int pipeline_core(TileDesc *d_tiles, int ntiles, double *ws, int pmax,
-        bool certify, int *d_active, int *h_active, hipStream_t s)
+        bool certify, int *d_list, int count, int *d_out, int *h_out,
+        hipStream_t s)
 {
     if(ntiles <= 0)
         return STARSH_SUCCESS;
@@ -387,8 +389,8 @@ int pipeline_core(TileDesc *d_tiles, int ntiles, double *ws, int pmax,
     }
     if(pm > lds_p)
     {
-        const int info = pipeline_jacobi_block(d_tiles, ntiles, ws, lds_p,
-                pm, jacobi_max_sweeps, certify, d_active, h_active, s);
+        const int info = pipeline_jacobi_block(d_tiles, d_list, count, ws,
+                pm, jacobi_max_sweeps, certify, d_out, h_out, s);
         if(info != STARSH_SUCCESS)
             return info;
         const size_t bytes = sizeof(double)*2*((size_t)pm+1)+

@@ -1,6 +1,6 @@
 // Core SVD of the tiles whose p x p core does not fit in LDS (p >
-// CORE_LDS_PMAX, core.hip): one-sided block Jacobi with the work of every tile spread over
-// the chip.
+// CORE_LDS_PMAX, core.hip): one-sided block Jacobi with the work of every
+// tile spread over the chip.
 //
 // The columns of W = R2^T are split into blocks of 32.  A sweep visits every
 // pair of blocks once, in rounds of disjoint pairs (circle method), one
@@ -26,14 +26,16 @@
 // 7-8 (numpy model on sin(kr)/r, exp and Matern cores).
 // Measured on MI355X, all launches of one compression, against one
 // workgroup per tile: 2D exp N=9973, tile 1000, SVD engine (10 cores of
-// 1000, 45 of 200-500) 1570 -> 32 ms; sin(kr)/r N=25000, tile 1536 (17 of
-// 400, 85 of 130-210) 163 -> 12 ms; 3D Matern N=65536, tile 2048, mixed
-// (up to 528) 191 -> 81 ms; a round of 500 pairs takes 120-160 us, of 1700
-// pairs 280 us.
+// 1000, 45 of 200-500) 1570 -> 23 ms; sin(kr)/r N=25000, tile 1536 (17 of
+// 400, 85 of 130-210) 163 -> 7.8 ms; 3D Matern N=65536, tile 2048, mixed
+// (up to 528) 191 -> 65 ms.  A round of a few hundred pairs takes 115-130 us,
+// about 95 of them the 63 steps, with nothing to rotate 13-19 us.  Only
+// tiles still rotating are launched, by a list the sweeps shorten: empty
+// workgroups of 68 KB of LDS queued for their turn (Matern 82 -> 69 ms).
 #include <float.h>
 #include <math.h>
 #include "pipeline.h"
-#include "jacobi_rotation.h"
+#include "jacobi_fast.h"
 
 typedef double double4_t __attribute__((ext_vector_type(4)));
 
@@ -41,7 +43,7 @@ namespace {
 
 constexpr int BW = 32;          // columns per block
 constexpr int PW = 2*BW;        // columns per block pair
-constexpr int NT = 256;
+constexpr int NT = 512;         // of a round: 8 waves
 
 __device__ inline int ld_of(int p)
 {
@@ -55,73 +57,98 @@ __device__ inline int blocks_of(int p)
     return nb+(nb & 1);
 }
 
-// jacobi_rotation() with two reciprocal square roots and no division: with
-// d = be - al, h = 2 ga and r = sqrt(d^2 + h^2), c^2 = (1 + |d|/r)/2 and
-// s = sign(d) h/(2 r c), the smaller of the two angles.  Outside the range
-// where the squares are safe it is jacobi_rotation() itself.
-__device__ inline void rotation(double al, double be, double ga, double &c,
-        double &s)
+// The 10 16 x 16 blocks of the upper triangle of G, five for each half of
+// the waves.
+constexpr int GA[2][5] = {{0, 0, 1, 0, 1}, {0, 1, 2, 3, 2}};
+constexpr int GB[2][5] = {{0, 1, 1, 2, 2}, {3, 3, 3, 3, 2}};
+
+// One wave's share of the Gram matrix: blocks GA/GB[H] over the 16-row blocks
+// g0, g0+4, ...  A and B operand have the same layout (lane: column lane%16,
+// row lane/16 of a step); any order of the rows gives the same sum, so a lane
+// takes rows 4 (lane/16) .. +3 of the block in its four steps and loads 32
+// contiguous bytes.
+template <int H>
+__device__ inline void gram(const double *WI, const double *WJ, int ld,
+        int nrb, int g0, int lane, double4_t (&g)[5])
 {
-    const double d = be-al, h = 2.0*ga;
-    const double big = fmax(fabs(d), fabs(h));
-    if(big >= 1e-140 && big < 1e140)
+    constexpr int NC = H == 0 ? 3 : 4;      // column groups it needs
+    const int lc = lane & 15, lr = lane >> 4;
+    for(int rb = g0; rb < nrb; rb += 4)
     {
-        const double ir = rsqrt(fma(d, d, h*h));
-        const double q = fma(0.5*fabs(d), ir, 0.5);
-        const double y = rsqrt(q);
-        c = q*y;
-        s = (d >= 0.0 ? 0.5 : -0.5)*h*ir*y;
+        double f[NC][4];
+#pragma unroll
+        for(int c = 0; c < NC; c++)
+        {
+            const double *src = (c < 2 ? WI : WJ)+
+                (int64_t)((c & 1)*16+lc)*ld+rb*16+4*lr;
+#pragma unroll
+            for(int v = 0; v < 4; v++)
+                f[c][v] = src[v];
+        }
+#pragma unroll
+        for(int v = 0; v < 4; v++)
+#pragma unroll
+            for(int t = 0; t < 5; t++)
+                g[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(f[GA[H][t]][v],
+                        f[GB[H][t]][v], g[t], 0, 0, 0);
     }
-    else
-        jacobi_rotation(al, be, ga, c, s);
 }
 
-// Exponent of the scale of W and the start of a tile's Jacobi state.
+// Largest entry of R2, kept in td.off2 until the first sweep is over, as the
+// bit pattern of a non-negative double (they order like integers); one
+// workgroup per 8 columns.
 __global__ __launch_bounds__(256) void jb_max_kernel(TileDesc *tiles,
-        const double *ws, int lds_p)
+        const int *list, const double *ws)
 {
-    TileDesc &td = tiles[blockIdx.x];
+    TileDesc &td = tiles[list[blockIdx.y]];
     const int p = td.p, k = td.k;
-    if(p <= lds_p)
-        return;
-    __shared__ double part[4];
     const double *R2 = ws+td.r_off;
     double v = 0.0;
     // R2 is upper triangular up to rounding, but every entry is taken
-    for(int c = threadIdx.x >> 6; c < p; c += 4)
+    const int c1 = min(p, (int)blockIdx.x*8+8);
+    for(int c = blockIdx.x*8+(threadIdx.x >> 6); c < c1; c += 4)
         for(int i = threadIdx.x & 63; i < p; i += 64)
             v = fmax(v, fabs(R2[(int64_t)c*k+i]));
     for(int o = 32; o > 0; o >>= 1)
         v = fmax(v, __shfl_xor(v, o, 64));
     if((threadIdx.x & 63) == 0)
-        part[threadIdx.x >> 6] = v;
-    __syncthreads();
-    if(threadIdx.x == 0)
-    {
-        const double wm = fmax(fmax(part[0], part[1]), fmax(part[2],
-                    part[3]));
-        int e = 0;
-        if(wm > 0.0 && wm < INFINITY)
-            frexp(wm, &e);
-        td.wexp = e;
-        td.jrot = 0;
-        td.jdone = 0;
-        td.sweeps = 0;
-        td.off2 = 0.0;
-    }
+        atomicMax((unsigned long long *)&td.off2,
+                (unsigned long long)__double_as_longlong(v));
+}
+
+// Exponent of the scale of W.
+__device__ inline int scale_exponent(const TileDesc &td)
+{
+    const double wm = td.off2;
+    int e = 0;
+    if(wm > 0.0 && wm < INFINITY)
+        frexp(wm, &e);
+    return e;
+}
+
+// The start of the tiles' Jacobi state.
+__global__ __launch_bounds__(256) void jb_state_kernel(TileDesc *tiles,
+        const int *list, int count)
+{
+    const int t = blockIdx.x*256+threadIdx.x;
+    if(t >= count)
+        return;
+    TileDesc &td = tiles[list[t]];
+    td.jrot = 0;
+    td.jdone = 0;
+    td.sweeps = 0;
+    td.off2 = 0.0;
 }
 
 // W = R2^T 2^-wexp (the power of two that brings the largest entry into
 // [1/2, 1), exact), rows padded to 16 and columns to 64 with zeros: zero
 // columns never rotate.  One 32 x 32 patch per workgroup, transposed in
 // LDS.
-__global__ __launch_bounds__(256) void jb_init_kernel(const TileDesc *tiles,
-        double *ws, int lds_p)
+__global__ __launch_bounds__(256) void jb_init_kernel(TileDesc *tiles,
+        const int *list, double *ws)
 {
-    const TileDesc &td = tiles[blockIdx.y];
+    TileDesc &td = tiles[list[blockIdx.y]];
     const int p = td.p, k = td.k;
-    if(p <= lds_p)
-        return;
     const int ld = ld_of(p), nc = blocks_of(p)*BW;
     const int pr = (ld+31)/32;
     const int bi = blockIdx.x % pr, bj = blockIdx.x / pr;
@@ -129,7 +156,10 @@ __global__ __launch_bounds__(256) void jb_init_kernel(const TileDesc *tiles,
         return;
     const double *R2 = ws+td.r_off;
     double *W = ws+td.j_off;
-    const double scale = ldexp(1.0, -td.wexp);
+    const int wexp = scale_exponent(td);
+    const double scale = ldexp(1.0, -wexp);
+    if(blockIdx.x == 0 && threadIdx.x == 0)
+        td.wexp = wexp;
     __shared__ double patch[32][33];
     const int x = threadIdx.x & 31, y = threadIdx.x >> 5;
     // W(i, j) = R2(j, i): column i of R2 is read along j
@@ -147,17 +177,28 @@ __global__ __launch_bounds__(256) void jb_init_kernel(const TileDesc *tiles,
     }
 }
 
-// One round of a sweep: workgroup (x, tile) handles pair x of the circle
-// method on the tile's column blocks.
-__global__ __launch_bounds__(NT, 2) void jb_round_kernel(TileDesc *tiles,
-        double *ws, int lds_p, int round)
+// Column at position x of the circle method at a step (position 0 is fixed).
+__device__ inline int column_of(int x, int step)
+{
+    int c = x+step;
+    c = c > PW-1 ? c-(PW-1) : c;
+    return x == 0 ? 0 : c;
+}
+
+// One round of a sweep: workgroup (x, y) handles pair x of the circle method
+// on the column blocks of tile list[y].
+__global__ __launch_bounds__(NT, 4) void jb_round_kernel(TileDesc *tiles,
+        const int *list, double *ws, int round)
 {
     __shared__ double G[PW*PW];
     __shared__ double J[PW*PW];
+    __shared__ double2 cs[NT/64][BW];
     __shared__ int perm[PW];
-    TileDesc &td = tiles[blockIdx.y];
+    if(list[blockIdx.y] < 0)
+        return;
+    TileDesc &td = tiles[list[blockIdx.y]];
     const int p = td.p;
-    if(p <= lds_p || td.jdone)
+    if(td.jdone)
         return;
     const int nbe = blocks_of(p);
     const int x = blockIdx.x, y = nbe-1-x;
@@ -172,85 +213,65 @@ __global__ __launch_bounds__(NT, 2) void jb_round_kernel(TileDesc *tiles,
     const int lc = lane & 15, lr = lane >> 4;
     const int nrb = ld/16;
 
-    // ---- 1. G = [WI WJ]^T [WI WJ], rows split over the waves in blocks of
-    // 16.  A and B operand have the same layout (lane: column lane%16, row
-    // lane/16 of a step); any order of the rows gives the same sum, so a
-    // lane takes rows 4 (lane/16) .. +3 of the block in its four steps and
-    // loads 32 contiguous bytes.
-    double4_t g[10];
+    // ---- 1. G = [WI WJ]^T [WI WJ]: four shares of the rows, two of the
+    // blocks
+    const int share = wave & 3, hw = wave >> 2;
+    double4_t g[5];
 #pragma unroll
-    for(int t = 0; t < 10; t++)
+    for(int t = 0; t < 5; t++)
         g[t] = double4_t{0.0, 0.0, 0.0, 0.0};
-    for(int rb = wave; rb < nrb; rb += 4)
-    {
-        double f[4][4];
-#pragma unroll
-        for(int c = 0; c < 4; c++)
-        {
-            const double *src = (c < 2 ? WI : WJ)+
-                (int64_t)((c & 1)*16+lc)*ld+rb*16+4*lr;
-#pragma unroll
-            for(int v = 0; v < 4; v++)
-                f[c][v] = src[v];
-        }
-#pragma unroll
-        for(int v = 0; v < 4; v++)
-        {
-            int t = 0;
-#pragma unroll
-            for(int a = 0; a < 4; a++)
-#pragma unroll
-                for(int b = a; b < 4; b++, t++)
-                    g[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(f[a][v],
-                            f[b][v], g[t], 0, 0, 0);
-        }
-    }
-    // sum over the waves in a fixed order: (0 + 2) + (1 + 3), through G and
+    if(hw == 0)
+        gram<0>(WI, WJ, ld, nrb, share, lane, g);
+    else
+        gram<1>(WI, WJ, ld, nrb, share, lane, g);
+    // sum over the shares in a fixed order: (0 + 2) + (1 + 3), through G and
     // J as scratch
     auto put = [&](double *dst) {
 #pragma unroll
-        for(int t = 0; t < 10; t++)
+        for(int t = 0; t < 5; t++)
 #pragma unroll
             for(int v = 0; v < 4; v++)
                 dst[(t*4+v)*64+lane] = g[t][v];
     };
     auto add = [&](const double *src) {
 #pragma unroll
-        for(int t = 0; t < 10; t++)
+        for(int t = 0; t < 5; t++)
 #pragma unroll
             for(int v = 0; v < 4; v++)
                 g[t][v] += src[(t*4+v)*64+lane];
     };
-    if(wave == 2)
-        put(G);
-    if(wave == 3)
-        put(J);
+    double *sg = G+hw*1280, *sj = J+hw*1280;
+    if(share == 2)
+        put(sg);
+    if(share == 3)
+        put(sj);
     __syncthreads();
-    if(wave == 0)
-        add(G);
-    if(wave == 1)
+    if(share == 0)
+        add(sg);
+    if(share == 1)
     {
-        add(J);
-        put(J);
+        add(sj);
+        put(sj);
     }
     __syncthreads();
-    if(wave == 0)
+    if(share == 0)
     {
-        add(J);
-        int t = 0;
+        add(sj);
 #pragma unroll
-        for(int a = 0; a < 4; a++)
+        for(int t = 0; t < 5; t++)
+        {
+            const int a = hw == 0 ? GA[0][t] : GA[1][t];
+            const int b = hw == 0 ? GB[0][t] : GB[1][t];
 #pragma unroll
-            for(int b = a; b < 4; b++, t++)
-#pragma unroll
-                for(int v = 0; v < 4; v++)
-                {
-                    // D layout: row lane/16 + 4 v, column lane%16
-                    const int i = a*16+lr+4*v, j = b*16+lc;
-                    G[i*PW+j] = g[t][v];
-                    if(b > a)
-                        G[j*PW+i] = g[t][v];
-                }
+            for(int v = 0; v < 4; v++)
+            {
+                // D layout: row lane/16 + 4 v, column lane%16
+                const int i = a*16+lr+4*v, j = b*16+lc;
+                G[i*PW+j] = g[t][v];
+                if(b > a)
+                    G[j*PW+i] = g[t][v];
+            }
+        }
     }
     __syncthreads();
     for(int e = threadIdx.x; e < PW*PW; e += NT)
@@ -264,22 +285,34 @@ __global__ __launch_bounds__(NT, 2) void jb_round_kernel(TileDesc *tiles,
     // the next rotations.
     const double ctol = (double)p*DBL_EPSILON;
     const int pj = lane & 31, half = lane >> 5;
+    __syncthreads();
+    // most visits of the last sweeps have nothing to rotate: all pairs are
+    // tested at once first
+    {
+        bool any = false;
+        for(int e = threadIdx.x; e < PW*PW; e += NT)
+        {
+            const int i = e >> 6, j = e & (PW-1);
+            if(i < j)
+                any |= jr_rotates_fast(G[i*(PW+1)], G[j*(PW+1)], G[e], ctol);
+        }
+        if(__syncthreads_or(any) == 0)
+            return;
+    }
     bool rotated = false;
     const int a0 = pj, b0 = PW-1-pj;    // positions of the pair at step 0
     double pc = 1.0, ps = 0.0;          // rotation J has not seen yet
     int pa = 0, pb = 1;
-    __syncthreads();
     for(int step = 0; step < PW-1; step++)
     {
-        const int ca = a0 == 0 ? 0 : 1+(a0-1+step) % (PW-1);
-        const int cb = 1+(b0-1+step) % (PW-1);
+        const int ca = column_of(a0, step), cb = column_of(b0, step);
         const double al = G[ca*PW+ca], be = G[cb*PW+cb];
         const double ga = G[ca*PW+cb];
         // J <- J R of the previous rotating step
 #pragma unroll
-        for(int q = 0; q < 8; q++)
+        for(int q = 0; q < 4; q++)
         {
-            double *row = J+(wave*16+q*2+half)*PW;
+            double *row = J+(wave*8+q*2+half)*PW;
             const double u = row[pa], v = row[pb];
             row[pa] = pc*u-ps*v;
             row[pb] = ps*u+pc*v;
@@ -287,31 +320,31 @@ __global__ __launch_bounds__(NT, 2) void jb_round_kernel(TileDesc *tiles,
         pc = 1.0;
         ps = 0.0;
         double c = 1.0, s = 0.0;
-        const bool rot = jr_rotates(al, be, ga, ctol);
+        const bool rot = jr_rotates_fast(al, be, ga, ctol);
         if(rot)
-            rotation(al, be, ga, c, s);
+            jacobi_rotation_fast(al, be, ga, c, s);
         if(__ballot(rot) == 0)
             continue;               // the same in every wave
         rotated = true;
+        // the rotations of the step for the rows (each wave its own copy)
+        if(half == 0)
+            cs[wave][pj] = double2{c, s};
         // every wave has read its rotations before G changes
         __syncthreads();
         // G <- R^T G R
 #pragma unroll
-        for(int q = 0; q < 4; q++)
+        for(int q = 0; q < 2; q++)
         {
-            const int i = wave*8+q*2+half;      // row pair
-            const int ra = __shfl(ca, i, 64), rb = __shfl(cb, i, 64);
-            const double ci = __shfl(c, i, 64), si = __shfl(s, i, 64);
+            const int i = wave*4+q*2+half;      // row pair
+            const int ra = column_of(i, step), rb = column_of(PW-1-i, step);
+            const double ci = cs[wave][i].x, si = cs[wave][i].y;
             const double gaa = G[ra*PW+ca], gab = G[ra*PW+cb];
             const double gba = G[rb*PW+ca], gbb = G[rb*PW+cb];
             const double xaa = c*gaa-s*gab, xab = s*gaa+c*gab;
             const double xba = c*gba-s*gbb, xbb = s*gba+c*gbb;
-            double yab = ci*xab-si*xbb, yba = si*xaa+ci*xba;
-            if(i == pj && rot)
-                yab = yba = 0.0;
             G[ra*PW+ca] = ci*xaa-si*xba;
-            G[ra*PW+cb] = yab;
-            G[rb*PW+ca] = yba;
+            G[ra*PW+cb] = ci*xab-si*xbb;
+            G[rb*PW+ca] = si*xaa+ci*xba;
             G[rb*PW+cb] = si*xab+ci*xbb;
         }
         pc = c;
@@ -323,9 +356,9 @@ __global__ __launch_bounds__(NT, 2) void jb_round_kernel(TileDesc *tiles,
     if(!rotated)
         return;
 #pragma unroll
-    for(int q = 0; q < 8; q++)
+    for(int q = 0; q < 4; q++)
     {
-        double *row = J+(wave*16+q*2+half)*PW;
+        double *row = J+(wave*8+q*2+half)*PW;
         const double u = row[pa], v = row[pb];
         row[pa] = pc*u-ps*v;
         row[pb] = ps*u+pc*v;
@@ -348,39 +381,47 @@ __global__ __launch_bounds__(NT, 2) void jb_round_kernel(TileDesc *tiles,
     }
     __syncthreads();
 
-    // ---- 3. W_pair <- W_pair J, rows split over the waves in blocks of
-    // 16; each wave reads all columns of its rows before it writes them.
-    // J is held as B operand in registers (16 steps of 4 rows x 4 column
-    // groups).  Logical row i of the block is physical row 4 (i%4) + i/4,
-    // so that the output lane stores 4 consecutive rows.
-    double jb[16][4];
-#pragma unroll
-    for(int q = 0; q < 16; q++)
-#pragma unroll
-        for(int n = 0; n < 4; n++)
-            jb[q][n] = J[(4*q+lr)*PW+perm[16*n+lc]];
+    // ---- 3. W_pair <- W_pair J, rows split over four shares of the waves in
+    // blocks of 16, the columns of J over two: both halves read a block's
+    // rows before either writes its columns.  Logical row i of the block is
+    // physical row 4 (i%4) + i/4, so that the output lane stores 4
+    // consecutive rows.
     const int prow = 4*(lc & 3)+(lc >> 2);
-    for(int rb = wave; rb < nrb; rb += 4)
-    {
-        double4_t acc[4];
+    const double *JB[2];
 #pragma unroll
-        for(int n = 0; n < 4; n++)
-            acc[n] = double4_t{0.0, 0.0, 0.0, 0.0};
-        double a[16];
+    for(int n = 0; n < 2; n++)
+        JB[n] = J+lr*PW+perm[hw*32+16*n+lc];
+    double *WD = hw == 0 ? WI : WJ;
+    double a[16];
+    auto load = [&](int rb) {
 #pragma unroll
         for(int q = 0; q < 16; q++)
             a[q] = (q < 8 ? WI : WJ)[(int64_t)(4*(q & 7)+lr)*ld+rb*16+prow];
+    };
+    if(share < nrb)
+        load(share);
+    for(int r0 = 0; r0 < nrb; r0 += 4)
+    {
+        const int rb = r0+share;
+        __syncthreads();
+        if(rb >= nrb)
+            continue;
+        double4_t acc[2];
+#pragma unroll
+        for(int n = 0; n < 2; n++)
+            acc[n] = double4_t{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
         for(int q = 0; q < 16; q++)
 #pragma unroll
-            for(int n = 0; n < 4; n++)
-                acc[n] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q], jb[q][n],
-                        acc[n], 0, 0, 0);
+            for(int n = 0; n < 2; n++)
+                acc[n] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q],
+                        JB[n][4*q*PW], acc[n], 0, 0, 0);
+        if(rb+4 < nrb)
+            load(rb+4);
 #pragma unroll
-        for(int n = 0; n < 4; n++)
+        for(int n = 0; n < 2; n++)
         {
-            double *dst = (n < 2 ? WI : WJ)+(int64_t)((n & 1)*16+lc)*ld+
-                rb*16+4*lr;
+            double *dst = WD+(int64_t)(n*16+lc)*ld+rb*16+4*lr;
 #pragma unroll
             for(int v = 0; v < 4; v++)
                 dst[v] = acc[n][v];
@@ -390,25 +431,27 @@ __global__ __launch_bounds__(NT, 2) void jb_round_kernel(TileDesc *tiles,
 
 // Whether the tile may end with the verdict "rank above the limit" alone
 // (its singular values are not asked for), and that limit.
-__device__ inline bool rank_limit(const TileDesc &td, int lds_p, int &limit)
+__device__ inline bool rank_limit(const TileDesc &td, int &limit)
 {
     const int mn = td.m < td.n ? td.m : td.n;
     limit = td.maxrank;
     if((td.rule & RSDD_RULE_HALF) && mn/2-1 < limit)
         limit = mn/2-1;
-    return td.nosv && td.p > lds_p && !td.jdone && td.p > limit;
+    return td.nosv && !td.jdone && td.p > limit;
 }
 
 // Squared norms of W's columns (to the tile's S) and the sum of the squares
 // of the Gram matrix's strict upper triangle (td.off2): one workgroup per
 // block pair I <= J.
-__global__ __launch_bounds__(NT) void jb_off_kernel(TileDesc *tiles,
-        double *ws, int lds_p)
+__global__ __launch_bounds__(256) void jb_off_kernel(TileDesc *tiles,
+        const int *list, double *ws)
 {
     __shared__ double part[3][16*64];
-    TileDesc &td = tiles[blockIdx.y];
+    if(list[blockIdx.y] < 0)
+        return;
+    TileDesc &td = tiles[list[blockIdx.y]];
     int limit;
-    if(!rank_limit(td, lds_p, limit))
+    if(!rank_limit(td, limit))
         return;
     const int p = td.p, nb = (p+BW-1)/BW;
     int bi = 0, rest = blockIdx.x;
@@ -479,13 +522,15 @@ __global__ __launch_bounds__(NT) void jb_off_kernel(TileDesc *tiles,
 // the rank rule allows (tol^2 of the total) is asked for, far more than any
 // rounding, so the verdict is the one the converged singular values give.
 __global__ __launch_bounds__(256) void jb_cert_kernel(TileDesc *tiles,
-        const double *ws, int lds_p)
+        const int *list, const double *ws)
 {
     __shared__ double d[1024];
     __shared__ double part[2][4];
-    TileDesc &td = tiles[blockIdx.x];
+    if(list[blockIdx.x] < 0)
+        return;
+    TileDesc &td = tiles[list[blockIdx.x]];
     int limit;
-    if(!rank_limit(td, lds_p, limit))
+    if(!rank_limit(td, limit))
         return;
     const int p = td.p;
     for(int i = threadIdx.x; i < p; i += 256)
@@ -525,80 +570,118 @@ __global__ __launch_bounds__(256) void jb_cert_kernel(TileDesc *tiles,
     }
 }
 
-// End of a sweep: tiles without a rotation are done; *active counts the
-// tiles that are not.
-__global__ __launch_bounds__(256) void jb_sweep_kernel(TileDesc *tiles,
-        int ntiles, int lds_p, int *active)
+// End of a sweep: tiles without a rotation are done; the others stay on the
+// list, in order, followed by -1.  out[0] = their number, out[1] = the largest
+// of their p.
+__global__ __launch_bounds__(1024) void jb_sweep_kernel(TileDesc *tiles,
+        int *list, int count, int *out)
 {
-    int c = 0;
-    for(int t = threadIdx.x; t < ntiles; t += blockDim.x)
+    __shared__ int wcount[16], wmax[16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int base = 0, pmax = 0;
+    for(int c0 = 0; c0 < count; c0 += 1024)
     {
-        TileDesc &td = tiles[t];
-        if(td.p <= lds_p || td.jdone)
-            continue;
-        if(td.jrot == 0)
-            td.jdone = 1;
-        else
+        const int q = c0+threadIdx.x;
+        bool keep = false;
+        int t = 0, p = 0;
+        if(q < count && (t = list[q]) >= 0)
         {
-            td.sweeps++;
-            td.jrot = 0;
-            c++;
+            TileDesc &td = tiles[t];
+            if(!td.jdone)
+            {
+                if(td.jrot == 0)
+                    td.jdone = 1;
+                else
+                {
+                    td.sweeps++;
+                    td.jrot = 0;
+                    td.off2 = 0.0;
+                    keep = true;
+                    p = td.p;
+                }
+            }
         }
+        const unsigned long long m = __ballot(keep);
+        for(int o = 32; o > 0; o >>= 1)
+            p = max(p, __shfl_xor(p, o, 64));
+        if(lane == 0)
+        {
+            wcount[wave] = __popcll(m);
+            wmax[wave] = p;
+        }
+        __syncthreads();
+        int before = base;
+        for(int w = 0; w < 16; w++)
+        {
+            before += w < wave ? wcount[w] : 0;
+            base += wcount[w];
+            pmax = max(pmax, wmax[w]);
+        }
+        // places before q only: an entry read later is never overwritten
+        if(keep)
+            list[before+__popcll(m & ((1ull << lane)-1))] = t;
+        __syncthreads();
     }
-    for(int o = 32; o > 0; o >>= 1)
-        c += __shfl_xor(c, o, 64);
-    __shared__ int part[4];
-    if((threadIdx.x & 63) == 0)
-        part[threadIdx.x >> 6] = c;
-    __syncthreads();
+    for(int q = base+threadIdx.x; q < count; q += 1024)
+        list[q] = -1;
     if(threadIdx.x == 0)
-        *active = part[0]+part[1]+part[2]+part[3];
+    {
+        out[0] = base;
+        out[1] = pmax;
+    }
 }
 
 } // namespace
 
-// Jacobi sweeps on every tile with p > lds_p: W (columns orthogonal on
-// return) in the tile's j_off region, ld = p rounded up to 16, scaled by
-// 2^-wexp, td.jdone 1; tiles that ended early with a rank certainly above
-// the limit have jdone 2, tiles that did not converge 0.  certify: some
-// tile may end that way.  h_active: pinned host int.
-int pipeline_jacobi_block(TileDesc *d_tiles, int ntiles, double *ws,
-        int lds_p, int pmax, int max_sweeps, bool certify, int *d_active,
-        int *h_active, hipStream_t s)
+// Jacobi sweeps on the count tiles of d_list (the tiles with a core beyond
+// LDS; the list is used up): W (columns orthogonal on return) in the tile's
+// j_off region, ld = p rounded up to 16, scaled by 2^-wexp, td.jdone 1; tiles
+// that ended early with a rank certainly above the limit have jdone 2, tiles
+// that did not converge 0.  certify: some tile may end that way.  d_out: two
+// device ints, h_out: two pinned host ints.
+int pipeline_jacobi_block(TileDesc *d_tiles, int *d_list, int count,
+        double *ws, int pmax, int max_sweeps, bool certify, int *d_out,
+        int *h_out, hipStream_t s)
 {
-    const int nb = (pmax+BW-1)/BW, nbe = nb+(nb & 1);
-    const int patches = (pmax+31)/32*nbe;
-    hipLaunchKernelGGL(jb_max_kernel, dim3(ntiles), dim3(256), 0, s, d_tiles,
-            ws, lds_p);
-    hipLaunchKernelGGL(jb_init_kernel, dim3(patches, ntiles), dim3(256), 0,
-            s, d_tiles, ws, lds_p);
+    if(count <= 0)
+        return STARSH_SUCCESS;
+    int nb = (pmax+BW-1)/BW, nbe = nb+(nb & 1);
+    hipLaunchKernelGGL(jb_state_kernel, dim3((count+255)/256), dim3(256), 0,
+            s, d_tiles, d_list, count);
+    hipLaunchKernelGGL(jb_max_kernel, dim3((pmax+7)/8, count), dim3(256), 0,
+            s, d_tiles, d_list, ws);
+    hipLaunchKernelGGL(jb_init_kernel, dim3((pmax+31)/32*nbe, count),
+            dim3(256), 0, s, d_tiles, d_list, ws);
     HIP_TRY(hipGetLastError());
     for(int sweep = 0; sweep < max_sweeps; sweep++)
     {
         for(int round = 0; round < nbe-1; round++)
-            hipLaunchKernelGGL(jb_round_kernel, dim3(nbe/2, ntiles),
-                    dim3(NT), 0, s, d_tiles, ws, lds_p, round);
+            hipLaunchKernelGGL(jb_round_kernel, dim3(nbe/2, count), dim3(NT),
+                    0, s, d_tiles, d_list, ws, round);
         // tiles headed for a rank above the limit: two sweeps are enough for
         // most, the others are tried again
-        if(certify && (sweep == 1 || sweep == 3 || sweep == 6))
+        if(certify && (sweep == 1 || sweep == 2 || sweep == 3 || sweep == 6))
         {
-            hipLaunchKernelGGL(jb_off_kernel, dim3(nb*(nb+1)/2, ntiles),
-                    dim3(NT), 0, s, d_tiles, ws, lds_p);
-            hipLaunchKernelGGL(jb_cert_kernel, dim3(ntiles), dim3(256), 0,
-                    s, d_tiles, ws, lds_p);
+            hipLaunchKernelGGL(jb_off_kernel, dim3(nb*(nb+1)/2, count),
+                    dim3(256), 0, s, d_tiles, d_list, ws);
+            hipLaunchKernelGGL(jb_cert_kernel, dim3(count), dim3(256), 0, s,
+                    d_tiles, d_list, ws);
         }
-        hipLaunchKernelGGL(jb_sweep_kernel, dim3(1), dim3(256), 0, s,
-                d_tiles, ntiles, lds_p, d_active);
+        hipLaunchKernelGGL(jb_sweep_kernel, dim3(1), dim3(1024), 0, s,
+                d_tiles, d_list, count, d_out);
         HIP_TRY(hipGetLastError());
         // no core of this size converges in two sweeps unless it was
         // diagonal from the start
         if(sweep < 1)
             continue;
-        HIP_TRY(hipMemcpyAsync(h_active, d_active, sizeof(int),
+        HIP_TRY(hipMemcpyAsync(h_out, d_out, 2*sizeof(int),
                     hipMemcpyDeviceToHost, s));
         HIP_TRY(hipStreamSynchronize(s));
-        if(*h_active == 0)
+        count = h_out[0];
+        if(count == 0)
             break;
+        nb = (h_out[1]+BW-1)/BW;
+        nbe = nb+(nb & 1);
     }
     return STARSH_SUCCESS;
 }

@@ -117,14 +117,16 @@ inline int64_t core_work_doubles(int p)
 }
 
 // One-sided Jacobi SVD of R2, singular values, rank by the reference rule
-// (each tile's own maxrank and tol) and X_r.  certify: some tile with nosv
-// has p above its rank limit.  d_active: a device int, h_active: a pinned
-// host int.
+// (each tile's own maxrank and tol) and X_r.  d_list: the count tiles with p
+// > CORE_LDS_PMAX (a device array, used up); certify: some tile with nosv has
+// p above its rank limit.  d_out: two device ints, h_out: two pinned host
+// ints.
 int pipeline_core(TileDesc *d_tiles, int ntiles, double *ws, int pmax,
-        bool certify, int *d_active, int *h_active, hipStream_t s);
-int pipeline_jacobi_block(TileDesc *d_tiles, int ntiles, double *ws,
-        int lds_p, int pmax, int max_sweeps, bool certify, int *d_active,
-        int *h_active, hipStream_t s);
+        bool certify, int *d_list, int count, int *d_out, int *h_out,
+        hipStream_t s);
+int pipeline_jacobi_block(TileDesc *d_tiles, int *d_list, int count,
+        double *ws, int pmax, int max_sweeps, bool certify, int *d_out,
+        int *h_out, hipStream_t s);
 
 // Exact engines (exact.hip): sketch Y = A[:, sel] (RSDD_RULE_SELECT tiles,
 // k columns from d_sel at each tile's sel_off), and the first piv_k column

@@ -77,7 +77,8 @@ struct Pool
 Pool ws_pool, uv_pool, pack_pool, stage_pool{nullptr, 0, true};
 // The small per-batch buffers (tile descriptors, kept-column flags, norms,
 // int8 Omega and digit planes, counters, R2 partials, selected columns,
-// pivots, Gram-Schmidt coefficients), kept too: a hipMalloc / hipFree pair per buffer and batch cost
+// pivots, Gram-Schmidt coefficients, tile lists), kept too: a hipMalloc /
+// hipFree pair per buffer and batch cost
 // host time on every call, and hipFree waits for the device.
 constexpr size_t SMALL_UNIT = (size_t)1 << 20;
 Pool tiles_pool{nullptr, 0, false, SMALL_UNIT},
@@ -89,7 +90,8 @@ Pool tiles_pool{nullptr, 0, false, SMALL_UNIT},
      part_pool{nullptr, 0, false, SMALL_UNIT},
      sel_pool{nullptr, 0, false, SMALL_UNIT},
      piv_pool{nullptr, 0, false, SMALL_UNIT},
-     coef_pool{nullptr, 0, false, SMALL_UNIT};
+     coef_pool{nullptr, 0, false, SMALL_UNIT},
+     list_pool{nullptr, 0, false, SMALL_UNIT};
 
 // Host view of the device counter of tiles still in a BCGS2 run.  The
 // counter is copied to pinned memory after every block of columns; the host
@@ -487,7 +489,8 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
     // part: split-K partials of R2, kept until the batch has synchronised
     Pool &tiles = tiles_pool, &keep = keep_pool, &norms = norms_pool,
          &om8 = om8_pool, &active = active_pool, &qd = qd_pool,
-         &part = part_pool, &coef = coef_pool, &selbuf = sel_pool, &pivbuf = piv_pool;
+         &part = part_pool, &coef = coef_pool,
+         &list = list_pool, &selbuf = sel_pool, &pivbuf = piv_pool;
     if(nsel > 0)
     {
         TRY(selbuf.reserve(sizeof(int)*(size_t)nsel));
@@ -510,7 +513,7 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
     TRY(norms.reserve(sizeof(double)*(size_t)nt*kmax));
     TRY(coef.reserve(sizeof(double)*(size_t)nt*kmax*GS_BLOCK));
     TRY(uv_pool.reserve(sizeof(double)*(uvoff > 0 ? uvoff : 1)));
-    TRY(active.reserve(sizeof(int)));
+    TRY(active.reserve(2*sizeof(int)));
     TileDesc *d_tiles = (TileDesc *)tiles.p;
     double *d_ws = (double *)ws_pool.p;
     HIP_TRY(hipMemcpyAsync(d_tiles, h.data(), sizeof(TileDesc)*nt,
@@ -691,8 +694,19 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
     }
     // 6. core SVD and rank
     TRY(probe.init());
-    TRY(pipeline_core(d_tiles, nt, d_ws, pmax, certify, (int *)active.p,
-                probe.h, s));
+    // (largest cores first, so that the last workgroups of a launch are short)
+    std::vector<int> large;
+    for(int t = 0; t < nt; t++)
+        if(h[t].p > CORE_LDS_PMAX)
+            large.push_back(t);
+    std::stable_sort(large.begin(), large.end(), [&](int a, int b) {
+        return h[a].p > h[b].p; });
+    TRY(list.reserve(sizeof(int)*(large.size()+1)));
+    if(!large.empty())
+        HIP_TRY(hipMemcpyAsync(list.p, large.data(), sizeof(int)*large.size(),
+                    hipMemcpyHostToDevice, s));
+    TRY(pipeline_core(d_tiles, nt, d_ws, pmax, certify, (int *)list.p,
+                (int)large.size(), (int *)active.p, probe.h, s));
     HIP_TRY(hipMemcpyAsync(h.data(), d_tiles, sizeof(TileDesc)*nt,
                 hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
@@ -755,7 +769,8 @@ void rsdd_release_pools(void)
     pack_pool.release();
     stage_pool.release();
     for(Pool *q : {&tiles_pool, &keep_pool, &norms_pool, &om8_pool,
-                &active_pool, &qd_pool, &part_pool, &sel_pool, &piv_pool, &coef_pool})
+                &active_pool, &qd_pool, &part_pool, &sel_pool, &piv_pool,
+                &coef_pool, &list_pool})
         q->release();
     for(PanelGraph &pg : panel_graphs)
         pg.reset();
