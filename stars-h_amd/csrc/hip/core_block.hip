@@ -2,12 +2,12 @@
 // CORE_LDS_PMAX, core.hip): one-sided block Jacobi with the work of every
 // tile spread over the chip.
 //
-// The columns of W = R2^T are split into blocks of 32.  A sweep visits every
+// The columns of W = R2^T are split into blocks of 16.  A sweep visits every
 // pair of blocks once, in rounds of disjoint pairs (circle method), one
 // launch per round and one workgroup per block pair and tile:
-//   1. Gram matrix G (64 x 64) of the pair's columns on FP64 MFMA;
-//   2. one sweep of two-sided Jacobi on G in LDS, all 32 disjoint column
-//      pairs of a step at once, the rotations accumulated in J (64 x 64);
+//   1. Gram matrix G (32 x 32) of the pair's columns on FP64 MFMA;
+//   2. one sweep of two-sided Jacobi on G in LDS, all 16 disjoint column
+//      pairs of a step at once, the rotations accumulated in J (32 x 32);
 //   3. W_pair <- W_pair J on FP64 MFMA (skipped when nothing rotated).
 // The rotations and the test |g_ij| > p eps |w_i| |w_j| are those of the
 // scalar one-sided method; G is formed afresh from the columns at every
@@ -19,19 +19,20 @@
 // What bounds it: a workgroup per tile (the scalar method with column
 // blocks in LDS, one rotation per half-wave) left the chip idle below 256
 // tiles and paid LDS traffic of O(p) per rotation; here a rotation costs
-// O(64) LDS traffic and the O(p) work is MFMA.  The inner Jacobi is bound by
-// LDS bandwidth (128 KB per step of 32 rotations).  Blocks of 32 keep G and
-// J (65 KB) at two workgroups per CU; the whole 63-step sweep over the 64
-// columns converges in 6 outer sweeps where 32 cross steps per visit need
-// 7-8 (numpy model on sin(kr)/r, exp and Matern cores).
+// O(32) LDS traffic and the O(p) work is MFMA.  A visit is a chain of 31
+// steps, each a rotation and two passes through LDS; with 32-column blocks
+// (63 steps on 64 x 64 matrices, half the rounds) a round took 118 us instead
+// of 35 at p = 150, 130 instead of 44 at 400, 178 instead of 76 at 1000 (four
+// waves), and Matern with 500-row cores was 7% slower as well.  The whole
+// 31-step sweep over both blocks' columns converges in about 6 outer sweeps
+// where the 16 cross steps alone need 7-8 (numpy model on sin(kr)/r, exp and
+// Matern cores).
 // Measured on MI355X, all launches of one compression, against one
 // workgroup per tile: 2D exp N=9973, tile 1000, SVD engine (10 cores of
-// 1000, 45 of 200-500) 1570 -> 23 ms; sin(kr)/r N=25000, tile 1536 (17 of
-// 400, 85 of 130-210) 163 -> 7.8 ms; 3D Matern N=65536, tile 2048, mixed
-// (up to 528) 191 -> 65 ms.  A round of a few hundred pairs takes 115-130 us,
-// about 95 of them the 63 steps, with nothing to rotate 13-19 us.  Only
-// tiles still rotating are launched, by a list the sweeps shorten: empty
-// workgroups of 68 KB of LDS queued for their turn (Matern 82 -> 69 ms).
+// 1000, 45 of 200-500) 1570 -> 22.5 ms; sin(kr)/r N=25000, tile 1536 (17 of
+// 400, 85 of 130-210) 163 -> 6.4 ms; 3D Matern N=65536, tile 2048, mixed
+// (up to 528) 191 -> 52 ms.  Only tiles still rotating are launched, by a
+// list the sweeps shorten.
 #include <float.h>
 #include <math.h>
 #include "pipeline.h"
@@ -41,9 +42,10 @@ typedef double double4_t __attribute__((ext_vector_type(4)));
 
 namespace {
 
-constexpr int BW = 32;          // columns per block
+constexpr int BW = 16;          // columns per block
 constexpr int PW = 2*BW;        // columns per block pair
-constexpr int NT = 512;         // of a round: 8 waves
+constexpr int NT = 256;         // threads of a round: 4 waves
+constexpr int OB = 32;          // columns per block of jb_off_kernel
 
 __device__ inline int ld_of(int p)
 {
@@ -51,47 +53,10 @@ __device__ inline int ld_of(int p)
 }
 
 // Number of column blocks, rounded up to even (the last may be empty).
-__device__ inline int blocks_of(int p)
+__host__ __device__ inline int blocks_of(int p)
 {
     const int nb = (p+BW-1)/BW;
     return nb+(nb & 1);
-}
-
-// The 10 16 x 16 blocks of the upper triangle of G, five for each half of
-// the waves.
-constexpr int GA[2][5] = {{0, 0, 1, 0, 1}, {0, 1, 2, 3, 2}};
-constexpr int GB[2][5] = {{0, 1, 1, 2, 2}, {3, 3, 3, 3, 2}};
-
-// One wave's share of the Gram matrix: blocks GA/GB[H] over the 16-row blocks
-// g0, g0+4, ...  A and B operand have the same layout (lane: column lane%16,
-// row lane/16 of a step); any order of the rows gives the same sum, so a lane
-// takes rows 4 (lane/16) .. +3 of the block in its four steps and loads 32
-// contiguous bytes.
-template <int H>
-__device__ inline void gram(const double *WI, const double *WJ, int ld,
-        int nrb, int g0, int lane, double4_t (&g)[5])
-{
-    constexpr int NC = H == 0 ? 3 : 4;      // column groups it needs
-    const int lc = lane & 15, lr = lane >> 4;
-    for(int rb = g0; rb < nrb; rb += 4)
-    {
-        double f[NC][4];
-#pragma unroll
-        for(int c = 0; c < NC; c++)
-        {
-            const double *src = (c < 2 ? WI : WJ)+
-                (int64_t)((c & 1)*16+lc)*ld+rb*16+4*lr;
-#pragma unroll
-            for(int v = 0; v < 4; v++)
-                f[c][v] = src[v];
-        }
-#pragma unroll
-        for(int v = 0; v < 4; v++)
-#pragma unroll
-            for(int t = 0; t < 5; t++)
-                g[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(f[GA[H][t]][v],
-                        f[GB[H][t]][v], g[t], 0, 0, 0);
-    }
 }
 
 // Largest entry of R2, kept in td.off2 until the first sweep is over, as the
@@ -149,7 +114,7 @@ __global__ __launch_bounds__(256) void jb_init_kernel(TileDesc *tiles,
 {
     TileDesc &td = tiles[list[blockIdx.y]];
     const int p = td.p, k = td.k;
-    const int ld = ld_of(p), nc = blocks_of(p)*BW;
+    const int ld = ld_of(p), nc = (p+63)/64*64;
     const int pr = (ld+31)/32;
     const int bi = blockIdx.x % pr, bj = blockIdx.x / pr;
     if(bj*32 >= nc)
@@ -187,11 +152,12 @@ __device__ inline int column_of(int x, int step)
 
 // One round of a sweep: workgroup (x, y) handles pair x of the circle method
 // on the column blocks of tile list[y].
-__global__ __launch_bounds__(NT, 4) void jb_round_kernel(TileDesc *tiles,
+__global__ __launch_bounds__(NT) void jb_round_kernel(TileDesc *tiles,
         const int *list, double *ws, int round)
 {
     __shared__ double G[PW*PW];
     __shared__ double J[PW*PW];
+    __shared__ double part[2][3*256];
     __shared__ double2 cs[NT/64][BW];
     __shared__ int perm[PW];
     if(list[blockIdx.y] < 0)
@@ -213,110 +179,115 @@ __global__ __launch_bounds__(NT, 4) void jb_round_kernel(TileDesc *tiles,
     const int lc = lane & 15, lr = lane >> 4;
     const int nrb = ld/16;
 
-    // ---- 1. G = [WI WJ]^T [WI WJ]: four shares of the rows, two of the
-    // blocks
-    const int share = wave & 3, hw = wave >> 2;
-    double4_t g[5];
-#pragma unroll
-    for(int t = 0; t < 5; t++)
-        g[t] = double4_t{0.0, 0.0, 0.0, 0.0};
-    if(hw == 0)
-        gram<0>(WI, WJ, ld, nrb, share, lane, g);
-    else
-        gram<1>(WI, WJ, ld, nrb, share, lane, g);
-    // sum over the shares in a fixed order: (0 + 2) + (1 + 3), through G and
-    // J as scratch
-    auto put = [&](double *dst) {
-#pragma unroll
-        for(int t = 0; t < 5; t++)
-#pragma unroll
-            for(int v = 0; v < 4; v++)
-                dst[(t*4+v)*64+lane] = g[t][v];
-    };
-    auto add = [&](const double *src) {
-#pragma unroll
-        for(int t = 0; t < 5; t++)
-#pragma unroll
-            for(int v = 0; v < 4; v++)
-                g[t][v] += src[(t*4+v)*64+lane];
-    };
-    double *sg = G+hw*1280, *sj = J+hw*1280;
-    if(share == 2)
-        put(sg);
-    if(share == 3)
-        put(sj);
-    __syncthreads();
-    if(share == 0)
-        add(sg);
-    if(share == 1)
+    // ---- 1. G = [WI WJ]^T [WI WJ], rows split over the waves in blocks of
+    // 16.  A and B operand have the same layout (lane: column lane%16, row
+    // lane/16 of a step); any order of the rows gives the same sum, so a
+    // lane takes rows 4 (lane/16) .. +3 of the block in its four steps and
+    // loads 32 contiguous bytes.
+    double4_t gii = {0.0, 0.0, 0.0, 0.0}, gij = gii, gjj = gii;
+    for(int r0 = wave; r0 < nrb; r0 += 4)
     {
-        add(sj);
-        put(sj);
-    }
-    __syncthreads();
-    if(share == 0)
-    {
-        add(sj);
+        const int64_t o = (int64_t)lc*ld+r0*16+4*lr;
+        double fi[4], fj[4];
 #pragma unroll
-        for(int t = 0; t < 5; t++)
+        for(int v = 0; v < 4; v++)
         {
-            const int a = hw == 0 ? GA[0][t] : GA[1][t];
-            const int b = hw == 0 ? GB[0][t] : GB[1][t];
+            fi[v] = WI[o+v];
+            fj[v] = WJ[o+v];
+        }
+#pragma unroll
+        for(int v = 0; v < 4; v++)
+        {
+            gii = __builtin_amdgcn_mfma_f64_16x16x4f64(fi[v], fi[v], gii,
+                    0, 0, 0);
+            gij = __builtin_amdgcn_mfma_f64_16x16x4f64(fi[v], fj[v], gij,
+                    0, 0, 0);
+            gjj = __builtin_amdgcn_mfma_f64_16x16x4f64(fj[v], fj[v], gjj,
+                    0, 0, 0);
+        }
+    }
+    // sum over the waves in a fixed order, halving their number
+#pragma unroll
+    for(int h = 2; h > 0; h >>= 1)
+    {
+        if(wave >= h && wave < 2*h)
 #pragma unroll
             for(int v = 0; v < 4; v++)
             {
-                // D layout: row lane/16 + 4 v, column lane%16
-                const int i = a*16+lr+4*v, j = b*16+lc;
-                G[i*PW+j] = g[t][v];
-                if(b > a)
-                    G[j*PW+i] = g[t][v];
+                part[wave-h][v*64+lane] = gii[v];
+                part[wave-h][256+v*64+lane] = gij[v];
+                part[wave-h][512+v*64+lane] = gjj[v];
             }
+        __syncthreads();
+        if(wave < h)
+#pragma unroll
+            for(int v = 0; v < 4; v++)
+            {
+                gii[v] += part[wave][v*64+lane];
+                gij[v] += part[wave][256+v*64+lane];
+                gjj[v] += part[wave][512+v*64+lane];
+            }
+        __syncthreads();
+    }
+    if(wave == 0)
+    {
+        // D layout: row lane/16 + 4 v, column lane%16
+#pragma unroll
+        for(int v = 0; v < 4; v++)
+        {
+            const int i = lr+4*v;
+            G[i*PW+lc] = gii[v];
+            G[i*PW+16+lc] = gij[v];
+            G[(16+lc)*PW+i] = gij[v];
+            G[(16+i)*PW+16+lc] = gjj[v];
         }
     }
-    __syncthreads();
     for(int e = threadIdx.x; e < PW*PW; e += NT)
-        J[e] = (e & (PW-1)) == (e >> 6) ? 1.0 : 0.0;
-
-    // ---- 2. one sweep of Jacobi on G.  Lane l of every wave computes the
-    // rotation of column pair l%32 of the step (so the step needs no
-    // exchange of rotations between waves); the 2 x 2 blocks (row pair i,
-    // column pair j = l%32) and the rows of J are split over the waves.  J
-    // is one step behind, so that its LDS traffic overlaps the latency of
-    // the next rotations.
-    const double ctol = (double)p*DBL_EPSILON;
-    const int pj = lane & 31, half = lane >> 5;
+        J[e] = e % PW == e/PW ? 1.0 : 0.0;
     __syncthreads();
+
     // most visits of the last sweeps have nothing to rotate: all pairs are
     // tested at once first
+    const double ctol = (double)p*DBL_EPSILON;
     {
         bool any = false;
         for(int e = threadIdx.x; e < PW*PW; e += NT)
         {
-            const int i = e >> 6, j = e & (PW-1);
+            const int i = e/PW, j = e % PW;
             if(i < j)
                 any |= jr_rotates_fast(G[i*(PW+1)], G[j*(PW+1)], G[e], ctol);
         }
         if(__syncthreads_or(any) == 0)
             return;
     }
+
+    // ---- 2. one sweep of Jacobi on G.  Lane l of every wave computes the
+    // rotation of column pair l%16 of the step (so the step needs no
+    // exchange of rotations between waves); the 16 lane groups of the
+    // workgroup take a row pair of G (2 x 2 blocks with column pair l%16) and
+    // two rows of J.  J is one step behind, so that its LDS traffic overlaps
+    // the latency of the next rotations.
+    const int pj = lane & 15;
+    const int slot = wave*4+lr;
     bool rotated = false;
-    const int a0 = pj, b0 = PW-1-pj;    // positions of the pair at step 0
     double pc = 1.0, ps = 0.0;          // rotation J has not seen yet
     int pa = 0, pb = 1;
-    for(int step = 0; step < PW-1; step++)
-    {
-        const int ca = column_of(a0, step), cb = column_of(b0, step);
-        const double al = G[ca*PW+ca], be = G[cb*PW+cb];
-        const double ga = G[ca*PW+cb];
-        // J <- J R of the previous rotating step
+    auto rotate_j = [&]() {
 #pragma unroll
-        for(int q = 0; q < 4; q++)
+        for(int q = 0; q < 2; q++)
         {
-            double *row = J+(wave*8+q*2+half)*PW;
+            double *row = J+(q*16+slot)*PW;
             const double u = row[pa], v = row[pb];
             row[pa] = pc*u-ps*v;
             row[pb] = ps*u+pc*v;
         }
+    };
+    for(int step = 0; step < PW-1; step++)
+    {
+        const int ca = column_of(pj, step), cb = column_of(PW-1-pj, step);
+        const double al = G[ca*PW+ca], be = G[cb*PW+cb];
+        const double ga = G[ca*PW+cb];
+        rotate_j();
         pc = 1.0;
         ps = 0.0;
         double c = 1.0, s = 0.0;
@@ -327,26 +298,22 @@ __global__ __launch_bounds__(NT, 4) void jb_round_kernel(TileDesc *tiles,
             continue;               // the same in every wave
         rotated = true;
         // the rotations of the step for the rows (each wave its own copy)
-        if(half == 0)
+        if(lane < BW)
             cs[wave][pj] = double2{c, s};
         // every wave has read its rotations before G changes
         __syncthreads();
         // G <- R^T G R
-#pragma unroll
-        for(int q = 0; q < 2; q++)
-        {
-            const int i = wave*4+q*2+half;      // row pair
-            const int ra = column_of(i, step), rb = column_of(PW-1-i, step);
-            const double ci = cs[wave][i].x, si = cs[wave][i].y;
-            const double gaa = G[ra*PW+ca], gab = G[ra*PW+cb];
-            const double gba = G[rb*PW+ca], gbb = G[rb*PW+cb];
-            const double xaa = c*gaa-s*gab, xab = s*gaa+c*gab;
-            const double xba = c*gba-s*gbb, xbb = s*gba+c*gbb;
-            G[ra*PW+ca] = ci*xaa-si*xba;
-            G[ra*PW+cb] = ci*xab-si*xbb;
-            G[rb*PW+ca] = si*xaa+ci*xba;
-            G[rb*PW+cb] = si*xab+ci*xbb;
-        }
+        const int ra = column_of(slot, step);
+        const int rb = column_of(PW-1-slot, step);
+        const double ci = cs[wave][slot].x, si = cs[wave][slot].y;
+        const double gaa = G[ra*PW+ca], gab = G[ra*PW+cb];
+        const double gba = G[rb*PW+ca], gbb = G[rb*PW+cb];
+        const double xaa = c*gaa-s*gab, xab = s*gaa+c*gab;
+        const double xba = c*gba-s*gbb, xbb = s*gba+c*gbb;
+        G[ra*PW+ca] = ci*xaa-si*xba;
+        G[ra*PW+cb] = ci*xab-si*xbb;
+        G[rb*PW+ca] = si*xaa+ci*xba;
+        G[rb*PW+cb] = si*xab+ci*xbb;
         pc = c;
         ps = s;
         pa = ca;
@@ -355,14 +322,7 @@ __global__ __launch_bounds__(NT, 4) void jb_round_kernel(TileDesc *tiles,
     }
     if(!rotated)
         return;
-#pragma unroll
-    for(int q = 0; q < 4; q++)
-    {
-        double *row = J+(wave*8+q*2+half)*PW;
-        const double u = row[pa], v = row[pb];
-        row[pa] = pc*u-ps*v;
-        row[pb] = ps*u+pc*v;
-    }
+    rotate_j();
     if(threadIdx.x == 0)
         atomicAdd(&td.jrot, 1);
     // the columns leave sorted by norm, the larger ones to the first block:
@@ -381,47 +341,37 @@ __global__ __launch_bounds__(NT, 4) void jb_round_kernel(TileDesc *tiles,
     }
     __syncthreads();
 
-    // ---- 3. W_pair <- W_pair J, rows split over four shares of the waves in
-    // blocks of 16, the columns of J over two: both halves read a block's
-    // rows before either writes its columns.  Logical row i of the block is
-    // physical row 4 (i%4) + i/4, so that the output lane stores 4
-    // consecutive rows.
+    // ---- 3. W_pair <- W_pair J, rows split over the waves in blocks of 16;
+    // a wave reads a block's rows before it writes them.  Logical row i of
+    // the block is physical row 4 (i%4) + i/4, so that the output lane stores
+    // 4 consecutive rows.
+    double jb[8][2];
+#pragma unroll
+    for(int q = 0; q < 8; q++)
+#pragma unroll
+        for(int n = 0; n < 2; n++)
+            jb[q][n] = J[(4*q+lr)*PW+perm[16*n+lc]];
     const int prow = 4*(lc & 3)+(lc >> 2);
-    const double *JB[2];
-#pragma unroll
-    for(int n = 0; n < 2; n++)
-        JB[n] = J+lr*PW+perm[hw*32+16*n+lc];
-    double *WD = hw == 0 ? WI : WJ;
-    double a[16];
-    auto load = [&](int rb) {
-#pragma unroll
-        for(int q = 0; q < 16; q++)
-            a[q] = (q < 8 ? WI : WJ)[(int64_t)(4*(q & 7)+lr)*ld+rb*16+prow];
-    };
-    if(share < nrb)
-        load(share);
-    for(int r0 = 0; r0 < nrb; r0 += 4)
+    for(int r0 = wave; r0 < nrb; r0 += 4)
     {
-        const int rb = r0+share;
-        __syncthreads();
-        if(rb >= nrb)
-            continue;
+        double a[8];
+#pragma unroll
+        for(int q = 0; q < 8; q++)
+            a[q] = (q < 4 ? WI : WJ)[(int64_t)(4*(q & 3)+lr)*ld+r0*16+prow];
         double4_t acc[2];
 #pragma unroll
         for(int n = 0; n < 2; n++)
             acc[n] = double4_t{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for(int q = 0; q < 16; q++)
+        for(int q = 0; q < 8; q++)
 #pragma unroll
             for(int n = 0; n < 2; n++)
-                acc[n] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q],
-                        JB[n][4*q*PW], acc[n], 0, 0, 0);
-        if(rb+4 < nrb)
-            load(rb+4);
+                acc[n] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q], jb[q][n],
+                        acc[n], 0, 0, 0);
 #pragma unroll
         for(int n = 0; n < 2; n++)
         {
-            double *dst = WD+(int64_t)(n*16+lc)*ld+rb*16+4*lr;
+            double *dst = (n == 0 ? WI : WJ)+(int64_t)lc*ld+r0*16+4*lr;
 #pragma unroll
             for(int v = 0; v < 4; v++)
                 dst[v] = acc[n][v];
@@ -453,15 +403,15 @@ __global__ __launch_bounds__(256) void jb_off_kernel(TileDesc *tiles,
     int limit;
     if(!rank_limit(td, limit))
         return;
-    const int p = td.p, nb = (p+BW-1)/BW;
+    const int p = td.p, nb = (p+OB-1)/OB;
     int bi = 0, rest = blockIdx.x;
     while(bi < nb && rest >= nb-bi)
         rest -= nb-bi++;
     if(bi >= nb)
         return;
     const int bj = bi+rest, ld = ld_of(p);
-    const double *WI = ws+td.j_off+(int64_t)bi*BW*ld;
-    const double *WJ = ws+td.j_off+(int64_t)bj*BW*ld;
+    const double *WI = ws+td.j_off+(int64_t)bi*OB*ld;
+    const double *WJ = ws+td.j_off+(int64_t)bj*OB*ld;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int lc = lane & 15, lr = lane >> 4;
     double4_t g[2][2];
@@ -502,7 +452,7 @@ __global__ __launch_bounds__(256) void jb_off_kernel(TileDesc *tiles,
         const int a = t >> 3, b = (t >> 2) & 1, v = t & 3;
         const double x = ((g[a][b][v]+part[0][t*64+lane])+
                 part[1][t*64+lane])+part[2][t*64+lane];
-        const int i = bi*BW+a*16+lr+4*v, j = bj*BW+b*16+lc;
+        const int i = bi*OB+a*16+lr+4*v, j = bj*OB+b*16+lc;
         if(i < j)
             off += x*x;
         else if(i == j && i < p)
@@ -645,16 +595,17 @@ int pipeline_jacobi_block(TileDesc *d_tiles, int *d_list, int count,
 {
     if(count <= 0)
         return STARSH_SUCCESS;
-    int nb = (pmax+BW-1)/BW, nbe = nb+(nb & 1);
     hipLaunchKernelGGL(jb_state_kernel, dim3((count+255)/256), dim3(256), 0,
             s, d_tiles, d_list, count);
     hipLaunchKernelGGL(jb_max_kernel, dim3((pmax+7)/8, count), dim3(256), 0,
             s, d_tiles, d_list, ws);
-    hipLaunchKernelGGL(jb_init_kernel, dim3((pmax+31)/32*nbe, count),
+    hipLaunchKernelGGL(jb_init_kernel, dim3((pmax+31)/32*
+                ((pmax+63)/64*2), count),
             dim3(256), 0, s, d_tiles, d_list, ws);
     HIP_TRY(hipGetLastError());
     for(int sweep = 0; sweep < max_sweeps; sweep++)
     {
+        const int nbe = blocks_of(pmax);
         for(int round = 0; round < nbe-1; round++)
             hipLaunchKernelGGL(jb_round_kernel, dim3(nbe/2, count), dim3(NT),
                     0, s, d_tiles, d_list, ws, round);
@@ -662,6 +613,7 @@ int pipeline_jacobi_block(TileDesc *d_tiles, int *d_list, int count,
         // most, the others are tried again
         if(certify && (sweep == 1 || sweep == 2 || sweep == 3 || sweep == 6))
         {
+            const int nb = (pmax+OB-1)/OB;
             hipLaunchKernelGGL(jb_off_kernel, dim3(nb*(nb+1)/2, count),
                     dim3(256), 0, s, d_tiles, d_list, ws);
             hipLaunchKernelGGL(jb_cert_kernel, dim3(count), dim3(256), 0, s,
@@ -680,8 +632,7 @@ int pipeline_jacobi_block(TileDesc *d_tiles, int *d_list, int count,
         count = h_out[0];
         if(count == 0)
             break;
-        nb = (h_out[1]+BW-1)/BW;
-        nbe = nb+(nb & 1);
+        pmax = h_out[1];
     }
     return STARSH_SUCCESS;
 }

@@ -1,5 +1,5 @@
 """Block Jacobi of the cores beyond LDS (csrc/hip/core_block.hip): tiles of
-known singular values whose core sizes sit at the edges of the 32-column
+known singular values whose core sizes sit at the edges of the 16-column
 blocks, the 16-row fragments and the even block count, against the spectrum
 they were built from; and the early verdict on a rank above the limit
 against the same tiles run to convergence."""
