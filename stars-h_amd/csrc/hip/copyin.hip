@@ -15,6 +15,7 @@
 #include <algorithm>
 #include <atomic>
 #include <condition_variable>
+#include <memory>
 #include <mutex>
 #include <thread>
 #include <vector>
@@ -28,17 +29,26 @@ constexpr int64_t PIECE = (int64_t)1 << 16;     // doubles per copy: 512 KiB
 // below this the threads cost more than they save
 constexpr int64_t SMALL = (int64_t)1 << 19;     // doubles: 4 MiB
 
-// The ring, kept between calls (128 MiB); one upload uses it at a time, a
-// second one at the same time takes the simple path.
+// The ring, kept between calls (as many slots as the largest upload took, at
+// most 128 MiB); one upload uses it at a time, a second one at the same time
+// takes the simple path.
 std::mutex ring_mu;
 double *ring = nullptr;
+int64_t ring_slots = 0;
 hipEvent_t ring_ev[NSLOT] = {};
 
-int ring_reserve()
+int ring_reserve(int64_t slots)
 {
-    if(ring == nullptr)
-        HIP_TRY(hipHostMalloc((void **)&ring, sizeof(double)*CHUNK*NSLOT,
+    if(ring_slots < slots)
+    {
+        if(ring != nullptr)
+            HIP_TRY(hipHostFree(ring));
+        ring = nullptr;
+        ring_slots = 0;
+        HIP_TRY(hipHostMalloc((void **)&ring, sizeof(double)*CHUNK*slots,
                     hipHostMallocDefault));
+        ring_slots = slots;
+    }
     for(int s = 0; s < NSLOT; s++)
         if(ring_ev[s] == nullptr)
             HIP_TRY(hipEventCreateWithFlags(&ring_ev[s],
@@ -73,7 +83,7 @@ struct Upload
     std::mutex mu;
     std::condition_variable cv;
     std::vector<int> left;      // pieces of a chunk not yet packed
-    int64_t allowed = NSLOT;    // chunks below this have a free slot
+    int64_t allowed = ring_slots;   // chunks below this have a free slot
     Upload(const double *const *s, const std::vector<int64_t> &st, int64_t n)
         : src(s), start(st), total(n), npieces((n+PIECE-1)/PIECE)
     {
@@ -94,7 +104,7 @@ struct Upload
                 std::unique_lock<std::mutex> g(mu);
                 cv.wait(g, [&] { return allowed > c; });
             }
-            gather(src, start, a, b, ring+(c % NSLOT)*CHUNK+(a-c*CHUNK));
+            gather(src, start, a, b, ring+(c % ring_slots)*CHUNK+(a-c*CHUNK));
             bool full;
             {
                 std::lock_guard<std::mutex> g(mu);
@@ -122,6 +132,10 @@ int upload_ring(double *d_dst, const double *const *src,
     std::vector<std::thread> threads;
     unsigned nth = std::thread::hardware_concurrency();
     nth = nth < 4 ? 2 : (nth > 16 ? 14 : nth-2);
+    // a thread is started for 2 MiB at least: 14 threads for the 5.4 MB of a
+    // 2500-point operator took longer than the copy (0.33 ms so)
+    nth = (unsigned)std::min<int64_t>(nth, std::max<int64_t>(1,
+                up.npieces/4));
     // a thread that cannot be started leaves its share to the others
     try
     {
@@ -143,15 +157,15 @@ int upload_ring(double *d_dst, const double *const *src,
             up.cv.wait(g, [&] { return up.left[(size_t)c] == 0; });
         }
         const int64_t a = c*CHUNK, len = std::min(CHUNK, total-a);
-        err = hipMemcpyAsync(d_dst+a, ring+(c % NSLOT)*CHUNK,
+        err = hipMemcpyAsync(d_dst+a, ring+(c % ring_slots)*CHUNK,
                 sizeof(double)*(size_t)len, hipMemcpyHostToDevice, s);
         if(err == hipSuccess)
-            err = hipEventRecord(ring_ev[c % NSLOT], s);
+            err = hipEventRecord(ring_ev[c % ring_slots], s);
         // two slots stay on their way while the others are packed
         if(err == hipSuccess && c >= 2)
         {
-            err = hipEventSynchronize(ring_ev[(c-2) % NSLOT]);
-            up.allow(c-2+NSLOT+1);
+            err = hipEventSynchronize(ring_ev[(c-2) % ring_slots]);
+            up.allow(c-2+ring_slots+1);
         }
     }
     up.allow(nchunks);          // also after an error: the threads run out
@@ -179,14 +193,15 @@ extern "C" int hip_upload_segments(double *d_dst, int64_t nseg,
         std::unique_lock<std::mutex> g(ring_mu, std::defer_lock);
         if(total > SMALL && g.try_lock())
         {
-            const int info = ring_reserve();
+            const int info = ring_reserve(std::min<int64_t>(NSLOT,
+                    (total+CHUNK-1)/CHUNK));
             if(info != STARSH_SUCCESS)
                 return info;
             return upload_ring(d_dst, src, start, total);
         }
-        std::vector<double> h((size_t)total);
-        gather(src, start, 0, total, h.data());
-        return starsh_hip_memcpy_h2d(d_dst, h.data(),
+        const std::unique_ptr<double[]> h(new double[(size_t)total]);
+        gather(src, start, 0, total, h.get());
+        return starsh_hip_memcpy_h2d(d_dst, h.get(),
                 sizeof(double)*(size_t)total);
     }
     catch(...)
@@ -202,4 +217,5 @@ extern "C" void hip_upload_release(void)
     if(ring != nullptr)
         (void)hipHostFree(ring);
     ring = nullptr;
+    ring_slots = 0;
 }

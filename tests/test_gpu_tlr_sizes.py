@@ -188,6 +188,32 @@ def test_uploads_from_two_threads():
     assert np.max(np.abs(out[0]-ref)) <= 1e-13*np.max(np.abs(ref))*np.sqrt(N)
 
 
+@pytest.mark.parametrize("total", [(1 << 19)+1, 1 << 21, (1 << 21)+1,
+                                   3*(1 << 21)+5, 11*(1 << 21)+7])
+def test_upload_sizes(total):
+    """Arrays of odd lengths, empty ones among them, whose sum sits at the
+    edges of the pinned ring's slots: one slot, its growth, and more slots
+    than it holds, from a ring that starts empty."""
+    L = S.lib()
+    if total == (1 << 19)+1:
+        assert L.starsh_hip_set_option(b"release_workspace",
+                                       C.c_double(0.0)) == 0
+    data = np.random.default_rng(total).random(total)
+    cuts = np.sort(np.random.default_rng(1).integers(0, total, 40))
+    cuts[5] = cuts[6]
+    parts = [np.ascontiguousarray(x) for x in np.split(data, cuts)]
+    src = (C.c_void_p*len(parts))(*[x.ctypes.data for x in parts])
+    size = (C.c_int64*len(parts))(*[len(x) for x in parts])
+    d = C.c_void_p()
+    assert L.starsh_hip_malloc(C.byref(d), C.c_size_t(8*total)) == 0
+    assert L.hip_upload_segments(d, C.c_int64(len(parts)), src, size) == 0
+    back = np.zeros(total)
+    assert L.starsh_hip_memcpy_d2h(back.ctypes.data_as(C.c_void_p), d,
+                                   C.c_size_t(8*total)) == 0
+    L.starsh_hip_free(d)
+    assert np.array_equal(back, data)
+
+
 @pytest.mark.parametrize("nrhs", [1, 3])
 def test_cg_columns_stop_on_their_own(nrhs):
     """Columns that converge at different iterations, among them one that
