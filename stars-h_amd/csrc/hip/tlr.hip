@@ -22,7 +22,8 @@
 // everything):
 //   N=2500, tile 250, 1 rhs (launch-bound)                  27.7 -> 10.7 us
 //   N=64000, tile 1600, ranks 8-31, 1 rhs, 358 MB, read
-//     twice at 5.3 TB/s                                      144 -> 138 us
+//     twice                                              129-146 -> 129-139 us
+//   the same with ranks to 133, 1566 MB                       578 -> 503 us
 //   N=30000, tile 1700, nonsymmetric, ranks to 90, 12 dense
 //     tiles, 10 rhs, 812 MB                                 4470 -> 260 us
 //   CG iteration, N=10000, tile 1000, 10 dense tiles         610 -> 72 us
