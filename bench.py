@@ -45,7 +45,7 @@ PEAK_FP64 = 78.6  # TFLOP/s, MI355X dense FP64 (vector and matrix)
 # profiles/c2_counters.md).  HBM bytes are FETCH_SIZE and WRITE_SIZE (KiB)
 # scaled by the same counters on a 1 GiB device copy (fetch x2.00, write
 # x1.00).
-C2_PLAIN_SKETCH_TRAFFIC = 7.332e9   # gen_gemm_kernel<2,2,256,1,false>
+C2_PLAIN_SKETCH_TRAFFIC = 1.843e9   # gen_gemm_kernel<2,2,128,1,false>
 C2_MIXED_PROJ_TRAFFIC = 0.660e9     # proj_i8_kernel<2,2,64,false>
 C2_MIXED_PROJ_VALU_INSTS = 1.030e9  # SQ_INSTS_VALU (wave64 instructions)
 C2_MIXED_PROJ_VALU_BUSY = 0.69      # VALUBusy at the kernel's clock

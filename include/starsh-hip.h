@@ -267,7 +267,7 @@ typedef struct starsh_hip_tuning
     int first_bucket;       /* mixed: chosen first bucket (0..4 on ladder
                              * 0, 0..5 on ladder 1), else -1 */
     int tile_schedule;      /* mixed: per-tile schedule kept (1) or not */
-    int qr_panel;           /* chosen Gram-Schmidt panel width (0: by batch,
+    int qr_panel;           /* chosen Gram-Schmidt panel width (0: by size,
                              * 4, 8) */
     int sketch_bn, sketch_rw;   /* plain: sketch GEMM column block and
                                  * 16-row groups per wave (0: by size) */

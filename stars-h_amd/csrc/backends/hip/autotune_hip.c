@@ -72,7 +72,7 @@ typedef struct sched_entry
     int form;               /* 0 plain, 1 mixed */
     int first;              /* mixed: first bucket (of `ladder`) */
     int ladder;             /* mixed: bucket ladder (0, 1) */
-    int panel;              /* Gram-Schmidt panel width, 0 = by batch */
+    int panel;              /* Gram-Schmidt panel width, 0 = by size */
     int gemm_bn[2], gemm_rw[2];     /* [0] sketch, [1] projection */
     unsigned long long geom;
     int ntile;

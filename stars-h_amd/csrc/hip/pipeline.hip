@@ -122,7 +122,7 @@ ActiveProbe probe;
 // at most 2048 rows), 4, or 8 (again up to 2048 rows); set by
 // starsh_hip_set_option("qr_panel").
 int qr_panel_width = 0;
-// The width chosen by the autotuner for the current call (0 = by batch);
+// The width chosen by the autotuner for the current call (0 = by size);
 // the option above wins.
 int qr_panel_tuned = 0;
 
