@@ -28,7 +28,9 @@
 //     tiles, 10 rhs, 812 MB                                 4470 -> 260 us
 //   CG iteration, N=10000, tile 1000, 10 dense tiles         610 -> 72 us
 // Reading U once for U^T X and keeping V (U^T X) (1.5 reads instead of 2)
-// needs a workgroup per tile: 96 + 40 us for the second line against 64 + 70.
+// needs a workgroup per tile: 96 + 40 us for the second line against 64 + 70;
+// the two tie there and at 430 MB (151 against 153 us), and reading twice
+// wins for smaller and larger operators and for more vectors.
 #include <stdio.h>
 #include "hip_common.h"
 #include "tlr.h"

@@ -188,14 +188,14 @@ def test_uploads_from_two_threads():
     assert np.max(np.abs(out[0]-ref)) <= 1e-13*np.max(np.abs(ref))*np.sqrt(N)
 
 
-@pytest.mark.parametrize("total", [(1 << 19)+1, 1 << 21, (1 << 21)+1,
+@pytest.mark.parametrize("total", [(1 << 20)+1, 1 << 21, (1 << 21)+1,
                                    3*(1 << 21)+5, 11*(1 << 21)+7])
 def test_upload_sizes(total):
     """Arrays of odd lengths, empty ones among them, whose sum sits at the
     edges of the pinned ring's slots: one slot, its growth, and more slots
     than it holds, from a ring that starts empty."""
     L = S.lib()
-    if total == (1 << 19)+1:
+    if total == (1 << 20)+1:
         assert L.starsh_hip_set_option(b"release_workspace",
                                        C.c_double(0.0)) == 0
     data = np.random.default_rng(total).random(total)
