@@ -247,8 +247,10 @@ int bcgs2(TileDesc *d_tiles, int ntiles, int which, double *ws, int kmax,
         TRY(pipeline_gs_block(d_tiles, ntiles, which, ws, j0, pb, kmax,
                     tau_first, TAU_SECOND, d_keep, d_norms, d_coef, rows_max,
                     d_active, s));
-        if(gs_next(j0) >= width_max)
-            break;
+        // also after the last block, where nothing reads it: a batch of one
+        // block that queued no small copy before its factors went to the host
+        // moved them at 29 instead of 52 GB/s (2D sqexp N=64000 mixed, 430 MB:
+        // 15.0 ms; with the copies 8.6-9.4, now and then 15)
         const int slot = block % NSLOT;
         HIP_TRY(hipMemcpyAsync(probe.h+slot, d_active, sizeof(int),
                     hipMemcpyDeviceToHost, s));
