@@ -13,7 +13,7 @@
 // singular values; Jacobi on R2^T converges in fewer sweeps than on R2.
 #include <float.h>
 #include "pipeline.h"
-#include "jacobi_fast.h"
+#include "jacobi_rotation.h"
 
 namespace {
 
@@ -40,10 +40,10 @@ __device__ inline bool rotate_pair(double *wa, double *wb, int p, int g,
     al = group_sum(al, g);
     be = group_sum(be, g);
     ga = group_sum(ga, g);
-    if(!jr_rotates_fast(al, be, ga, ctol))
+    if(!jr_rotates(al, be, ga, ctol))
         return false;
     double c, s;
-    jacobi_rotation_fast(al, be, ga, c, s);
+    jacobi_rotation(al, be, ga, c, s);
     for(int i = gl; i < p; i += g)
     {
         double u = wa[i], v = wb[i];
@@ -80,10 +80,10 @@ __device__ inline bool rotate_pair_reg(double *wa, double *wb, int p, int g,
     al = group_sum(al, g);
     be = group_sum(be, g);
     ga = group_sum(ga, g);
-    if(!jr_rotates_fast(al, be, ga, ctol))
+    if(!jr_rotates(al, be, ga, ctol))
         return false;
     double c, s;
-    jacobi_rotation_fast(al, be, ga, c, s);
+    jacobi_rotation(al, be, ga, c, s);
 #pragma unroll
     for(int q = 0; q < E; q++)
     {

@@ -36,7 +36,7 @@
 #include <float.h>
 #include <math.h>
 #include "pipeline.h"
-#include "jacobi_fast.h"
+#include "jacobi_rotation.h"
 
 typedef double double4_t __attribute__((ext_vector_type(4)));
 
@@ -255,7 +255,7 @@ __global__ __launch_bounds__(NT) void jb_round_kernel(TileDesc *tiles,
         {
             const int i = e/PW, j = e % PW;
             if(i < j)
-                any |= jr_rotates_fast(G[i*(PW+1)], G[j*(PW+1)], G[e], ctol);
+                any |= jr_rotates(G[i*(PW+1)], G[j*(PW+1)], G[e], ctol);
         }
         if(__syncthreads_or(any) == 0)
             return;
@@ -291,9 +291,9 @@ __global__ __launch_bounds__(NT) void jb_round_kernel(TileDesc *tiles,
         pc = 1.0;
         ps = 0.0;
         double c = 1.0, s = 0.0;
-        const bool rot = jr_rotates_fast(al, be, ga, ctol);
+        const bool rot = jr_rotates(al, be, ga, ctol);
         if(rot)
-            jacobi_rotation_fast(al, be, ga, c, s);
+            jacobi_rotation(al, be, ga, c, s);
         if(__ballot(rot) == 0)
             continue;               // the same in every wave
         rotated = true;

@@ -9,7 +9,10 @@ and must vanish to working precision relative to the rotated norms.  The
 cases cover ordinary magnitudes and the ends of the FP64 range, where the
 squares of d = be - al and h = 2 ga inside the formula underflow or
 overflow (al, be near 1e-160, 1e-200, 1e-300, 1e200, 1e300; d == 0 with
-h*h below the smallest double), and no value may become NaN or Inf.
+h*h below the smallest double), norms and angles of very different size
+(|h| << |d|), and no value may become NaN or Inf.  The kernels start from
+hardware approximations of 1/sqrt(x) and 1/x (below 2^-24 measured); here
+those are rounded to single precision, which is no better.
 Columns of two rows check the whole step (sums, test, rotation, update) at
 magnitudes whose squares are normal numbers.
 """
@@ -61,8 +64,7 @@ def _gram_cases():
     return out
 
 
-def test_rotation_orthogonalises_across_the_fp64_range(rot_bin):
-    cases = _gram_cases()
+def _check_rotations(rot_bin, cases):
     res = _run(rot_bin, [f"g {float(al)!r} {float(be)!r} {float(ga)!r}"
                          for al, be, ga in cases])
     assert len(res) == len(cases)
@@ -79,6 +81,48 @@ def test_rotation_orthogonalises_across_the_fp64_range(rot_bin):
         rel = abs(off) / Fr(math.sqrt(float(na / A))) / \
             Fr(math.sqrt(float(nb / A))) / A
         assert float(rel) <= 2e-15, (al, be, ga, float(rel))
+
+
+def test_rotation_orthogonalises_across_the_fp64_range(rot_bin):
+    _check_rotations(rot_bin, _gram_cases())
+
+
+def _skew_cases():
+    """Norms up to 260 orders apart, cosines from 1e-13 to 0.999, on either
+    side of the 1e-130 below which the norms are taken one at a time."""
+    rng = np.random.default_rng(17)
+    out = []
+    for _ in range(400):
+        al = 10.0 ** rng.uniform(-20, 1)
+        be = al * 10.0 ** -rng.uniform(0, 240)
+        cosang = 10.0 ** -rng.uniform(0.0005, 13) * rng.choice([-1, 1])
+        pair = (al, be) if rng.integers(2) else (be, al)
+        out.append(pair + (cosang * math.sqrt(al) * math.sqrt(be),))
+    for be in (0.9e-130, 1.0e-130, 1.1e-130):
+        for cosang in (1e-12, 1e-3, 0.9):
+            out.append((1.0, be, cosang * math.sqrt(be)))
+            out.append((be, 1.3 * be, cosang * be))
+    return out
+
+
+def test_rotation_of_norms_and_angles_far_apart(rot_bin):
+    _check_rotations(rot_bin, _skew_cases())
+
+
+def test_rotation_test_on_both_sides_of_its_switch(rot_bin):
+    """The verdict |ga| > ctol |a||b| (ctol = 2 eps) just above and just
+    below the threshold, with the smaller norm on either side of 1e-130 and
+    the larger one on either side of 1e130."""
+    ctol = 2 * 2.220446049250313e-16
+    lines, want = [], []
+    for al, be in ((1.0, 0.5), (1.0, 1.1e-130), (1.0, 0.9e-130),
+                   (3e-131, 2e-130), (1e-200, 1e-180), (0.9e130, 2.0),
+                   (1.1e130, 2.0), (1e300, 1e250)):
+        for f, w in ((1.0 + 1e-12, 1), (1.0 - 1e-12, 0)):
+            ga = f * ctol * math.sqrt(al) * math.sqrt(be)
+            lines.append(f"g {al!r} {be!r} {ga!r}")
+            want.append(w)
+    assert [int(r[0]) for r in _run(rot_bin, lines)] == want
 
 
 def test_rotation_test_does_not_underflow(rot_bin):
