@@ -168,7 +168,12 @@ int upload_ring(double *d_dst, const double *const *src,
             up.allow(c-2+ring_slots+1);
         }
     }
-    up.allow(nchunks);          // also after an error: the threads run out
+    // after an error the copies queued so far still read their slots (and
+    // write d_dst, which the caller may free): wait for them before the
+    // threads run out and refill the slots
+    if(err != hipSuccess)
+        (void)hipStreamSynchronize(s);
+    up.allow(nchunks);
     for(auto &t : threads)
         t.join();
     HIP_TRY(err);
