@@ -31,30 +31,40 @@ constexpr int64_t PIECE = (int64_t)1 << 16;     // doubles per copy: 512 KiB
 constexpr int64_t SMALL = (int64_t)1 << 20;     // doubles: 8 MiB
 
 // The ring, kept between calls (as many slots as the largest upload took, at
-// most 128 MiB); one upload uses it at a time, a second one at the same time
-// takes the simple path.
+// most 128 MiB); one upload uses it at a time.  A second one at the same time,
+// or one that gets no pinned memory or no thread, takes the simple path.
 std::mutex ring_mu;
 double *ring = nullptr;
 int64_t ring_slots = 0;
 hipEvent_t ring_ev[NSLOT] = {};
 
-int ring_reserve(int64_t slots)
+// False (and no HIP error left behind) where the ring cannot be had.
+bool ring_reserve(int64_t slots)
 {
     if(ring_slots < slots)
     {
         if(ring != nullptr)
-            HIP_TRY(hipHostFree(ring));
+            (void)hipHostFree(ring);
         ring = nullptr;
         ring_slots = 0;
-        HIP_TRY(hipHostMalloc((void **)&ring, sizeof(double)*CHUNK*slots,
-                    hipHostMallocDefault));
+        if(hipHostMalloc((void **)&ring, sizeof(double)*CHUNK*slots,
+                    hipHostMallocDefault) != hipSuccess)
+        {
+            ring = nullptr;
+            (void)hipGetLastError();
+            return false;
+        }
         ring_slots = slots;
     }
     for(int s = 0; s < NSLOT; s++)
-        if(ring_ev[s] == nullptr)
-            HIP_TRY(hipEventCreateWithFlags(&ring_ev[s],
-                        hipEventDisableTiming));
-    return STARSH_SUCCESS;
+        if(ring_ev[s] == nullptr && hipEventCreateWithFlags(&ring_ev[s],
+                    hipEventDisableTiming) != hipSuccess)
+        {
+            ring_ev[s] = nullptr;
+            (void)hipGetLastError();
+            return false;
+        }
+    return true;
 }
 
 // Copies elements [a, b) of the concatenated arrays to dst; start[q] is the
@@ -125,6 +135,8 @@ struct Upload
     }
 };
 
+// Returns NO_THREADS, with nothing done, if no thread can be started.
+constexpr int NO_THREADS = -100;     // none of the library's codes
 int upload_ring(double *d_dst, const double *const *src,
         const std::vector<int64_t> &start, int64_t total)
 {
@@ -146,7 +158,7 @@ int upload_ring(double *d_dst, const double *const *src,
     catch(...)
     {
         if(threads.empty())
-            return STARSH_MALLOC_ERROR;
+            return NO_THREADS;
     }
     hipError_t err = hipSuccess;
     const int64_t nchunks = (int64_t)up.left.size();
@@ -198,12 +210,15 @@ extern "C" int hip_upload_segments(double *d_dst, int64_t nseg,
         std::unique_lock<std::mutex> g(ring_mu, std::defer_lock);
         if(total > SMALL && g.try_lock())
         {
-            const int info = ring_reserve(std::min<int64_t>(NSLOT,
-                    (total+CHUNK-1)/CHUNK));
-            if(info != STARSH_SUCCESS)
-                return info;
-            return upload_ring(d_dst, src, start, total);
+            if(ring_reserve(std::min<int64_t>(NSLOT, (total+CHUNK-1)/CHUNK)))
+            {
+                const int info = upload_ring(d_dst, src, start, total);
+                if(info != NO_THREADS)
+                    return info;
+            }
+            g.unlock();
         }
+        // small, or the ring is in use or cannot be had
         const std::unique_ptr<double[]> h(new double[(size_t)total]);
         gather(src, start, 0, total, h.get());
         return starsh_hip_memcpy_h2d(d_dst, h.get(),

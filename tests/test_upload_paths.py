@@ -1,7 +1,8 @@
 """Host test of the factor upload's failure paths (stars-h_amd/csrc/hip/
 copyin.hip compiled for the host, the runtime's calls replaced by
-copyin_host.cpp): after a failed copy nothing is left queued and no slot is
-refilled under a queued copy."""
+copyin_host.cpp): where the pinned ring or its threads cannot be had, the
+arrays go through ordinary memory; after a failed copy nothing is left queued
+and no slot is refilled under a queued copy."""
 import os
 import subprocess
 
@@ -34,7 +35,7 @@ def _run(binary, mode):
     return [int(x) for x in res.stdout.split()]
 
 
-@pytest.mark.parametrize("mode", ["ok"])
+@pytest.mark.parametrize("mode", ["ok", "pin", "thread"])
 def test_arrays_arrive(upload_bin, mode):
     assert _run(upload_bin, mode) == [0, 1, 0, 0]
 
