@@ -518,7 +518,7 @@ int starsh_itersolvers__dcg_hip(STARSH_blrm *matrix, int nrhs, double *B,
         info = starsh_hip_cg_start(n, nrhs, tol, dR, dpart, dst);
     /* The iterations are queued without waiting: a column that has met its
      * stopping rule is left alone by the kernels, and the states are read
-     * back after 4, 8 and then every 16 iterations (two dot products read
+     * back after 4, 12 and then every 16 iterations (two dot products read
      * back per iteration took as long as its kernels). */
     int look = 4, batch = 4;
     for(int it = 0; it < n && info == STARSH_SUCCESS; it++)
@@ -533,15 +533,16 @@ int starsh_itersolvers__dcg_hip(STARSH_blrm *matrix, int nrhs, double *B,
         look += batch;
         info = starsh_hip_memcpy_d2h(hst, dst+(size_t)((it+1) & 1)*nrhs,
                 sizeof(tlr_cg_state)*nrhs);
-        int last = -1, finished = 0;
+        int last = -1, finished = 0, running = 0;
         for(int q = 0; info == STARSH_SUCCESS && q < nrhs; q++)
         {
             finished += hst[q].done >= 0;
+            running += hst[q].done == -1;
             last = hst[q].done > last ? hst[q].done : last;
         }
-        if(info == STARSH_SUCCESS && finished == nrhs)
+        if(info == STARSH_SUCCESS && running == 0)
         {
-            result = last;
+            result = finished == nrhs ? last : -1;
             break;
         }
     }

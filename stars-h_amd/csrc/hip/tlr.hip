@@ -390,7 +390,7 @@ __global__ __launch_bounds__(256) void cg_start_kernel(const double *part,
         tlr_cg_state &s = st[blockIdx.x];
         s.rsold = rs*rs;
         s.rscheck = rs*tol;
-        s.done = -1;
+        s.done = s.rscheck < 0.0 ? -2 : -1;
     }
 }
 
@@ -400,7 +400,7 @@ __global__ __launch_bounds__(256) void cg_step_kernel(int64_t n,
         const double *q, double *x, double *r, double *part2)
 {
     const tlr_cg_state s = st[blockIdx.y];
-    if(s.done >= 0)
+    if(s.done != -1)
         return;
     const int64_t o = blockIdx.y*n;
     const double pq = sum_parts(part1+(int64_t)blockIdx.y*CG_BLOCKS,
@@ -425,7 +425,7 @@ __global__ __launch_bounds__(256) void cg_next_kernel(int64_t n, int it,
         const double *r, double *p)
 {
     tlr_cg_state s = st[blockIdx.y];
-    if(s.done < 0)
+    if(s.done == -1)
     {
         const double rs = sqrt(sum_parts(part2+(int64_t)blockIdx.y*CG_BLOCKS,
                     gridDim.x));

@@ -73,7 +73,8 @@ int starsh_hip_tlr_time(const tlr_plan *pl, double *d_tmp, int nrhs,
 
 /* Conjugate gradients on the library stream, nrhs columns of n (n apart).
  * State of a column: |r|^2, the value |r| is checked against, and the
- * iteration that met it (-1: none yet). */
+ * iteration that met it (-1: none yet; -2: the value is negative, and as in
+ * cg.c the column is left alone and never meets it). */
 typedef struct
 {
     double rsold, rscheck;

@@ -238,3 +238,23 @@ def test_cg_columns_stop_on_their_own(nrhs):
         assert np.linalg.norm(Y[:, q]-X[:, q]) <= 2e-10*cond*np.linalg.norm(
             X[:, q])
     p.free_matrix()
+
+
+def _covariance(N=700):
+    fn = S.init("HIP", oversample=16)
+    rng = np.random.default_rng(3)
+    p = S.TLRProblem("spatial", N, 2, 100, kernel="exp", beta=0.1,
+                     noise=0.01, points=rng.random((2, N)))
+    assert p.approximate(60, 1e-9, 0, fn) == 0
+    return p, p.dmml(np.eye(N)), rng
+
+
+def test_cg_leaves_columns_of_a_negative_rule_alone():
+    """A negative tolerance gives every column a negative check value: the
+    reference skips such columns and never converges."""
+    p, A, rng = _covariance(300)
+    B = rng.standard_normal((len(A), 2))
+    X0 = rng.standard_normal(B.shape)
+    it, X = p.cg(B, X0, -0.5)
+    assert it == -1 and np.array_equal(X, X0)
+    p.free_matrix()
