@@ -105,13 +105,15 @@ typedef struct starsh_hip_stats
     double wall_seconds;     /* whole API call incl. copy-back */
     double copy_seconds;     /* device-to-host copy of U, V and D */
     double dominant_kernel_seconds; /* summed duration of the sketch kernel */
-    long long dominant_kernel_launches;
+    long long dominant_kernel_launches; /* of the sketch kernel: one per batch,
+                                or one per chunk of columns computed */
     long long ntiles;        /* far-field tiles compressed */
     long long nfalse_far;    /* tiles that turned out to be dense */
     int rank_min, rank_max;
     double rank_avg;
     double flops_algorithmic;   /* work of the reference algorithm */
-    double sketch_bytes_or_flops; /* algorithmic flops of the sketch kernel */
+    double sketch_bytes_or_flops; /* 2 m n flop for every sketch column that
+                                was computed */
     /* host-side timeline of the call (seconds; their sum with the device
      * batches is the wall time) */
     double prepare_seconds;  /* argument checks, point upload, U/V malloc */

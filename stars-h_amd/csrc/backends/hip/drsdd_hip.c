@@ -758,7 +758,7 @@ int hip_driver_run(const hip_batch *B, STARSH_int ntiles, const int *pidx,
         st->dominant_kernel_seconds += out.sketch_seconds;
         st->sketch_bytes_or_flops += out.sketch_flops;
         st->proj_kernel_seconds += out.proj_seconds;
-        st->dominant_kernel_launches += 1;
+        st->dominant_kernel_launches += out.sketch_launches;
         double tc = hip_driver_now();
         for(STARSH_int t = b0; t < b1; t++)
         {

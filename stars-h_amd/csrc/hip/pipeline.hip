@@ -643,12 +643,13 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
     // to its tail, as for the truncation itself, so the rank rule stays
     // conservative (flag 8).
     // columns sketched: all, or, of a tile exhausted in the block at gs_blk,
-    // the chunks up to the one that holds that block
+    // the chunks up to the one that holds that block (a captured Gram-Schmidt
+    // has all chunks computed before it)
     double sketch_flops = 0.0;
     for(int t = 0; t < nt; t++)
     {
         int cols = h[t].k;
-        if(nchunk > 1 && (h[t].flags & 1))
+        if(nchunk > 1 && !qr_graph && (h[t].flags & 1))
             for(int c = 0; c < nchunk; c++)
                 if(chunk[c].beg <= h[t].gs_blk && chunk[c].end < cols &&
                         chunk[c].end > h[t].gs_blk)
@@ -749,6 +750,7 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
     }
     out->sketch_seconds = ms_sk*1e-3;
     out->sketch_flops = sketch_flops;
+    out->sketch_launches = chunks_done > 1 ? chunks_done : 1;
     for(int t = 0; t < nt; t++)
     {
         out->rank[t] = h[t].rank;

@@ -86,6 +86,7 @@ typedef struct rsdd_output
     double device_seconds;
     double sketch_seconds;       /* sketch kernels (HIP events) */
     double sketch_flops;         /* 2 m n flop per sketch column computed */
+    int sketch_launches;
     double proj_seconds;         /* projection kernels (HIP events) */
 } RsddOutput;
 
