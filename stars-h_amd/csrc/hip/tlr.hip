@@ -15,6 +15,18 @@
 // With one right-hand side a lane multiplies its own values; with more, up
 // to 16 at a time go through FP64 MFMA (the columns past nrhs are zeros).
 //
+// Rounding: an MFMA adds its products to the accumulator one by one, so a
+// long chain of them loses what a lane's short one kept.  Chains end after 32
+// products (coefficients) or 16 (rows) and go to a sum of their own.  Relative
+// errors against long double, for chains as long as a wave's share, now, and
+// with a workgroup per tile and four right-hand sides at a time:
+//   N=2500, tile 250, rank 30, 4 rhs            4.2, 2.9, 2.3 e-16
+//   N=16000, tile 1000, rank 60, 16 rhs         7.2, 3.2, 2.6 e-16
+//   N=30000, tile 1700, dense tiles, 10 rhs     7.2, 2.5, 13.6 e-16
+//   N=64000, tile 1600, rank 31, 1 rhs          3.1, 2.6, 2.7 e-16
+// at 0-1% of the time (16-product chains in the coefficients too, 2.7 and 3.0
+// e-16 for the first two, cost 5%).
+//
 // What bounds it: HBM; every factor is read twice, every dense tile once.
 // Measured on MI355X, before and after (one workgroup per tile forming U^T X
 // and then V (U^T X) row by row, and strips of 64 rows, dense tiles one
@@ -49,6 +61,15 @@ template <bool ONE>
 struct Acc
 {
     double4_t v = {0.0, 0.0, 0.0, 0.0};
+    // adds another's sums and clears them
+    __device__ inline void take(Acc &o)
+    {
+        if constexpr(ONE)
+            v[0] += o.v[0];
+        else
+            v += o.v;
+        o.v = double4_t{0.0, 0.0, 0.0, 0.0};
+    }
     __device__ inline void add(double f, double b)
     {
         if constexpr(ONE)
@@ -133,9 +154,11 @@ __global__ __launch_bounds__(256) void tlr_coef1_kernel(const tlr_unit *units,
 // The same for up to 16 right-hand sides on MFMA: rows split over the four
 // waves in groups of 64, a lane taking rows 4 (lane/16) .. +3 of each block
 // of 16 (any order of the rows gives the same sum), so that it loads 32
-// contiguous bytes of a column.
-__global__ __launch_bounds__(256) void tlr_coef_kernel(const tlr_unit *units,
-        const double *fac, const double *x, int ldx, int nrhs, double *tmp)
+// contiguous bytes of a column.  Three workgroups per CU: with registers for
+// two, N=40000, tile 1265, 7 rhs took 93 instead of 85.5 us.
+__global__ __launch_bounds__(256, 3) void tlr_coef_kernel(
+        const tlr_unit *units, const double *fac, const double *x, int ldx,
+        int nrhs, double *tmp)
 {
     __shared__ double part[3][2][256];
     const tlr_unit u = units[blockIdx.x];
@@ -189,15 +212,18 @@ __global__ __launch_bounds__(256) void tlr_coef_kernel(const tlr_unit *units,
                     f[h][1][v] = in && ok[1] ? F[1][r] : 0.0;
                     b[h][v] = in && okq ? X[r] : 0.0;
                 }
+        auto sums = [&](int a) {
+            Acc<false> p[2];
 #pragma unroll
-        for(int h = 0; h < 4; h++)
+            for(int v = 0; v < 8; v++)
 #pragma unroll
-            for(int v = 0; v < 4; v++)
-            {
-                acc[0].add(f[h][0][v], b[h][v]);
-                if(two)
-                    acc[1].add(f[h][1][v], b[h][v]);
-            }
+                for(int h = 0; h < 4; h += 2)
+                    p[h/2].add(f[h+v/4][a][v&3], b[h+v/4][v&3]);
+            acc[a].v += p[0].v+p[1].v;
+        };
+        sums(0);
+        if(two)
+            sums(1);
     }
     if(wave > 0)
 #pragma unroll
@@ -220,12 +246,14 @@ __global__ __launch_bounds__(256) void tlr_coef_kernel(const tlr_unit *units,
             }
 }
 
-// Rows of a strip of 16 RF rows of one block row.
+// Rows of a strip of 16 RF rows of one block row.  Up to 32 rows four
+// workgroups per CU (with three, N=30000, tile 1100, 3 rhs took 224 instead of
+// 212 us).
 template <int RF, bool ONE>
-__global__ __launch_bounds__(256) void tlr_rows_kernel(const tlr_chunk *chunks,
-        const tlr_entry *entries, const double *fac, const double *tmp,
-        const double *x, int ldx, int nrhs, double alpha, double beta,
-        double *y, int ldy)
+__global__ __launch_bounds__(256, RF <= 2 ? 4 : 2) void tlr_rows_kernel(
+        const tlr_chunk *chunks, const tlr_entry *entries, const double *fac,
+        const double *tmp, const double *x, int ldx, int nrhs, double alpha,
+        double beta, double *y, int ldy)
 {
     __shared__ double part[3][RF][Acc<ONE>::N*64];
     const tlr_chunk ch = chunks[blockIdx.x];
@@ -242,7 +270,7 @@ __global__ __launch_bounds__(256) void tlr_rows_kernel(const tlr_chunk *chunks,
 #pragma unroll
     for(int a = 0; a < RF; a++)
         row[a] = ch.rofs+min(a*16+lc, ch.nrows-1);
-    Acc<ONE> acc[RF];
+    Acc<ONE> acc[RF], sum[RF];      // of 16 columns, of those before them
     for(int e = ch.first+wave; e < ch.last; e += 4)
     {
         const tlr_entry en = entries[e];
@@ -275,6 +303,9 @@ __global__ __launch_bounds__(256) void tlr_rows_kernel(const tlr_chunk *chunks,
 #pragma unroll
                 for(int a = 0; a < RF; a++)
                     acc[a].add(f[a][v], b[v]);
+#pragma unroll
+            for(int a = 0; a < RF; a++)
+                sum[a].take(acc[a]);
         }
         if(k0 < en.cols)
         {
@@ -299,16 +330,19 @@ __global__ __launch_bounds__(256) void tlr_rows_kernel(const tlr_chunk *chunks,
 #pragma unroll
                     for(int a = 0; a < RF; a++)
                         acc[a].add(f[a][v], b[v]);
+#pragma unroll
+            for(int a = 0; a < RF; a++)
+                sum[a].take(acc[a]);
         }
     }
 #pragma unroll
     for(int a = 0; a < RF; a++)
     {
-        acc[a].close();
+        sum[a].close();
         if(wave > 0)
 #pragma unroll
             for(int q = 0; q < Acc<ONE>::N; q++)
-                part[wave-1][a][q*64+lane] = acc[a].v[q];
+                part[wave-1][a][q*64+lane] = sum[a].v[q];
     }
     __syncthreads();
     if(wave == 0 && (ONE ? lane < 16 : okq))
@@ -320,7 +354,7 @@ __global__ __launch_bounds__(256) void tlr_rows_kernel(const tlr_chunk *chunks,
                 const int r = a*16+Acc<ONE>::row(q, lane);
                 if(r >= ch.nrows)
                     continue;
-                const double s = ((acc[a].v[q]+part[0][a][q*64+lane])+
+                const double s = ((sum[a].v[q]+part[0][a][q*64+lane])+
                         part[1][a][q*64+lane])+part[2][a][q*64+lane];
                 double *yy = y+(int64_t)(ONE ? q0 : q0+lc)*ldy+ch.row0+r;
                 *yy = beta == 0.0 ? alpha*s : fma(alpha, s, beta*(*yy));

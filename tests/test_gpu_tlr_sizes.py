@@ -4,6 +4,7 @@ no multiple of 16 or 64 rows, ranks around the 16- and 32-column groups and
 the 64-column pieces of an entry, one right-hand side (lane sums) and more
 (MFMA, groups of 16), dense tiles and their transposes."""
 import ctypes as C
+from fractions import Fraction
 
 import numpy as np
 import pytest
@@ -142,6 +143,69 @@ def _large(N, nb, symm, ranks, rng):
                 Y[rj] += v @ (u.T @ X[ri])
         return Y
     return M, apply, keep
+
+@pytest.mark.parametrize("nrhs", [1, 2])
+def test_long_sums_go_in_blocks(nrhs):
+    """Sums of 1700 products that start with 1 and go on with values below
+    half a unit of it, which a single chain of additions loses one by one:
+    dense tiles, transposed dense tiles and coefficients.  Every kernel adds
+    at most 32 products to one partial sum, and then the partial sums (at
+    most 28 per wave, and four waves): the error is at most that many units
+    of rounding."""
+    L = S.lib()
+    n = 1700
+    t = 0.99*2.0**-54
+    exact = float(Fraction(1)+(n-1)*Fraction(t))
+    u = 2.0**-53
+    col = np.full(n, t)
+    col[0] = 1.0
+    ones = np.ones((n, 1))
+    p = S.TLRProblem("spatial", 2*n, 2, n, symm="S", kernel="exp",
+                     points=np.random.default_rng(0).random((2, 2*n)))
+    tiles = [tuple(x) for x in p.tiles()]
+    assert sorted(tiles) == [(0, 0), (1, 0), (1, 1)]
+    dense = np.asfortranarray(np.tile(col, (n, 1)))
+    by_rows = np.asfortranarray(np.tile(col[:, None], (1, n)))
+    lowrank = (ones, np.asfortranarray(col[:, None]))
+    none = (np.zeros((n, 0), order="F"), np.zeros((n, 0), order="F"))
+    # what each block row of y = A (1, ..., 1) starts its sums with
+    for name, blocks, where in (
+            ("dense", {(0, 0): dense, (1, 0): none, (1, 1): none}, 0),
+            ("transposed", {(0, 0): none, (1, 0): by_rows, (1, 1): none}, 0),
+            ("coefficients", {(0, 0): lowrank, (1, 0): none,
+                              (1, 1): none}, 0),
+            ("twin's coefficients", {(0, 0): none, (1, 0): lowrank[::-1],
+                                     (1, 1): none}, 0)):
+        near = [q for q in tiles if not isinstance(blocks[q], tuple)]
+        far = [q for q in tiles if isinstance(blocks[q], tuple)]
+        F = C.POINTER(S.BLRF)()
+        assert L.starsh_blrf_new_from_coo(
+            C.byref(F), p.P, C.c_char(b"S"), p.C, p.C,
+            S.STARSH_int(len(far)), _ints([x for q in far for x in q]),
+            S.STARSH_int(len(near)), _ints([x for q in near for x in q]),
+            C.c_int(p.F.contents.type)) == 0
+        PA = C.POINTER(S.Array)
+        M = S.BLRM()
+        M.format = F
+        rk = [blocks[q][0].shape[1] for q in far]
+        one = np.ones((n, 1), order="F")
+        UV = [[_array(f if f.shape[1] else one) for f in blocks[q]]
+              for q in far]
+        M.far_rank = (C.c_int*max(1, len(far)))(*rk)
+        M.far_U = (PA*max(1, len(far)))(*[x[0] for x in UV])
+        M.far_V = (PA*max(1, len(far)))(*[x[1] for x in UV])
+        M.near_D = (PA*max(1, len(near)))(*[_array(blocks[q]) for q in near])
+        M.onfly = 0
+        X = np.ones((2*n, nrhs), order="F")
+        Y = np.zeros((2*n, nrhs), order="F")
+        dp = C.POINTER(C.c_double)
+        assert L.starsh_blrm__dmml_hip(
+            C.cast(C.byref(M), C.c_void_p), nrhs, 1.0, X.ctypes.data_as(dp),
+            2*n, 0.0, Y.ctypes.data_as(dp), 2*n) == 0
+        got = Y[where*n:(where+1)*n]
+        err = np.max(np.abs(got-exact))/u
+        print(name, nrhs, "error", err, "units", flush=True)
+        assert err <= 32+28+4
 
 
 def test_uploads_from_two_threads():
