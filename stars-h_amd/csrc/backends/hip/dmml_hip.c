@@ -186,9 +186,10 @@ int starsh_hip_tlr_new(starsh_hip_tlr **out, STARSH_blrm *M)
      * a tile with a twin: j), and the strips in the opposite order: what the
      * first launch read last is read first by the second, and again first by
      * the next product, while it is in the 256 MB cache in front of the
-     * memory.  N=64000, tile 1600, one vector: 358 MB 134.6 us with both in
-     * the tiles' order, 128.7 so; 700 MB 250 and 233; four vectors, 586 MB
-     * 329 and 315; below 130 MB and above 1.5 GB 2-4% */
+     * memory.  N=64000, tile 1600, one vector, with both in one direction
+     * and so: 358 MB 117.3 and 116.3 us, 431 MB 142.4 and 141.0, 700 MB
+     * 229.0 and 228.4, four vectors, 586 MB 323 and 316; 126 MB, which the
+     * cache holds, 46.0 and 47.0 */
     for(STARSH_int b = 0; b < nbr; b++)
         first[b+1] += first[b];
     for(STARSH_int bi = 0; bi < nfar; bi++)

@@ -27,22 +27,23 @@
 // at 0-1% of the time (16-product chains in the coefficients too, 2.7 and 3.0
 // e-16 for the first two, cost 5%).
 //
-// What bounds it: HBM; every factor is read twice, every dense tile once.
-// Measured on MI355X, before and after (one workgroup per tile forming U^T X
+// What bounds it: memory; every factor is read twice, every dense tile once.
+// A kernel that only reads runs at 6.0-6.2 TB/s here, 7.0 below 268 MB, which
+// the cache in front of the memory holds; the coefficients of C2's operator
+// (N=64000, tile 1600, 431 MB) run at 5.9, its rows at 6.4.  Measured on MI355X, before and after (one workgroup per tile forming U^T X
 // and then V (U^T X) row by row, and strips of 64 rows, dense tiles one
 // column at a time, right-hand sides in groups of four that each re-read
 // everything):
 //   N=2500, tile 250, 1 rhs (launch-bound)                  27.7 -> 10.7 us
 //   N=64000, tile 1600, ranks 8-31, 1 rhs, 358 MB, read
-//     twice                                              129-146 -> 129-139 us
-//   the same with ranks to 133, 1566 MB                       578 -> 503 us
+//     twice                                              129-146 -> 116-122 us
+//   the same with ranks to 133, 1566 MB                       578 -> 500 us
+//   C2's operator (2D sqexp, 431 MB), 1 rhs               149-152 -> 141 us
 //   N=30000, tile 1700, nonsymmetric, ranks to 90, 12 dense
 //     tiles, 10 rhs, 812 MB                                 4470 -> 260 us
 //   CG iteration, N=10000, tile 1000, 10 dense tiles         610 -> 72 us
 // Reading U once for U^T X and keeping V (U^T X) (1.5 reads instead of 2)
-// needs a workgroup per tile: 96 + 40 us for the second line against 64 + 70;
-// the two tie there and at 430 MB (151 against 153 us), and reading twice
-// wins for smaller and larger operators and for more vectors.
+// needs a workgroup per tile: 100 + 49 us for C2's operator against 74 + 67.
 #include <stdio.h>
 #include "hip_common.h"
 #include "tlr.h"
@@ -52,6 +53,16 @@ typedef double double4_t __attribute__((ext_vector_type(4)));
 namespace {
 
 constexpr int RHS = 16;         // right-hand sides per group
+
+// With more strips of 64 rows than this, one right-hand side goes through
+// tlr_rows1_kernel.  tlr_rows_kernel<4, true> has more loads in flight but
+// takes 154 registers, three workgroups per CU, 768 on the chip: 1000 strips
+// (C2's operator, 431 MB) left a second round nearly empty, 150 us for the
+// product against 141 with a lane per row (76 registers, six workgroups);
+// 358 MB 117.9 against 116.3, 700 MB 227.4 against 227.1.  Within one round it
+// wins: 563 strips 41.9 against 44.5 us, 625 46.2 against 46.9, 704 55.9
+// against 56.5.
+constexpr int ROWS1_STRIPS = 768;
 
 // Sums of one 16 x 16 fragment over its k: four MFMA steps' worth of a lane's
 // values f (row lane%16 of op(F)) times b.  With one right-hand side a lane
@@ -361,6 +372,85 @@ __global__ __launch_bounds__(256, RF <= 2 ? 4 : 2) void tlr_rows_kernel(
             }
 }
 
+// Rows of a 64-row strip, one right-hand side: a lane takes a row, so that a
+// column is one load of 512 contiguous bytes and its coefficient is the same
+// for the whole wave (it comes through the scalar unit).
+__global__ __launch_bounds__(256) void tlr_rows1_kernel(
+        const tlr_chunk *chunks, const tlr_entry *entries, const double *fac,
+        const double *tmp, const double *x, double alpha, double beta,
+        double *y)
+{
+    constexpr int KB = 16;
+    __shared__ double part[3][64];
+    const tlr_chunk ch = chunks[blockIdx.x];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // rows past the strip repeat its last one (their sums are not stored)
+    const int row = ch.rofs+min(lane, ch.nrows-1);
+    double sum = 0.0;
+    tlr_entry next = {};
+    if(ch.first+wave < ch.last)
+        next = entries[ch.first+wave];
+    for(int e = ch.first+wave; e < ch.last; e += 4)
+    {
+        const tlr_entry en = next;
+        next = entries[min(e+4, ch.last-1)];
+        const bool tr = en.kind == 2;
+        const double *F = fac+en.f_off+(tr ? (int64_t)row*en.ld : row);
+        const int64_t fs = tr ? 1 : en.ld;
+        const double *T = (en.kind == 0 ? tmp : x)+en.src_off;
+        double s0 = 0.0, s1 = 0.0;
+        for(int k0 = 0; k0 < en.cols; k0 += KB)
+        {
+            const int n = min(en.cols-k0, KB);  // as every test of it, uniform
+            double f[KB];
+#pragma unroll
+            for(int k = 0; k < KB; k += 4)
+                if(n >= k+4)
+                {
+#pragma unroll
+                    for(int v = 0; v < 4; v++)
+                        f[k+v] = F[(k0+k+v)*fs];
+                }
+                else
+                {
+#pragma unroll
+                    for(int v = 0; v < 3; v++)
+                        if(n > k+v)
+                            f[k+v] = F[(k0+k+v)*fs];
+                }
+#pragma unroll
+            for(int k = 0; k < KB; k += 4)
+                if(n >= k+4)
+                {
+#pragma unroll
+                    for(int v = 0; v < 4; v += 2)
+                    {
+                        s0 = fma(f[k+v], T[k0+k+v], s0);
+                        s1 = fma(f[k+v+1], T[k0+k+v+1], s1);
+                    }
+                }
+                else
+                {
+#pragma unroll
+                    for(int v = 0; v < 3; v++)
+                        if(n > k+v)
+                            s0 = fma(f[k+v], T[k0+k+v], s0);
+                }
+        }
+        sum += s0+s1;
+    }
+    if(wave > 0)
+        part[wave-1][lane] = sum;
+    __syncthreads();
+    if(wave == 0 && lane < ch.nrows)
+    {
+        const double s = ((sum+part[0][lane])+part[1][lane])+part[2][lane];
+        double *yy = y+ch.row0+lane;
+        *yy = beta == 0.0 ? alpha*s : fma(alpha, s, beta*(*yy));
+    }
+}
+
 // ---- vector kernels of conjugate gradients, one column of length n per
 // blockIdx.y (columns n apart).  Nothing of an iteration goes to the host:
 // the dot products stay as partial sums of at most CG_BLOCKS blocks, which
@@ -573,7 +663,16 @@ int starsh_hip_tlr_apply(const tlr_plan *pl, double *d_tmp, int nrhs,
         {
             case 16: if(one) ROWS(1, true); else ROWS(1, false); break;
             case 32: if(one) ROWS(2, true); else ROWS(2, false); break;
-            case 64: if(one) ROWS(4, true); else ROWS(4, false); break;
+            case 64:
+                if(one && pl->nchunks > ROWS1_STRIPS)
+                    hipLaunchKernelGGL(tlr_rows1_kernel, dim3(pl->nchunks),
+                            dim3(256), 0, s, pl->d_chunks, pl->d_entries,
+                            pl->d_fac, d_tmp, d_x, alpha, beta, d_y);
+                else if(one)
+                    ROWS(4, true);
+                else
+                    ROWS(4, false);
+                break;
             default: return STARSH_WRONG_PARAMETER;
         }
 #undef ROWS
