@@ -188,8 +188,10 @@ int starsh_hip_tlr_new(starsh_hip_tlr **out, STARSH_blrm *M)
      * the next product, while it is in the 256 MB cache in front of the
      * memory.  N=64000, tile 1600, one vector, with both in one direction
      * and so: 358 MB 117.3 and 116.3 us, 431 MB 142.4 and 141.0, 700 MB
-     * 229.0 and 228.4, four vectors, 586 MB 323 and 316; 126 MB, which the
-     * cache holds, 46.0 and 47.0 */
+     * 229.0 and 228.4; two vectors, 359 MB 159.0 and 152.5, 16, 716 MB 310
+     * and 300.  It costs up to 2% where the cache holds the operator anyway
+     * (126 MB 46.0 and 47.0) and without twins, whose factors it is about
+     * (four vectors, 686 MB 166.6 and 169.5) */
     for(STARSH_int b = 0; b < nbr; b++)
         first[b+1] += first[b];
     for(STARSH_int bi = 0; bi < nfar; bi++)

@@ -16,16 +16,15 @@
 // to 16 at a time go through FP64 MFMA (the columns past nrhs are zeros).
 //
 // Rounding: an MFMA adds its products to the accumulator one by one, so a
-// long chain of them loses what a lane's short one kept.  Chains end after 32
-// products (coefficients) or 16 (rows) and go to a sum of their own.  Relative
-// errors against long double, for chains as long as a wave's share, now, and
-// with a workgroup per tile and four right-hand sides at a time:
-//   N=2500, tile 250, rank 30, 4 rhs            4.2, 2.9, 2.3 e-16
-//   N=16000, tile 1000, rank 60, 16 rhs         7.2, 3.2, 2.6 e-16
+// long chain of them loses what a lane's short one kept.  Chains end after 16
+// products and go to a sum of their own.  Relative errors against long double,
+// for chains as long as a wave's share, now, and with a workgroup per tile and
+// four right-hand sides at a time:
+//   N=2500, tile 250, rank 30, 4 rhs            4.2, 2.7, 2.3 e-16
+//   N=16000, tile 1000, rank 60, 16 rhs         7.2, 3.0, 2.6 e-16
 //   N=30000, tile 1700, dense tiles, 10 rhs     7.2, 2.5, 13.6 e-16
-//   N=64000, tile 1600, rank 31, 1 rhs          3.1, 2.6, 2.7 e-16
-// at 0-1% of the time (16-product chains in the coefficients too, 2.7 and 3.0
-// e-16 for the first two, cost 5%).
+//   N=64000, tile 1600, rank 31, 1 rhs          3.1, 2.7, 2.7 e-16
+// Chains of 8 (2.3 and 2.7 e-16 for the first two) spill: 20-30% slower.
 //
 // What bounds it: memory; every factor is read twice, every dense tile once.
 // A kernel that only reads runs at 6.0-6.2 TB/s here, 7.0 below 268 MB, which
@@ -40,7 +39,7 @@
 //   the same with ranks to 133, 1566 MB                       578 -> 500 us
 //   C2's operator (2D sqexp, 431 MB), 1 rhs               149-152 -> 141 us
 //   N=30000, tile 1700, nonsymmetric, ranks to 90, 12 dense
-//     tiles, 10 rhs, 812 MB                                 4470 -> 260 us
+//     tiles, 10 rhs, 812 MB                                 4470 -> 225 us
 //   CG iteration, N=10000, tile 1000, 10 dense tiles         610 -> 72 us
 // Reading U once for U^T X and keeping V (U^T X) (1.5 reads instead of 2)
 // needs a workgroup per tile: 100 + 49 us for C2's operator against 74 + 67.
@@ -166,7 +165,11 @@ __global__ __launch_bounds__(256) void tlr_coef1_kernel(const tlr_unit *units,
 // waves in groups of 64, a lane taking rows 4 (lane/16) .. +3 of each block
 // of 16 (any order of the rows gives the same sum), so that it loads 32
 // contiguous bytes of a column.  Three workgroups per CU: with registers for
-// two, N=40000, tile 1265, 7 rhs took 93 instead of 85.5 us.
+// two, N=40000, tile 1265, 7 rhs took 93 instead of 85.5 us.  Lanes past the
+// unit's columns or the right-hand sides load column 0 instead of branching
+// around the load (only the vectors are set to zero there; the other columns'
+// sums are not stored): N=64000, tile 1600, 2 rhs 200 -> 152 us, 16 rhs 716 MB
+// 430 -> 303, and the registers allow the four short chains.
 __global__ __launch_bounds__(256, 3) void tlr_coef_kernel(
         const tlr_unit *units, const double *fac, const double *x, int ldx,
         int nrhs, double *tmp)
@@ -202,13 +205,16 @@ __global__ __launch_bounds__(256, 3) void tlr_coef_kernel(
 #pragma unroll
                 for(int v = 0; v < 4; v++)
                 {
-                    f[h][0][v] = ok[0] ? F[0][r+v] : 0.0;
-                    b[h][v] = okq ? X[r+v] : 0.0;
+                    f[h][0][v] = F[0][r+v];
+                    b[h][v] = X[r+v];
                 }
                 if(two)
 #pragma unroll
                     for(int v = 0; v < 4; v++)
-                        f[h][1][v] = ok[1] ? F[1][r+v] : 0.0;
+                        f[h][1][v] = F[1][r+v];
+#pragma unroll
+                for(int v = 0; v < 4; v++)
+                    b[h][v] = okq ? b[h][v] : 0.0;
             }
         }
         else
@@ -224,13 +230,13 @@ __global__ __launch_bounds__(256, 3) void tlr_coef_kernel(
                     b[h][v] = in && okq ? X[r] : 0.0;
                 }
         auto sums = [&](int a) {
-            Acc<false> p[2];
+            Acc<false> p[4];
 #pragma unroll
-            for(int v = 0; v < 8; v++)
+            for(int v = 0; v < 4; v++)
 #pragma unroll
-                for(int h = 0; h < 4; h += 2)
-                    p[h/2].add(f[h+v/4][a][v&3], b[h+v/4][v&3]);
-            acc[a].v += p[0].v+p[1].v;
+                for(int h = 0; h < 4; h++)
+                    p[h].add(f[h][a][v], b[h][v]);
+            acc[a].v += (p[0].v+p[1].v)+(p[2].v+p[3].v);
         };
         sums(0);
         if(two)
@@ -308,7 +314,11 @@ __global__ __launch_bounds__(256, RF <= 2 ? 4 : 2) void tlr_rows_kernel(
                     f[a][v] = F[a][(k0+4*lr+v)*fs];
 #pragma unroll
             for(int v = 0; v < 4; v++)
-                b[v] = okq ? T[(int64_t)(k0+4*lr+v)*ts] : 0.0;
+                b[v] = T[(int64_t)(k0+4*lr+v)*ts];
+            if(!ONE)
+#pragma unroll
+                for(int v = 0; v < 4; v++)
+                    b[v] = okq ? b[v] : 0.0;
 #pragma unroll
             for(int v = 0; v < 4; v++)
 #pragma unroll
