@@ -25,8 +25,9 @@ struct starsh_hip_tlr
     tlr_plan plan;
     size_t fac_doubles;
     int64_t tmp_units;       /* sum over far tiles of 2 r */
-    int64_t noalloc_units;   /* the same plus n per twin tile: the size the
-                                allocation-free product is limited by */
+    int64_t noalloc_units;   /* the same plus n per twin tile: what the fixed
+                                limit of the allocation-free product counts
+                                (its kernels no longer store the n) */
     double *d_tmp;
     int tmp_nrhs;            /* right-hand sides d_tmp has room for */
 };
@@ -372,10 +373,10 @@ int starsh_hip_tlr_dmml_noalloc(starsh_hip_tlr *T, int nrhs, double alpha,
         (int64_t)nrhs;
     if(need > TLR_SCRATCH_DOUBLES)
     {
-        STARSH_ERROR("the coefficients of this product need %lld doubles "
-                "((2 x sum of far-field ranks + rows of the transposed "
-                "tiles) x nrhs); the allocation-free product holds at most "
-                "%lld (use starsh_hip_tlr_dmml)",
+        STARSH_ERROR("the size of this product, %lld ((2 x sum of far-field "
+                "ranks + rows of the transposed tiles) x nrhs), is above the "
+                "limit of the allocation-free product, %lld (use "
+                "starsh_hip_tlr_dmml)",
                 (long long)need, (long long)TLR_SCRATCH_DOUBLES);
         return STARSH_WRONG_PARAMETER;
     }
