@@ -617,10 +617,12 @@ int hip_driver_finish(STARSH_blrm **matrix, STARSH_blrf *format,
 static size_t tile_bytes(int m, int n, int k, int maxrank)
 {
     size_t r = (size_t)(maxrank < k ? maxrank : k);
-    /* FP64 buffers, factors, int8 Omega, int8 digit planes of Q */
+    /* FP64 buffers (Y, Bt and Q2, R2, the Gram-Schmidt's coefficients and
+     * then the core's matrix, X, the singular values), factors, int8 Omega,
+     * int8 digit planes of Q */
     return sizeof(double)*((size_t)m*k+2*(size_t)n*k+(size_t)k*k+
             (size_t)(k+15)*(k+63)+16+(size_t)k*r+
-            (size_t)33*k+(size_t)(m+n)*r)+(size_t)(n+63)*k+
+            (size_t)k+(size_t)(m+n)*r)+(size_t)(n+63)*k+
         4*(size_t)(m+63)*(size_t)(k+15)+8*(size_t)(k+15);
 }
 

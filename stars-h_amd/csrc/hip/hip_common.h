@@ -73,7 +73,8 @@ struct TileDesc
     int64_t bt_off;    // Bt = A^T Q (n x k, ld n)
     int64_t q2_off;    // Q2 (n x k, ld n)
     int64_t r_off;     // R2 (k x k, ld k)
-    int64_t j_off;     // working matrix of a core beyond LDS
+    int64_t j_off;     // Gram-Schmidt coefficients, then the working matrix
+                       // of a core beyond LDS (tile_work_doubles)
     int64_t w_off;     // X_r (p x r, ld p): left singular vectors of B
     int64_t s_off;     // singular values, k entries
     int64_t u_off;     // U (m x maxrank, ld m)

@@ -58,7 +58,7 @@ int pipeline_colnorm(const TileDesc *d_tiles, int ntiles, int which,
 // in the first pass, or tau_second in the second, are set to zero and
 // flagged in d_keep.  A tile whose whole panel was dropped in the first pass
 // is marked done; *d_active counts the tiles that still have blocks to
-// process.  d_norms: ntiles x kmax doubles, d_coef: ntiles x kmax x GS_BLOCK.
+// process.  d_norms: ntiles x kmax doubles.
 // The first block (j0 = 0) takes GS_FIRST columns.
 constexpr int GS_BLOCK = 32, GS_FIRST = 64;
 inline int gs_next(int j0)
@@ -67,8 +67,8 @@ inline int gs_next(int j0)
 }
 int pipeline_gs_block(TileDesc *d_tiles, int ntiles, int which, double *ws,
         int j0, int pb, int kmax, double tau_first, double tau_second,
-        int *d_keep, double *d_norms, double *d_coef, int rows_max,
-        int *d_active, hipStream_t s);
+        int *d_keep, double *d_norms, int rows_max, int *d_active,
+        hipStream_t s);
 
 // *d_active = number of tiles with a nonzero width (k or p).
 int pipeline_count_active(const TileDesc *d_tiles, int ntiles, int which,
@@ -109,11 +109,16 @@ int pipeline_proj_i8(const TileDesc *d_tiles, int ntiles, int nmax, int kmax,
 // rotated in the tile's j_off region (core_block.hip).
 constexpr int CORE_LDS_PMAX = 128;
 
-// Doubles of a tile's j_off region for a core of up to p rows.
-inline int64_t core_work_doubles(int p)
+// Doubles of a tile's j_off region at sketch width k: the coefficients of
+// its Gram-Schmidt blocks (k x GS_BLOCK), then the working matrix of a core of
+// up to min(k, pmax) rows.
+inline int64_t tile_work_doubles(int k, int pmax)
 {
-    return p <= CORE_LDS_PMAX ? 0 :
+    const int p = k < pmax ? k : pmax;
+    const int64_t coef = k <= GS_FIRST ? 0 : (int64_t)k*GS_BLOCK;
+    const int64_t core = p <= CORE_LDS_PMAX ? 0 :
         (int64_t)((p+15)/16*16)*((p+63)/64*64);
+    return coef > core ? coef : core;
 }
 
 // One-sided Jacobi SVD of R2, singular values, rank by the reference rule

@@ -77,9 +77,8 @@ struct Pool
 Pool ws_pool, uv_pool, pack_pool, stage_pool{nullptr, 0, true};
 // The small per-batch buffers (tile descriptors, kept-column flags, norms,
 // int8 Omega and digit planes, counters, R2 partials, selected columns,
-// pivots, Gram-Schmidt coefficients, tile lists), kept too: a hipMalloc /
-// hipFree pair per buffer and batch cost
-// host time on every call, and hipFree waits for the device.
+// pivots, tile lists), kept too: a hipMalloc / hipFree pair per buffer and
+// batch cost host time on every call, and hipFree waits for the device.
 constexpr size_t SMALL_UNIT = (size_t)1 << 20;
 Pool tiles_pool{nullptr, 0, false, SMALL_UNIT},
      keep_pool{nullptr, 0, false, SMALL_UNIT},
@@ -90,7 +89,6 @@ Pool tiles_pool{nullptr, 0, false, SMALL_UNIT},
      part_pool{nullptr, 0, false, SMALL_UNIT},
      sel_pool{nullptr, 0, false, SMALL_UNIT},
      piv_pool{nullptr, 0, false, SMALL_UNIT},
-     coef_pool{nullptr, 0, false, SMALL_UNIT},
      list_pool{nullptr, 0, false, SMALL_UNIT};
 
 // Host view of the device counter of tiles still in a BCGS2 run.  The
@@ -142,14 +140,14 @@ struct PanelGraph
 {
     struct Key
     {
-        const void *tiles, *ws, *keep, *active, *norms, *coef;
+        const void *tiles, *ws, *keep, *active, *norms;
         int ntiles, which, kmax, width_max, rows_max, pb;
         double tau_first;
         bool operator==(const Key &o) const
         {
             return tiles == o.tiles && ws == o.ws && keep == o.keep &&
                 active == o.active && norms == o.norms &&
-                coef == o.coef && ntiles == o.ntiles &&
+                ntiles == o.ntiles &&
                 which == o.which && kmax == o.kmax &&
                 width_max == o.width_max && rows_max == o.rows_max &&
                 pb == o.pb && tau_first == o.tau_first;
@@ -169,7 +167,7 @@ PanelGraph panel_graphs[2];      // which = 0, 1
 // it queues precede the block that reads them); empty if they all are.
 int bcgs2(TileDesc *d_tiles, int ntiles, int which, double *ws, int kmax,
         int width_max, int rows_max, int *d_keep, double *d_norms,
-        double *d_coef, double tau_first, int *d_active, hipStream_t s,
+        double tau_first, int *d_active, hipStream_t s,
         const std::function<int(int)> &need = nullptr)
 {
     const int pw = qr_panel_width ? qr_panel_width : qr_panel_tuned;
@@ -181,7 +179,7 @@ int bcgs2(TileDesc *d_tiles, int ntiles, int which, double *ws, int kmax,
             TRY(need(width_max));
         PanelGraph &pg = panel_graphs[which ? 1 : 0];
         const PanelGraph::Key key{d_tiles, ws, d_keep, d_active, d_norms,
-            d_coef, ntiles, which, kmax, width_max, rows_max, pb, tau_first};
+            ntiles, which, kmax, width_max, rows_max, pb, tau_first};
         TRY(pipeline_count_active(d_tiles, ntiles, which, d_active, s));
         // captured and launched on a stream of its own, ordered after and
         // before the library stream's work by events: the copy-back threads
@@ -206,7 +204,7 @@ int bcgs2(TileDesc *d_tiles, int ntiles, int which, double *ws, int kmax,
                     j0 = gs_next(j0))
                 info = pipeline_gs_block(d_tiles, ntiles, which, ws, j0, pb,
                         kmax, tau_first, TAU_SECOND, d_keep, d_norms,
-                        d_coef, rows_max, d_active, cs);
+                        rows_max, d_active, cs);
             hipError_t e = hipStreamEndCapture(cs, &graph);
             if(info != STARSH_SUCCESS || e != hipSuccess)
             {
@@ -245,7 +243,7 @@ int bcgs2(TileDesc *d_tiles, int ntiles, int which, double *ws, int kmax,
         if(need)
             TRY(need(std::min(gs_next(j0), width_max)));
         TRY(pipeline_gs_block(d_tiles, ntiles, which, ws, j0, pb, kmax,
-                    tau_first, TAU_SECOND, d_keep, d_norms, d_coef, rows_max,
+                    tau_first, TAU_SECOND, d_keep, d_norms, rows_max,
                     d_active, s));
         // also after the last block, where nothing reads it: a batch of one
         // block that queued no small copy before its factors went to the host
@@ -468,7 +466,7 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
         d.r_off = off; off += k*k;
         off = (off+15)/16*16;
         d.j_off = off;
-        off += core_work_doubles((int)(k < CORE_PMAX ? k : CORE_PMAX));
+        off += tile_work_doubles((int)k, CORE_PMAX);
         d.w_off = off; off += k*rmax;
         d.s_off = off; off += k;
         d.u_off = uvoff; uvoff += m*rmax;
@@ -491,8 +489,7 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
     // part: split-K partials of R2, kept until the batch has synchronised
     Pool &tiles = tiles_pool, &keep = keep_pool, &norms = norms_pool,
          &om8 = om8_pool, &active = active_pool, &qd = qd_pool,
-         &part = part_pool, &coef = coef_pool,
-         &list = list_pool, &selbuf = sel_pool, &pivbuf = piv_pool;
+         &part = part_pool, &list = list_pool, &selbuf = sel_pool, &pivbuf = piv_pool;
     if(nsel > 0)
     {
         TRY(selbuf.reserve(sizeof(int)*(size_t)nsel));
@@ -513,7 +510,6 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
     TRY(tiles.reserve(sizeof(TileDesc)*nt));
     TRY(keep.reserve(sizeof(int)*(size_t)nt*kmax));
     TRY(norms.reserve(sizeof(double)*(size_t)nt*kmax));
-    TRY(coef.reserve(sizeof(double)*(size_t)nt*kmax*GS_BLOCK));
     TRY(uv_pool.reserve(sizeof(double)*(uvoff > 0 ? uvoff : 1)));
     TRY(active.reserve(2*sizeof(int)));
     TileDesc *d_tiles = (TileDesc *)tiles.p;
@@ -593,7 +589,7 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
     // columns of panels that are never launched count as dropped
     HIP_TRY(hipMemsetAsync(keep.p, 0, sizeof(int)*(size_t)nt*kmax, s));
     TRY(bcgs2(d_tiles, nt, 0, d_ws, kmax, kmax, mmax, (int *)keep.p,
-                (double *)norms.p, (double *)coef.p,
+                (double *)norms.p,
                 in->tau > 0 ? in->tau : TAU_FIRST, (int *)active.p, s,
                 nchunk <= 1 ? std::function<int(int)>() : [&](int c) -> int {
                     while(chunks_done < nchunk && chunk[chunks_done].beg < c)
@@ -686,8 +682,7 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
     if(pmax > 0)
     {
         TRY(bcgs2(d_tiles, nt, 1, d_ws, kmax, pmax, nmax, (int *)keep.p,
-                    (double *)norms.p, (double *)coef.p, TAU_FIRST,
-                    (int *)active.p, s));
+                    (double *)norms.p, TAU_FIRST, (int *)active.p, s));
         dump("Q2", d_ws+h[0].q2_off, (int64_t)h[0].n*h[0].p, s);
         const int nz = pipeline_r2_split(nt, pmax, nmax);
         if(nz > 1)
@@ -774,7 +769,7 @@ void rsdd_release_pools(void)
     stage_pool.release();
     for(Pool *q : {&tiles_pool, &keep_pool, &norms_pool, &om8_pool,
                 &active_pool, &qd_pool, &part_pool, &sel_pool, &piv_pool,
-                &coef_pool, &list_pool})
+                &list_pool})
         q->release();
     for(PanelGraph &pg : panel_graphs)
         pg.reset();

@@ -50,7 +50,9 @@ __global__ __launch_bounds__(256) void colnorm_kernel(const TileDesc *tiles,
 // width p; it starts as Bt[:, :p]) are orthogonalised in blocks of GS_BLOCK.
 // For each block, twice:
 //   1. C = Q_prev^T W and W -= Q_prev C against the columns before the block
-//      (gs_dot_kernel, gs_update_kernel: FP64 MFMA, spread over the chip);
+//      (gs_dot_kernel, gs_update_kernel: FP64 MFMA, spread over the chip; C,
+//      at most k x 32, in the tile's j_off region, which the core SVD takes
+//      over afterwards);
 //   2. the block's own columns in panels of PB, one workgroup per tile
 //      (gs_inner_kernel): projection against the block's earlier columns,
 //      then the panel itself with deflation.  A column whose norm after
@@ -118,8 +120,7 @@ __device__ inline GsView gs_view(const TileDesc &t, int which, double *ws,
 // of the rows gives the same sum, so a lane takes rows 4 (lane/16) .. +3 of
 // a 16-row block in its four MFMA steps and loads 32 contiguous bytes.
 __global__ __launch_bounds__(256) void gs_dot_kernel(const TileDesc *tiles,
-        int which, double *ws, int j0, int pass, double *coef,
-        double *norms, int kmax)
+        int which, double *ws, int j0, int pass, double *norms, int kmax)
 {
     __shared__ double part[3][16*64];
     __shared__ double npart[4][32];
@@ -210,7 +211,7 @@ __global__ __launch_bounds__(256) void gs_dot_kernel(const TileDesc *tiles,
     __syncthreads();
     if(wave > 0)
         return;
-    double *C = coef+(int64_t)blockIdx.y*kmax*GSB;
+    double *C = ws+t.j_off;
 #pragma unroll
     for(int q = 0; q < 16; q++)
     {
@@ -229,8 +230,7 @@ __global__ __launch_bounds__(256) void gs_dot_kernel(const TileDesc *tiles,
 // fragment is row 4 (i%4) + i/4 of it, so that a lane's four outputs are
 // contiguous.
 __global__ __launch_bounds__(256) void gs_update_kernel(
-        const TileDesc *tiles, int which, double *ws, int j0, int pass,
-        const double *coef, int kmax)
+        const TileDesc *tiles, int which, double *ws, int j0, int pass)
 {
     __shared__ double Cs[2][32][GSB];
     const TileDesc &t = tiles[blockIdx.y];
@@ -242,7 +242,7 @@ __global__ __launch_bounds__(256) void gs_update_kernel(
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lc = lane & 15, lr = lane >> 4;
     const int r0 = blockIdx.x*128+wave*32;
-    const double *C = coef+(int64_t)blockIdx.y*kmax*GSB;
+    const double *C = ws+t.j_off;
     double4_t acc[2][2];
 #pragma unroll
     for(int a = 0; a < 2; a++)
@@ -681,8 +681,8 @@ int pipeline_count_active(const TileDesc *d_tiles, int ntiles, int which,
 
 int pipeline_gs_block(TileDesc *d_tiles, int ntiles, int which, double *ws,
         int j0, int pb, int kmax, double tau_first, double tau_second,
-        int *d_keep, double *d_norms, double *d_coef, int rows_max,
-        int *d_active, hipStream_t s)
+        int *d_keep, double *d_norms, int rows_max, int *d_active,
+        hipStream_t s)
 {
     if(ntiles <= 0)
         return STARSH_SUCCESS;
@@ -691,11 +691,10 @@ int pipeline_gs_block(TileDesc *d_tiles, int ntiles, int which, double *ws,
         if(j0 > 0)
         {
             hipLaunchKernelGGL(gs_dot_kernel, dim3(j0/32, ntiles), dim3(256),
-                    0, s, d_tiles, which, ws, j0, pass, d_coef, d_norms,
-                    kmax);
+                    0, s, d_tiles, which, ws, j0, pass, d_norms, kmax);
             hipLaunchKernelGGL(gs_update_kernel, dim3((rows_max+127)/128,
                         ntiles), dim3(256), 0, s, d_tiles, which, ws, j0,
-                    pass, d_coef, kmax);
+                    pass);
         }
         // 8-column panels re-read the block's earlier columns half as often
         // as 4-column ones, at the same two tiles per CU; above 2048 rows

@@ -3,6 +3,8 @@
 classes (1024, 2048 rows): tiles of a prescribed range, whose dimension lies
 below, at and above the sketch width, give the spectrum they were built from
 and orthonormal factors."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -15,7 +17,6 @@ EPS = np.finfo(float).eps
 
 
 def _check(tiles, spectra, panel):
-    import ctypes as C
     L = S.lib()
     assert L.starsh_hip_set_option(b"qr_panel", C.c_double(panel)) == 0
     try:
@@ -57,3 +58,46 @@ def test_rows(rows):
         spectra += [s, s]
     print("rows", rows, flush=True)
     _check(tiles, spectra, 0)
+
+
+def _free_bytes():
+    free, total = C.c_size_t(), C.c_size_t()
+    assert S.lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def test_workspace_of_tiles_of_unlike_widths():
+    """2080 tiles of 64 with a sketch 20 wide and 3 tiles of 1100 with one
+    1010 wide in one batch: the device memory kept afterwards stays within
+    the budget (workspace_gb) and the rounding of the pools, whatever the
+    widest tile of the batch is."""
+    L = S.lib()
+    budget = 0.45*2**30
+    rng = np.random.default_rng(0)
+    S.init("HIP", oversample=10)
+
+    def problems():
+        return [S.TLRProblem("spatial", N, 2, nb, kernel="exp", beta=0.1,
+                             points=rng.random((2, N)))
+                for N, nb in ((4096, 64), (3300, 1100))]
+    assert L.starsh_hip_set_option(b"workspace_gb",
+                                   C.c_double(budget/2**30)) == 0
+    try:
+        # code objects, streams and pinned memory first
+        assert S.approximate_batch(problems()[:1], [10], 1e-3) == 0
+        assert L.starsh_hip_set_option(b"release_workspace",
+                                       C.c_double(0)) == 0
+        before = _free_bytes()
+        ps = problems()
+        assert S.approximate_batch(ps, [10, 1000], 1e-3) == 0
+        used = before-_free_bytes()
+        print("used MiB", used/2**20, "tiles", [len(p.tiles()) for p in ps],
+              flush=True)
+        for p in ps:
+            p.free_matrix()
+    finally:
+        assert L.starsh_hip_set_option(b"workspace_gb", C.c_double(96)) == 0
+        assert L.starsh_hip_set_option(b"release_workspace",
+                                       C.c_double(0)) == 0
+    # five pools of 64 MiB units at most
+    assert used <= budget+5*2**26
