@@ -259,9 +259,10 @@ int bcgs2(TileDesc *d_tiles, int ntiles, int which, double *ws, int kmax,
 
 // Diagnostic: when STARSH_HIP_DEBUG_DUMP names a directory, the buffers of
 // tile 0 are written there after each stage (raw doubles, column-major).
+constexpr const char *DUMP_DIR = "STARSH_HIP_DEBUG_DUMP";
 void dump(const char *name, const double *d_src, int64_t count, hipStream_t s)
 {
-    const char *dir = getenv("STARSH_HIP_DEBUG_DUMP");
+    const char *dir = getenv(DUMP_DIR);
     if(dir == nullptr || count <= 0)
         return;
     std::vector<double> h(count);
@@ -578,8 +579,11 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
         else
         {
             nchunk = pipeline_sketch_chunks(kmax, chunk);
-            TRY(pipeline_sketch_gen(d_tiles, nt, mmax, chunk[0], g, s));
-            chunks_done = 1;
+            // a dump takes all columns
+            do
+                TRY(pipeline_sketch_gen(d_tiles, nt, mmax,
+                            chunk[chunks_done++], g, s));
+            while(chunks_done < nchunk && getenv(DUMP_DIR) != nullptr);
         }
     }
     HIP_TRY(hipEventRecord(ev[3], s));
@@ -640,12 +644,13 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
     // conservative (flag 8).
     // columns sketched: all, or, of a tile exhausted in the block at gs_blk,
     // the chunks up to the one that holds that block (a captured Gram-Schmidt
-    // has all chunks computed before it)
+    // or a dump has all chunks computed before it)
     double sketch_flops = 0.0;
     for(int t = 0; t < nt; t++)
     {
         int cols = h[t].k;
-        if(nchunk > 1 && !qr_graph && (h[t].flags & 1))
+        if(nchunk > 1 && !qr_graph && getenv(DUMP_DIR) == nullptr &&
+                (h[t].flags & 1))
             for(int c = 0; c < nchunk; c++)
                 if(chunk[c].beg <= h[t].gs_blk && chunk[c].end < cols &&
                         chunk[c].end > h[t].gs_blk)

@@ -3,11 +3,13 @@ widths on either side of every rule, with tiles that exhaust their range in
 the first chunk, in a later one and not at all, against forced column blocks
 (whose chunks lie elsewhere): the same ranks and products."""
 import ctypes as C
+import os
 
 import numpy as np
 import pytest
 
 import starsh_hip as S
+from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -44,3 +46,28 @@ def test_chunks(kernel, beta, width):
         # the same columns in other blocks: rounding only, and what the rank
         # rule leaves out is the same to first order
         assert np.max(np.abs(y-got[0][1])) <= 1e-12*np.max(np.abs(y))
+
+
+def test_dump_holds_every_column(tmp_path):
+    """STARSH_HIP_DEBUG_DUMP writes the whole sketch of tile (0, 0), Y = A
+    Omega, also the columns past its range that are otherwise never
+    computed."""
+    print("case: dump of the sketch, 2D sqexp N=2400 nb=800", flush=True)
+    os.environ["STARSH_HIP_DEBUG_DUMP"] = str(tmp_path)
+    try:
+        fn = S.init("HIP", oversample=16)
+        p = S.TLRProblem("spatial", 2400, 2, 800, symm="S", seed=4,
+                         kernel="sqrexp", beta=0.1)
+        assert p.approximate(400, 1e-7, 0, fn) == 0
+    finally:
+        del os.environ["STARSH_HIP_DEBUG_DUMP"]
+    Y = np.fromfile(tmp_path/"Y.bin").reshape(416, 800).T
+    st, sz = p.cluster_ranges()
+    rows = np.arange(st[0], st[0]+sz[0])
+    A = O.kernel_block(O.kernel("sqrexp", 2, beta=0.1), p.points(),
+                       p.points(), rows, rows)
+    om = O.omega(800, 416)
+    # rounding of 800 products and of the entries (a few ulp)
+    bound = 800*np.finfo(float).eps*(np.abs(A) @ np.abs(om))
+    assert np.all(np.abs(Y-A @ om) <= bound)
+    p.free_matrix()
