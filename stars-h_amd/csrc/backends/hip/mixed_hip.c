@@ -268,19 +268,22 @@ int hip_mixed_tiles(const hip_batch *B, STARSH_int ntiles, const int *pidx,
         }
         /* optional per-tile record of the rounds (STARSH_HIP_MIXED_TRACE):
          * round, problem, tile, sketch width, rank, accepted, predicted
-         * rank, first and last singular values, Jacobi sweeps and size p
-         * of the core */
+         * rank, first and last singular values (nan where the core ended
+         * with the verdict that the rank is above the limit, before they
+         * converged), Jacobi sweeps and size p of the core */
         FILE *tf = getenv("STARSH_HIP_MIXED_TRACE") ?
             fopen(getenv("STARSH_HIP_MIXED_TRACE"), round ? "a" : "w") : NULL;
         for(STARSH_int u = 0; tf && u < npend; u++)
         {
             const int q = pq[u], os = B->hp[q].oversample;
-            const double pr = predicted_rank(sv+(size_t)u*NBMAX, k[u], os,
-                    B->tol[q]);
+            const double *s = sv+(size_t)u*NBMAX;
+            const int known = (fl[u] & 16) == 0;
+            const double pr = known ? predicted_rank(s, k[u], os, B->tol[q]) :
+                NAN;
             fprintf(tf, "%d %d %lld %d %d %d %.3g %.3e %.3e %d %d\n", round,
                     q,
                     (long long)pi[u], k[u], rk[u], acc[u], pr,
-                    sv[(size_t)u*NBMAX], sv[(size_t)u*NBMAX+k[u]-1],
+                    known ? s[0] : NAN, known ? s[k[u]-1] : NAN,
                     (fl[u] >> 8) & 255, fl[u] >> 16);
         }
         if(tf)

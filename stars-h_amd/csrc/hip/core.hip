@@ -242,9 +242,11 @@ __device__ void finish_core(TileDesc &td, double *ws, const double *W,
             r = -1;
         s_rank = r;
         td.rank = r;
-        // bit 2: not converged; bits 8-15: sweeps, 16-26: p (diagnostics)
-        td.flags |= (unconverged ? 4 : 0) | (min(sweeps, 255) << 8) |
-            (p << 16);
+        // bit 2: not converged; 4: ended with the verdict alone, the
+        // singular values have not converged; bits 8-15: sweeps, 16-26: p
+        // (diagnostics)
+        td.flags |= (unconverged ? 4 : 0) | (above ? 16 : 0) |
+            (min(sweeps, 255) << 8) | (p << 16);
     }
     __syncthreads();
     const int r = s_rank;
