@@ -609,9 +609,15 @@ int pipeline_jacobi_block(TileDesc *d_tiles, int *d_list, int count,
         for(int round = 0; round < nbe-1; round++)
             hipLaunchKernelGGL(jb_round_kernel, dim3(nbe/2, count), dim3(NT),
                     0, s, d_tiles, d_list, ws, round);
-        // tiles headed for a rank above the limit: two sweeps are enough for
-        // most, the others are tried again
-        if(certify && (sweep == 1 || sweep == 2 || sweep == 3 || sweep == 6))
+        // Tiles headed for a rank above the limit are tried after sweeps 3
+        // to 7, a try being 7-8% of a sweep.  Of those that end so, sin(kr)/r
+        // (17 tiles of 400) loses 16 after sweep 4, the SVD engine on 2D exp
+        // (10 of 1000) 4 after 3 and 6 after 4, 56 tiles of 12 exp problems
+        // (400) and 32 of 3D Matern (528) more by 5 to 7; after sweep 2 it
+        // was one of 248.  Device time without any try, with tries after 2,
+        // 3, 4 and 7, and so: 50.9, 35.8, 35.8 ms; 79.1, 47.1, 46.6; 84.5,
+        // 83, 80.5; 229, 227, 225.
+        if(certify && sweep >= 2 && sweep <= 6)
         {
             const int nb = (pmax+OB-1)/OB;
             hipLaunchKernelGGL(jb_off_kernel, dim3(nb*(nb+1)/2, count),

@@ -329,11 +329,16 @@ extern "C" int starsh_hip_gen_gemm_bn(int bn)
 // The sketch's columns go in chunks, computed as the Gram-Schmidt reaches
 // them: a tile whose range is exhausted by then has no use for the rest (the
 // random columns after that point are dropped unread).  A chunk is one column
-// block.  Wide blocks reuse each generated entry most (820 tiles of 1600,
-// 2D sqexp: 22.6 ms for a block of 256, 14.4 for 128), so the first chunk is
+// block.  Wide blocks reuse each generated entry most, so the first chunk is
 // narrow only where tiles that need every column lose nothing by it: with
 // more than 256 columns, when the padding that the narrow blocks save pays
-// for them (417-448 and 513-640 columns, say, but not 449-512).  2D sqexp
+// for them (417-448 and 513-640 columns, say, but not 449-512).  The costs of
+// 64, 128 and 256 columns measured, scaled to 22.6 for 256: 2D sqexp 820
+// tiles of 1600 8.2, 14.4 (23.7 ms for 256); 2D exp the same 8.6, 14.6, 820
+// of 500 7.8, 14.0; 3D Matern 136 of 2048 8.4, 12.3; sin(kr)/r 153 of 1536
+// 7.3, 11.8; Coulomb 6.9, 12.4.  The highest are taken: with the lowest,
+// 449-512 columns would go narrow as well, 5% slower for the 2D kernels.  2D
+// sqexp
 // N=64000, 416 columns, all tiles exhausted within 96: sketch 45.3 -> 15.3
 // ms; sin(kr)/r N=25000, 400 columns, 17 of 153 tiles needing all: 11.7 ->
 // 9.4 ms.
@@ -349,7 +354,7 @@ int pipeline_sketch_chunks(int k, SketchChunk *c)
     // block for the last r columns, and its cost
     auto block = [](int r) { return r <= 64 ? 64 : r <= 128 ? 128 : 256; };
     auto cost = [](int bn) {
-        return bn == 64 ? 9.5 : bn == 128 ? 14.4 : 22.6; };
+        return bn == 64 ? 8.6 : bn == 128 ? 14.6 : 22.6; };
     int beg = 0;
     if(fb > 0)
         while(beg < k)
