@@ -19,6 +19,24 @@ namespace {
 
 constexpr int JACOBI_SWEEPS_DEFAULT = 60;
 
+// Four waves per tile keep a group of 8 or more lanes per column pair up to 64
+// rows and leave room for other tiles on the CU; above, W takes the room and
+// sixteen waves shorten its chain.  With cores on both sides, few tiles go in
+// one launch of sixteen waves, as those of a second one would wait for the
+// first; many go in one launch for each.  Device time of whole compressions
+// (2D exp and sqexp), all with four waves, all with sixteen, in two launches:
+//   55 tiles, largest core at most 50 rows      1.35   1.46      - ms
+//   55, 107                                     5.28   3.62   4.10
+//   210, 96 (tiles of 1600)                    14.6   13.4   13.9
+//   276, 86                                     4.71   3.95   4.12
+//   465, 96                                     6.20   4.03   4.18
+//   820, 50                                     2.45   3.28      -
+//   820, 96 (tiles of 250)                      6.90   5.32   4.87
+//   820, 110                                    9.65   7.50   7.30
+//   820, 96, most below 64 (tiles of 1600)     33.6   34.4   33.7
+//   1035, 86                                    7.87   8.27   7.89
+constexpr int CORE_SMALL_PMAX = 64, CORE_SPLIT_TILES = 512;
+
 __device__ inline double group_sum(double v, int g)
 {
     return group_sum_lanes(v, g);
@@ -262,12 +280,12 @@ __device__ void finish_core(TileDesc &td, double *ws, const double *W,
     }
 }
 
-// The tiles with p <= lds_p: W in LDS, one workgroup per tile.  Dynamic
-// LDS: 2 (lds_p+1) doubles of singular values, W (lds_p^2 doubles), then
-// lds_p ints.
+// The tiles with above < p <= lds_p: W in LDS, one workgroup per tile.
+// Dynamic LDS: 2 (lds_p+1) doubles of singular values, W (lds_p^2 doubles),
+// then lds_p ints.
 template <int NT>
 __global__ __launch_bounds__(NT) void core_kernel(TileDesc *tiles,
-        double *ws, int lds_p, int max_sweeps)
+        double *ws, int above, int lds_p, int max_sweeps)
 {
     extern __shared__ double dyn[];
     double *sig = dyn, *W = dyn+2*(lds_p+1);
@@ -275,7 +293,7 @@ __global__ __launch_bounds__(NT) void core_kernel(TileDesc *tiles,
     __shared__ unsigned long long s_wmax;
     TileDesc &td = tiles[blockIdx.x];
     const int p = td.p, k = td.k;
-    if(p > lds_p)
+    if(p > lds_p || p <= above)
         return;
     if(p <= 0)
     {
@@ -333,15 +351,15 @@ __global__ __launch_bounds__(1024) void core_finish_kernel(TileDesc *tiles,
 }
 
 template <int NT>
-int launch_core(TileDesc *d_tiles, int ntiles, double *ws, int lds_p,
-        int max_sweeps, hipStream_t s)
+int launch_core(TileDesc *d_tiles, int ntiles, double *ws, int above,
+        int lds_p, int max_sweeps, hipStream_t s)
 {
     const size_t bytes = sizeof(double)*(2*((size_t)lds_p+1)+
             (size_t)lds_p*lds_p)+sizeof(int)*(size_t)lds_p;
     HIP_TRY(hipFuncSetAttribute((const void *)core_kernel<NT>,
                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
     hipLaunchKernelGGL(core_kernel<NT>, dim3(ntiles), dim3(NT), bytes, s,
-            d_tiles, ws, lds_p, max_sweeps);
+            d_tiles, ws, above, lds_p, max_sweeps);
     HIP_TRY(hipGetLastError());
     return STARSH_SUCCESS;
 }
@@ -370,28 +388,21 @@ int pipeline_core(TileDesc *d_tiles, int ntiles, double *ws, int pmax,
         return STARSH_WRONG_PARAMETER;
     const int pm = pmax > 0 ? pmax : 1;
     const int lds_p = pm <= CORE_LDS_PMAX ? pm : CORE_LDS_PMAX;
-    // Four waves per tile keep a group of 8 or more lanes per column pair up
-    // to 64 rows and leave room for other tiles on the CU; above, and with
-    // few tiles, W fills the LDS or the chip is not full and sixteen waves
-    // win (55 cores of 40-110 rows: 4.8 -> 2.4 ms; 820 of 34-96: 2.2
-    // against 2.7 ms, so they keep four).
-    if(lds_p <= 64 || (lds_p <= 96 && ntiles > 512))
-    {
-        const int info = launch_core<256>(d_tiles, ntiles, ws, lds_p,
+    // up to which size the tiles take four waves
+    const int small = lds_p <= CORE_SMALL_PMAX ? lds_p :
+        ntiles > CORE_SPLIT_TILES ? CORE_SMALL_PMAX : -1;
+    int info = STARSH_SUCCESS;
+    if(small > 0)
+        info = launch_core<256>(d_tiles, ntiles, ws, -1, small,
                 jacobi_max_sweeps, s);
-        if(info != STARSH_SUCCESS)
-            return info;
-    }
-    else
-    {
-        const int info = launch_core<1024>(d_tiles, ntiles, ws, lds_p,
+    if(info == STARSH_SUCCESS && lds_p > small)
+        info = launch_core<1024>(d_tiles, ntiles, ws, small, lds_p,
                 jacobi_max_sweeps, s);
-        if(info != STARSH_SUCCESS)
-            return info;
-    }
+    if(info != STARSH_SUCCESS)
+        return info;
     if(pm > lds_p)
     {
-        const int info = pipeline_jacobi_block(d_tiles, d_list, count, ws,
+        info = pipeline_jacobi_block(d_tiles, d_list, count, ws,
                 pm, jacobi_max_sweeps, certify, d_out, h_out, s);
         if(info != STARSH_SUCCESS)
             return info;

@@ -22,14 +22,14 @@
 // O(32) LDS traffic and the O(p) work is MFMA.  A visit is a chain of 31
 // steps, each a rotation and two passes through LDS; with 32-column blocks
 // (63 steps on 64 x 64 matrices, half the rounds) a round took 118 us instead
-// of 35 at p = 150, 130 instead of 44 at 400, 178 instead of 76 at 1000 (four
-// waves), and Matern with 500-row cores was 7% slower as well.  The whole
+// of 35 at p = 150, 130 instead of 44 at 400, 178 instead of 76-82 at 1000
+// (four waves), and Matern with 500-row cores was 7% slower as well.  The whole
 // 31-step sweep over both blocks' columns converges in about 6 outer sweeps
 // where the 16 cross steps alone need 7-8 (numpy model on sin(kr)/r, exp and
 // Matern cores).
 // Measured on MI355X, all launches of one compression, against one
 // workgroup per tile: 2D exp N=9973, tile 1000, SVD engine (10 cores of
-// 1000, 45 of 200-500) 1570 -> 22.5 ms; sin(kr)/r N=25000, tile 1536 (17 of
+// 1000, 45 of 200-500) 1570 -> 22 ms; sin(kr)/r N=25000, tile 1536 (17 of
 // 400, 85 of 130-210) 163 -> 6.4 ms; 3D Matern N=65536, tile 2048, mixed
 // (up to 528) 191 -> 52 ms.  Only tiles still rotating are launched, by a
 // list the sweeps shorten.

@@ -51,15 +51,16 @@ int pipeline_proj_gen(const TileDesc *d_tiles, int ntiles, int mmax,
 int pipeline_colnorm(const TileDesc *d_tiles, int ntiles, int which,
         double *ws, double *d_norm, int kmax, hipStream_t s);
 
-// Block Gram-Schmidt applied twice for the GS_BLOCK columns at j0 (a
-// multiple of GS_BLOCK), in panels of pb (qr.hip).  which: 0 = Q (width k),
-// 1 = Q2 (width p; the columns are read from Bt and written to Q2).  Columns
-// whose norm after projection is at most tau_first times their original norm
-// in the first pass, or tau_second in the second, are set to zero and
-// flagged in d_keep.  A tile whose whole panel was dropped in the first pass
-// is marked done; *d_active counts the tiles that still have blocks to
+// Block Gram-Schmidt applied twice for the block of columns at j0 (GS_FIRST
+// columns at 0, GS_BLOCK after that; gs_next gives the next one), in panels of
+// pb (qr.hip).  which: 0 = Q (width k), 1 = Q2 (width p; the columns are read
+// from Bt and written to Q2).  Columns whose norm after projection is at most
+// tau_first times their original norm in the first pass, or tau_second in
+// the second, are set to zero and cleared in d_keep.  A tile that drops four
+// columns in a row in the first pass (a group starting at a multiple of four,
+// or what is left of the last one) is marked done, unless its sketch is a
+// selection of columns; *d_active counts the tiles that still have blocks to
 // process.  d_norms: ntiles x kmax doubles.
-// The first block (j0 = 0) takes GS_FIRST columns.
 constexpr int GS_BLOCK = 32, GS_FIRST = 64;
 inline int gs_next(int j0)
 {

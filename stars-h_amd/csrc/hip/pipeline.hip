@@ -245,10 +245,14 @@ int bcgs2(TileDesc *d_tiles, int ntiles, int which, double *ws, int kmax,
         TRY(pipeline_gs_block(d_tiles, ntiles, which, ws, j0, pb, kmax,
                     tau_first, TAU_SECOND, d_keep, d_norms, rows_max,
                     d_active, s));
-        // also after the last block, where nothing reads it: a batch of one
-        // block that queued no small copy before its factors went to the host
-        // moved them at 29 instead of 52 GB/s (2D sqexp N=64000 mixed, 430 MB:
-        // 15.0 ms; with the copies 8.6-9.4, now and then 15)
+        // Also after the last block, where nothing reads it.  The runtime
+        // moves the factors with one of several DMA engines and keeps to it
+        // for some calls; on one of them a piece of 32 MiB takes 0.595 ms, on
+        // another 1.105 (30 GB/s).  A small copy in the same direction shortly
+        // before makes it take the faster one in most calls: 2D sqexp
+        // N=64000 mixed, 430 MB, three processes of 12 compressions: 8.6-11.8
+        // ms and 15.2 three times; without it 15.2 in the first seven or
+        // eight calls of each and 8.7-11.3 after that.
         const int slot = block % NSLOT;
         HIP_TRY(hipMemcpyAsync(probe.h+slot, d_active, sizeof(int),
                     hipMemcpyDeviceToHost, s));

@@ -112,3 +112,28 @@ def test_early_verdict_on_the_rank():
     print(with_s, without, ref, flush=True)
     assert without == with_s == ref
     assert ref[:3] == [-1, -1, -1] and ref[3] == maxrank
+
+
+def test_many_cores_on_both_sides_of_a_launch():
+    """More than 512 tiles with cores from 0 (a zero tile) to 128 rows go in
+    two launches, up to 64 rows and above: every tile has its spectrum and
+    rank, as in a batch of few tiles (one launch)."""
+    sizes = [0, 1, 2, 63, 64, 65, 66, 127, 128]+[5, 20, 40, 70, 100]*102
+    tol = 1e-3
+    tiles, spectra = [], []
+    for q, p in enumerate(sizes):
+        s = 0.9**np.arange(p)
+        spectra.append(s)
+        tiles.append(_tile(p+9, p+5, s, q) if p else np.zeros((30, 20)))
+    print(len(tiles), "tiles", flush=True)
+    got = _lowrank(0, tiles, 140, 10, tol, True)
+    few = _lowrank(0, tiles[:20], 140, 10, tol, True)
+    for t, ((r, u, v, sv), s, p) in enumerate(zip(got, spectra, sizes)):
+        # rounding of the sketch, the projection and the rotations: each a
+        # few units of p eps of the largest singular value
+        bound = 20*max(p, 1)*np.finfo(float).eps
+        assert r == _dsvfr(s, tol), (t, p)
+        assert np.max(np.abs(sv[:p]-s), initial=0.0) <= bound, (t, p)
+        if t < len(few):
+            assert few[t][0] == r
+            assert np.max(np.abs(few[t][3]-sv)) <= 2*bound, (t, p)
