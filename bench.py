@@ -45,7 +45,9 @@ PEAK_FP64 = 78.6  # TFLOP/s, MI355X dense FP64 (vector and matrix)
 # profiles/c2_counters.md).  HBM bytes are FETCH_SIZE and WRITE_SIZE (KiB)
 # scaled by the same counters on a 1 GiB device copy (fetch x2.00, write
 # x1.00).
-C2_PLAIN_SKETCH_TRAFFIC = 1.843e9   # gen_gemm_kernel<2,2,128,1,false>
+# the first chunk of the sketch, gen_gemm_kernel<2,2,BN,RW,false> by its column
+# block and row groups (the autotuner's choice, or 128 x 1)
+C2_PLAIN_SKETCH_TRAFFIC = {(128, 1): 1.841e9, (128, 2): 2.007e9}
 C2_MIXED_PROJ_TRAFFIC = 0.660e9     # proj_i8_kernel<2,2,64,false>
 C2_MIXED_PROJ_VALU_INSTS = 1.030e9  # SQ_INSTS_VALU (wave64 instructions)
 C2_MIXED_PROJ_VALU_BUSY = 0.69      # VALUBusy at the kernel's clock
@@ -397,14 +399,20 @@ def main():
         # flops 2 m n k per tile, time from HIP events around the launch
         t = plain["sketch_kernel_seconds"]
         a = plain["sketch_flops"] / t / 1e12 if t > 0 else 0.0
+        tuned = plain.get("schedule") or {}
+        shape = (tuned.get("sketch_bn") or 128, tuned.get("sketch_rw") or 1)
+        forced = any(o.startswith("gemm_") for o in args.set)
         rooflines["plain"] = {
             "kernel": "gen_gemm_kernel (sketch Y = A Omega, FP64 MFMA, "
-                      "tile generated in registers)",
+                      "tile generated in registers), column block x row "
+                      "groups " + ("as set" if forced else
+                                   f"{shape[0]} x {shape[1]}"),
             "bound": "mfma", "achieved": round(a, 3), "peak": PEAK_FP64,
             "unit": "TFLOP/s", "frac": round(a / PEAK_FP64, 4),
             "frac_of_attainable": (round(a / probe["mfma"], 4)
                                    if probe else None),
-            "traffic": C2_PLAIN_SKETCH_TRAFFIC if c2 else None}
+            "traffic": (C2_PLAIN_SKETCH_TRAFFIC.get(shape)
+                        if c2 and not forced else None)}
     if "mixed" in forms:
         # mixed form: the int8 projection B^T = A^T Q dominates; it is
         # bound by VALU issue (FP64 tile generation and digit splitting),
