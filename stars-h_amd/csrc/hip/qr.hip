@@ -456,7 +456,8 @@ __global__ __launch_bounds__(NT, 2) void gs_inner_kernel(TileDesc *tiles,
             // come from one reduction (one barrier), then column c leaves
             // the later ones.  Once per pass is enough: the second pass
             // starts from columns that are orthogonal up to rounding over
-            // tau.
+            // tau (max|Q^T Q - I| is 3-6 eps over spectra of eleven orders,
+            // steps and cliffs, as with two sweeps in each pass).
             const double tau2 = ps == 0 ? tau2_first : tau2_second;
             int dropped = 0;
 #pragma unroll
