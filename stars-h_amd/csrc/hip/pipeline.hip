@@ -494,7 +494,8 @@ int rsdd_batch(const RsddInput *in, RsddOutput *out)
     // part: split-K partials of R2, kept until the batch has synchronised
     Pool &tiles = tiles_pool, &keep = keep_pool, &norms = norms_pool,
          &om8 = om8_pool, &active = active_pool, &qd = qd_pool,
-         &part = part_pool, &list = list_pool, &selbuf = sel_pool, &pivbuf = piv_pool;
+         &part = part_pool, &list = list_pool, &selbuf = sel_pool,
+         &pivbuf = piv_pool;
     if(nsel > 0)
     {
         TRY(selbuf.reserve(sizeof(int)*(size_t)nsel));

@@ -29,10 +29,10 @@
 // What bounds it: memory; every factor is read twice, every dense tile once.
 // A kernel that only reads runs at 6.0-6.2 TB/s here, 7.0 below 268 MB, which
 // the cache in front of the memory holds; the coefficients of C2's operator
-// (N=64000, tile 1600, 431 MB) run at 5.9, its rows at 6.4.  Measured on MI355X, before and after (one workgroup per tile forming U^T X
-// and then V (U^T X) row by row, and strips of 64 rows, dense tiles one
-// column at a time, right-hand sides in groups of four that each re-read
-// everything):
+// (N=64000, tile 1600, 431 MB) run at 5.8, its rows at 6.3.  Measured on
+// MI355X, before and after (one workgroup per tile forming U^T X and then
+// V (U^T X) row by row, and strips of 64 rows, dense tiles one column at a
+// time, right-hand sides in groups of four that each re-read everything):
 //   N=2500, tile 250, 1 rhs (launch-bound)                  27.7 -> 10.7 us
 //   N=64000, tile 1600, ranks 8-31, 1 rhs, 358 MB, read
 //     twice                                              129-146 -> 116-122 us

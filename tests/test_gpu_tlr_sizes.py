@@ -278,6 +278,32 @@ def test_upload_sizes(total):
     assert np.array_equal(back, data)
 
 
+@pytest.mark.parametrize("nrhs", [1, 3])
+def test_cg_solves(nrhs):
+    """Random columns, and one that is an eigenvector and converges at once,
+    against the dense solution."""
+    N = 700
+    fn = S.init("HIP", oversample=16)
+    rng = np.random.default_rng(3)
+    p = S.TLRProblem("spatial", N, 2, 100, kernel="exp", beta=0.1,
+                     noise=0.5, points=rng.random((2, N)))
+    assert p.approximate(60, 1e-9, 0, fn) == 0
+    A = p.dmml(np.eye(N))
+    X = rng.standard_normal((N, nrhs))
+    if nrhs > 1:
+        X[:, 1] = np.linalg.eigh(0.5*(A+A.T))[1][:, -1]
+    B = A @ X
+    it, Y = p.cg(B, np.zeros_like(B), 1e-10)
+    print("iterations", it, flush=True)
+    assert 0 < it < N
+    # |x - x'| <= cond |r|/|b| |x|, cond below |A|/noise
+    cond = np.linalg.norm(A, 2)/0.5
+    for q in range(nrhs):
+        assert np.linalg.norm(Y[:, q]-X[:, q]) <= 2e-10*cond*np.linalg.norm(
+            X[:, q])
+    p.free_matrix()
+
+
 def _covariance(N=700):
     fn = S.init("HIP", oversample=16)
     rng = np.random.default_rng(3)
